@@ -19,12 +19,11 @@
 //   A brick whose box exceeds its 64 KB arena slot falls back to
 //   device-scope float atomics into the finished mesh (k_brick_spill, after
 //   phase 2).
-// phase 2 (k_brick_gather): one workgroup per mesh tile (16^3; 4 x 16 x 16
-//   for the three channels) evaluates the
-//   candidate bricks in parallel, compacts those whose boxes meet the tile
-//   (in candidate order), and every thread adds them, in that order, to the
-//   cells of the x row it owns; the tile is written with plain stores, no barrier per
-//   brick, so the mesh is never cleared first.
+// phase 2 (k_brick_gather): one workgroup per mesh tile (4, 8 or 16 x planes
+//   of 16 x 16 cells) evaluates the candidate bricks in parallel, compacts
+//   those whose boxes meet the tile (in candidate order), and every wave adds
+//   them, in that order, to the x planes it owns; the tile is written with
+//   plain stores, no barrier per brick, so the mesh is never cleared first.
 //
 // Device-scope float atomics cannot complete inside one XCD's L2 (the eight
 // L2s are not coherent with each other), so the plain scatter pays a far
@@ -38,9 +37,9 @@ namespace pmx {
 struct BrickArgs {
   float* mesh[3];        // C output meshes [B][nx][ny][nz] (overwritten)
   float* arena;          // box arena
-  long long arena_cap;   // floats
   long long slot;        // arena floats per brick
   int accum;             // gather adds to the mesh instead of overwriting
+  int vec4;              // the gather may store the mesh 16 bytes at a time
   int* meta;             // 8 ints per brick: lo[3], ext[3], R (how far the
                          // box reaches past the brick), overflow flag
   int* ctr;              // [2] overflow count, [3] box radius (written by
@@ -77,8 +76,6 @@ __device__ __forceinline__ bool ok_pos(float x, float y, float z) {
 // in slabs of whole x planes, one pass over the particles per slab.
 constexpr int kDT = 512;
 constexpr int kWinFloats = 10112;
-// gather tile x lengths of the density and of the three-channel paint
-constexpr int kGatherTx1 = 16, kGatherTx3 = 4;
 constexpr int kDW = kDT / 64;
 constexpr int kPPT = 2048 / kDT;
 
@@ -377,12 +374,26 @@ __global__ __launch_bounds__(1024) void k_brick_reduce(const int* __restrict__ m
   }
 }
 
-// TX: the tile's x length, the cells each thread owns (16 for the density;
-// 4 for the three channels, whose 3 x 16 accumulators would take 124 VGPRs
-// and half the waves: 281 us at 256^3 with 16, 249 with 8, 235 with 4)
-template <int C, int TX>
+// four consecutive floats of a box row, at any dword
+typedef float Vec4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// One workgroup of 4 waves per mesh tile of 4 PX x 16 x 16 cells: wave w owns
+// the x planes w PX .. w PX + PX - 1, a lane 4 consecutive z cells of one y
+// row in each of them, so one 16-byte load per lane covers a whole 16 x 16
+// plane of a box.  Bound by the load instructions and, on few tiles, by the
+// chain of boxes each wave walks: a wave visits only the boxes that meet its
+// own planes (one ballot), and has the loads of kGatherU boxes in flight
+// together.  Against a thread per (y, z) column reading 16 x cells one float
+// at a time, with the cells outside the box loaded and dropped: density at
+// 256^3 122 -> 92 us, 16 x 64^3 38 -> 26, 128^3 37 -> 22, 64^3 28 -> 12.5,
+// 32^3 21 -> 7.8; the three channels, which had one float of 4 cells per
+// load, gain little: at 128 x 160 x 96 31 -> 29, at 64^3 12.4 -> 12.9.
+// The sums, and their order, are the same: so are the results, bit for bit.
+constexpr int kGatherU = 2;
+template <int C, int PX>
 __global__ __launch_bounds__(256) void k_brick_gather(BrickArgs a) {
-  constexpr int PER = TX;  // owned cells per thread: (k, iy, iz), k < TX
+  constexpr int U = kGatherU;
+  constexpr int TX = 4 * PX;
   __shared__ short cand[3][1024];
   __shared__ int ncand[3];
   __shared__ int lst[256][8];  // overlapping bricks of one chunk
@@ -400,7 +411,7 @@ __global__ __launch_bounds__(256) void k_brick_gather(BrickArgs a) {
             Tz = min(kTile, d.nz - t0z);
   const int R = a.ctr[3];
   // candidate bricks per dimension (wave w builds list w)
-  const int wv = tid >> 6, ln = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), ln = tid & 63;
   if (wv < 3) {
     const int e = wv == 0 ? g.ex : (wv == 1 ? g.ey : g.ez);
     const int gd = wv == 0 ? g.gx : (wv == 1 ? g.gy : g.gz);
@@ -424,15 +435,17 @@ __global__ __launch_bounds__(256) void k_brick_gather(BrickArgs a) {
   __syncthreads();
   const int nc0 = ncand[0], nc1 = ncand[1], nc2 = ncand[2];
   const int total = nc0 * nc1 * nc2;
-  // owned cells: (x = t0x + k, y = t0y + iy, z = t0z + iz), k = 0..15
-  const int iy = tid / kTile, iz = tid % kTile;
-  const int cy = t0y + iy, cz = t0z + iz;
-  const bool yz_ok = iy < Ty && iz < Tz;
-  float acc[C][PER];
+  // owned cells: x = x0w + k (k < PX), y = cy, z = cz + i (i < 4)
+  const int x0w = t0x + wv * PX;
+  const int cy = t0y + (ln >> 2), cz = t0z + 4 * (ln & 3);
+  const bool yz_ok = cy < d.ny && cz < d.nz;
+  float acc[C][PX][4];
 #pragma unroll
   for (int c = 0; c < C; ++c)
 #pragma unroll
-    for (int k = 0; k < PER; ++k) acc[c][k] = 0.0f;
+    for (int k = 0; k < PX; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[c][k][i] = 0.0f;
   for (int base = 0; base < total; base += 256) {
     // 1. evaluate one candidate per thread, compact the overlapping ones in
     //    candidate order (ballot within a wave, wave counts across)
@@ -442,11 +455,13 @@ __global__ __launch_bounds__(256) void k_brick_gather(BrickArgs a) {
     if (ci < total) {
       const int i2 = ci % nc2, r = ci / nc2, i1 = r % nc1, i0 = r / nc1;
       const int bid = (cand[0][i0] * g.nby + cand[1][i1]) * g.nbz + cand[2][i2];
-      const int* m = a.meta + 8LL * ((long long)b * g.nbricks + bid);
-      const int e0 = m[3], e1 = m[4], e2 = m[5];
+      const int4* m = reinterpret_cast<const int4*>(
+          a.meta + 8LL * ((long long)b * g.nbricks + bid));
+      const int4 ma = m[0], mb = m[1];
+      const int e0 = ma.w, e1 = mb.x, e2 = mb.y;
       if (e0 > 0) {
-        const int a0 = imod(m[0], d.nx), a1 = imod(m[1], d.ny),
-                  a2 = imod(m[2], d.nz);
+        const int a0 = imod(ma.x, d.nx), a1 = imod(ma.y, d.ny),
+                  a2 = imod(ma.z, d.nz);
         ok = box_meets(a0, e0, t0x, Tx, d.nx) &&
              box_meets(a1, e1, t0y, Ty, d.ny) &&
              box_meets(a2, e2, t0z, Tz, d.nz);
@@ -473,35 +488,93 @@ __global__ __launch_bounds__(256) void k_brick_gather(BrickArgs a) {
       for (int q = 0; q < 7; ++q) lst[pos][q] = rec[q];
     }
     __syncthreads();
-    // 2. every thread adds the bricks, in list order, to its own cells
-    if (yz_ok) {
-      for (int j = 0; j < nl; ++j) {
-        const int e1 = lst[j][5], e2 = lst[j][6];
-        const int oy = wrap_off(cy, lst[j][2], d.ny);
-        const int oz = wrap_off(cz, lst[j][3], d.nz);
-        if (oy >= e1 || oz >= e2) continue;
-        const int e0 = lst[j][4];
-        const int vol = e0 * e1 * e2;
-        const float* src =
-            a.arena + ((long long)b * g.nbricks + lst[j][0]) * a.slot;
-        const int a0 = lst[j][1];
-        // branch-free: every load is issued (out-of-box ones read box
-        // element 0) before the first is consumed, so the 16 x C loads of
-        // one brick are in flight together instead of one round trip each
-        float v[C][PER];
-        bool in[PER];
+    // 2. every wave adds the bricks that meet its planes, in list order, to
+    //    its own cells, the loads of U bricks in flight together
+    for (int l0 = 0; l0 < nl; l0 += 64) {
+      bool meets = false;
+      if (l0 + ln < nl) {
+        const int a0 = lst[l0 + ln][1], e0 = lst[l0 + ln][4];
 #pragma unroll
-        for (int k = 0; k < PER; ++k) {
-          const int ox = wrap_off(t0x + k, a0, d.nx);
-          in[k] = k < Tx && ox < e0;
-          const int bi = in[k] ? (ox * e1 + oy) * e2 + oz : 0;
+        for (int k = 0; k < PX; ++k)
+          meets = meets || (x0w + k < d.nx && wrap_off(x0w + k, a0, d.nx) < e0);
+      }
+      unsigned long long todo = __ballot(meets);
+      while (todo) {
+        float v[U][C][PX][4];
+        bool in[U][PX], inz[U][4];
 #pragma unroll
-          for (int c = 0; c < C; ++c) v[c][k] = src[c * vol + bi];
+        for (int u = 0; u < U; ++u) {
+          const bool any = todo != 0;  // wave-uniform
+          const int j = l0 + (any ? __ffsll(todo) - 1 : 0);
+          todo &= todo - 1;
+          auto rd = [&](int q) {
+            return __builtin_amdgcn_readfirstlane(lst[j][q]);
+          };
+          const int a0 = rd(1), a1 = rd(2), a2 = rd(3), e0 = rd(4), e1 = rd(5),
+                    e2 = rd(6);
+          const int vol = e0 * e1 * e2, pl = e1 * e2;
+          const float* src =
+              a.arena + ((long long)b * g.nbricks + rd(0)) * a.slot;
+          const int oy = wrap_off(cy, a1, d.ny);
+          const bool yin = any && yz_ok && oy < e1;
+          const int o = cz - a2;
+          if (e2 <= d.nz - 4) {
+            // the four cells lie in one run of box offsets: o .. o + 3 from
+            // o = -3 on, o + nz .. below that (nothing of o + i < 0 with
+            // o > -4 is in a box this short)
+            const int oz = o > -4 ? o : o + d.nz;
+            const bool lane = yin && oz < e2;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              inz[u][i] = lane && oz + i >= 0 && oz + i < e2;
+            const int bi = lane ? oy * e2 + oz : 0;
+#pragma unroll
+            for (int k = 0; k < PX; ++k) {
+              const int ox = wrap_off(x0w + k, a0, d.nx);
+              in[u][k] = x0w + k < d.nx && ox < e0;
+              const float* p = src + (in[u][k] ? ox * pl : 0);
+#pragma unroll
+              for (int c = 0; c < C; ++c) {
+                const Vec4u q =
+                    *reinterpret_cast<const Vec4u*>(p + c * vol + bi);
+                v[u][c][k][0] = q.x;
+                v[u][c][k][1] = q.y;
+                v[u][c][k][2] = q.z;
+                v[u][c][k][3] = q.w;
+              }
+            }
+          } else {
+            // a box that nearly spans the mesh: each cell by itself
+            int zi[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const bool zok = cz + i < d.nz;
+              const int oz = wrap_off(cz + (zok ? i : 0), a2, d.nz);
+              inz[u][i] = yin && zok && oz < e2;
+              zi[i] = inz[u][i] ? oy * e2 + oz : 0;
+            }
+#pragma unroll
+            for (int k = 0; k < PX; ++k) {
+              const int ox = wrap_off(x0w + k, a0, d.nx);
+              in[u][k] = x0w + k < d.nx && ox < e0;
+              const float* p = src + (in[u][k] ? ox * pl : 0);
+#pragma unroll
+              for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[u][c][k][i] = p[c * vol + zi[i]];
+            }
+          }
         }
 #pragma unroll
-        for (int k = 0; k < PER; ++k)
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-          for (int c = 0; c < C; ++c) acc[c][k] += in[k] ? v[c][k] : 0.0f;
+          for (int k = 0; k < PX; ++k)
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                acc[c][k][i] +=
+                    in[u][k] && inz[u][i] ? v[u][c][k][i] : 0.0f;
       }
     }
     __syncthreads();  // lst is rewritten by the next chunk
@@ -509,14 +582,30 @@ __global__ __launch_bounds__(256) void k_brick_gather(BrickArgs a) {
   if (!yz_ok) return;
   // every cell of the mesh is written here (the mesh needs no clearing);
   // with accum the painted values are added to the mesh's own
+  const bool whole = a.vec4 && cz + 4 <= d.nz;
 #pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    if (k < Tx) {
+  for (int k = 0; k < PX; ++k) {
+    if (x0w + k < d.nx) {
       const long long cell =
-          (((long long)b * d.nx + t0x + k) * d.ny + cy) * d.nz + cz;
+          (((long long)b * d.nx + x0w + k) * d.ny + cy) * d.nz + cz;
 #pragma unroll
-      for (int c = 0; c < C; ++c)
-        a.mesh[c][cell] = a.accum ? a.mesh[c][cell] + acc[c][k] : acc[c][k];
+      for (int c = 0; c < C; ++c) {
+        float* out = a.mesh[c] + cell;
+        if (whole) {
+          float4 r = make_float4(acc[c][k][0], acc[c][k][1], acc[c][k][2],
+                                 acc[c][k][3]);
+          if (a.accum) {
+            const float4 o = *reinterpret_cast<const float4*>(out);
+            r = make_float4(o.x + r.x, o.y + r.y, o.z + r.z, o.w + r.w);
+          }
+          *reinterpret_cast<float4*>(out) = r;
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (cz + i < d.nz)
+              out[i] = a.accum ? out[i] + acc[c][k][i] : acc[c][k][i];
+        }
+      }
     }
   }
 }
@@ -594,10 +683,16 @@ int launch_brick_paint(float* const* mesh, int C, const float* X,
   a.accum = accumulate ? 1 : 0;
   for (int c = 0; c < C; ++c) a.mesh[c] = mesh[c];
   a.slot = (long long)C * kBoxFloats;
-  a.arena = work;
-  a.arena_cap = (long long)d.B * g.nbricks * a.slot;
-  a.meta = reinterpret_cast<int*>(work + a.arena_cap);
+  // 16-byte aligned, with at least 3 floats in front: the gather's 16-byte
+  // loads may start 3 floats before a box (those values are dropped)
+  a.arena = reinterpret_cast<float*>(
+      (reinterpret_cast<uintptr_t>(work + 3) + 15) & ~uintptr_t(15));
+  const long long arena_floats = (long long)d.B * g.nbricks * a.slot;
+  a.meta = reinterpret_cast<int*>(a.arena + arena_floats);
   a.ctr = a.meta + 8LL * d.B * g.nbricks;
+  a.vec4 = d.nz % 4 == 0;
+  for (int c = 0; c < C; ++c)
+    if (reinterpret_cast<uintptr_t>(mesh[c]) % 16 != 0) a.vec4 = 0;
   a.X = X;
   a.w = w;
   a.wstride = wstride;
@@ -619,16 +714,22 @@ int launch_brick_paint(float* const* mesh, int C, const float* X,
   PMX_LAUNCH_CHECK();
   {
     ProfScope prof_(C == 1 ? kProfPaintGather : kProfPaintWGather, s);
-    const int tx = C == 1 ? kGatherTx1 : kGatherTx3;
-    const int nt = ((d.nx + tx - 1) / tx) * ((d.ny + kTile - 1) / kTile) *
-                   ((d.nz + kTile - 1) / kTile);
-    dim3 grid(nt, d.B);
-    if (C == 1)
-      hipLaunchKernelGGL((k_brick_gather<1, kGatherTx1>), grid, dim3(256), 0,
-                         s, a);
-    else
-      hipLaunchKernelGGL((k_brick_gather<3, kGatherTx3>), grid, dim3(256), 0,
-                         s, a);
+    // tiles of 16 planes where they fill the chip four times over (1024
+    // workgroups), else of 8 (two workgroups per CU or more), else of 4: at
+    // 1024 tiles of 16 (16 x 64^3) 25.8 us against 29.0 with 8 and 37.8 with
+    // 4, at 512 (128^3) 24.4 / 21.5 / 27.2, at 64 (64^3) 17.1 / 13.9 / 12.5.
+    // The three channels always take 4, 72 VGPRs against 106 with 8: 312 us
+    // against 324 at 256^3, 29.4 against 31.3 at 128 x 160 x 96.
+    const long long yz = (long long)((d.ny + kTile - 1) / kTile) *
+                         ((d.nz + kTile - 1) / kTile);
+    const long long t16 = (d.nx + 15) / 16 * yz * d.B;
+    const int px = t16 < 256 || C == 3 ? 1 : (t16 < 1024 ? 2 : 4);
+    dim3 grid((unsigned)((d.nx + 4 * px - 1) / (4 * px) * yz), d.B);
+    auto kern = C == 1 ? (px == 1   ? k_brick_gather<1, 1>
+                          : px == 2 ? k_brick_gather<1, 2>
+                                    : k_brick_gather<1, 4>)
+                       : k_brick_gather<3, 1>;
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a);
     PMX_LAUNCH_CHECK();
     const long long nq = (long long)d.B * g.nbricks;
     const dim3 sgrid((unsigned)std::min<long long>(nq, 256));
