@@ -1,0 +1,383 @@
+// Force readout of the particle grid straight from the potential, for gfx950.
+//
+// F = fac * readout(D phi), D the fourth-order central difference of
+// stencil.hip, phi the potential: the same values as the force mesh of
+// k_grad_mesh read by k_readout_kick_drift (cic.hip), without that mesh.
+// One workgroup takes one brick of the particle grid (particles that start
+// close stay close), loads the box of potential cells its particles' stencils
+// reach into LDS, and every particle forms the gradient at its 8 corners
+// there; closing kick, opening kick and drift follow in registers.
+//
+// What bounds it: the LDS reads (56 potential values per particle as 28
+// two-float reads; late positions spread them unevenly over the banks, 10
+// clocks a read instead of 4) and the VALU work (about 230 operations per
+// particle and 120 per thread for the fill), each about 140 of the 252 us it
+// takes at 256^3, then the particle streams (48 bytes per particle).  The
+// gradient mesh it replaces costs 12 bytes per cell written and 8 scattered
+// 12-byte gathers per particle; the potential boxes overlap (about 2.7 times
+// the mesh at a = 0.5) but are a third of the bytes and come from the 256 MB
+// cache in rows of whole quads.  Gradient + readout before -> here, one force
+// evaluation: 256^3 (a = 0.1 to 1) 327 -> 252 us, 512^3 (a = 0.5) 2760 ->
+// 1683, 16 x 64^3 73 -> 53; at 32^3 to 64^3 the two kernels took 8 to 11 us
+// against 11 here, but one launch less makes the run 1 to 3 % faster.
+#include "pmx_internal.h"
+
+namespace pmx {
+
+constexpr float kD1 = 2.0f / 3.0f, kD2 = 1.0f / 12.0f;
+static __device__ __forceinline__ float dstencil(float m2, float m1, float p1,
+                                                 float p2) {
+  return kD1 * (p1 - m1) - kD2 * (p2 - m2);
+}
+
+// n / d by one high multiplication with m = ceil(2^32 / d), d >= 2: exact while
+// n d < 2^32 (here n < 2^14 quads, d < 2^12)
+static __device__ __forceinline__ unsigned magic(unsigned d) {
+  return 0xffffffffu / d + 1u;
+}
+
+static __device__ __forceinline__ bool finite_pos(float x, float y, float z) {
+  return fabsf(x) < 1.0e9f && fabsf(y) < 1.0e9f && fabsf(z) < 1.0e9f;
+}
+
+typedef float V4 __attribute__((ext_vector_type(4)));
+typedef float V2 __attribute__((ext_vector_type(2)));
+typedef float V2u __attribute__((ext_vector_type(2), aligned(4)));
+
+// Gradient readout at one particle.  pair(a, b, c) is the potential at the
+// lower corner + (a, b, c) and + (a, b, c + 1), a, b, c in -2 .. 3 with one
+// of a, b outside 0 .. 1 only where c = 0: 28 loads of two values for the 56
+// cells of the 8 corners' differences.  Each difference and the order of
+// their weighted sum are those of k_grad_mesh and k_readout_kick_drift.
+template <class Pair>
+static __device__ __forceinline__ void grad_readout(const Pair& pair, float x,
+                                                    float y, float z,
+                                                    float (&out)[3]) {
+  constexpr int OX[8] = {0, 1, 0, 0, 1, 1, 0, 1};
+  constexpr int OY[8] = {0, 0, 1, 0, 1, 0, 1, 1};
+  constexpr int OZ[8] = {0, 0, 0, 1, 0, 1, 1, 1};
+  V2 vx[6][2], vy[2][6], vz[2][2][3];
+#pragma unroll
+  for (int e = 0; e < 6; ++e)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) vx[e][b] = pair(e - 2, b, 0);
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int e = 0; e < 6; ++e)
+      vy[a][e] = e == 2 || e == 3 ? vx[a + 2][e - 2] : pair(a, e - 2, 0);
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      vz[a][b][0] = pair(a, b, -2);
+      vz[a][b][1] = vx[a + 2][b];
+      vz[a][b][2] = pair(a, b, 2);
+    }
+  const float fx = floorf(x), fy = floorf(y), fz = floorf(z);
+  const float wx[2] = {1.0f - fabsf(x - fx), 1.0f - fabsf(x - (fx + 1.0f))};
+  const float wy[2] = {1.0f - fabsf(y - fy), 1.0f - fabsf(y - (fy + 1.0f))};
+  const float wz[2] = {1.0f - fabsf(z - fz), 1.0f - fabsf(z - (fz + 1.0f))};
+  float ax = 0.f, ay = 0.f, az = 0.f;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int a = OX[q], b = OY[q], c = OZ[q];
+    const float k = (wx[a] * wy[b]) * wz[c];
+    ax += dstencil(vx[a][b][c], vx[a + 1][b][c], vx[a + 3][b][c],
+                   vx[a + 4][b][c]) * k;
+    ay += dstencil(vy[a][b][c], vy[a][b + 1][c], vy[a][b + 3][c],
+                   vy[a][b + 4][c]) * k;
+    const V2* const l = vz[a][b];
+    az += dstencil(l[c / 2][c % 2], l[(c + 1) / 2][(c + 1) % 2],
+                   l[(c + 3) / 2][(c + 3) % 2], l[(c + 4) / 2][(c + 4) % 2]) *
+          k;
+  }
+  out[0] = ax;
+  out[1] = ay;
+  out[2] = az;
+}
+
+// element e of the 12-byte record at byte offset off of a uniform base: one
+// 32-bit address register
+static __device__ __forceinline__ float ldo(const float* base, unsigned off,
+                                            int e) {
+  return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) +
+                                        off)[e];
+}
+static __device__ __forceinline__ void sto(float v, float* base, unsigned off,
+                                           int e) {
+  reinterpret_cast<float*>(reinterpret_cast<char*>(base) + off)[e] = v;
+}
+
+constexpr int kBoxT = 512;  // 4 particles per thread, one after the other
+// LDS window, floats: two workgroups per CU.  A box longer than it is taken in
+// x windows that overlap by 5 planes: with 13568 floats and three workgroups
+// (80 VGPRs) the late boxes take two, 287 us against 262 at 256^3.
+constexpr int kBoxWin = 20224;
+
+// META: the bricks' boxes are those the paint of the same positions stored
+// (paint.hip), so the potential and the particles are loaded together;
+// otherwise the workgroup finds the box first.
+template <bool META>
+__global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
+    float* X, float* P, float* F, const float* __restrict__ phi,
+    const int* __restrict__ meta, MeshDims d, BrickGrid g, KickDrift c) {
+  __shared__ float win[kBoxWin];
+  __shared__ int red[META ? 1 : kBoxT / 64][6];
+  const int tid = threadIdx.x;
+  const int bid = (int)xcd_block(blockIdx.x, gridDim.x);
+  const int b = blockIdx.y;
+  int q0[3], cnt[3];
+  brick_block(g, bid, q0, cnt);
+  // z fastest, then x: the 4 rows of a wave read LDS rows a plane apart,
+  // whose pitch spreads them over the banks
+  const int cx = cnt[0], cz = cnt[2], nloc = cx * cnt[1] * cz;
+  // the brick's first particle (uniform); particle t of the brick is poff(t)
+  // bytes from there
+  const long long o0 =
+      3 * ((long long)b * d.N +
+           ((long long)q0[0] * g.gy + q0[1]) * g.gz + q0[2]);
+  auto poff = [&](int t) {
+    const int tt = t < nloc ? t : 0;
+    const int lz = tt % cz, q = tt / cz, lx = q % cx, ly = q / cx;
+    return 12u * (unsigned)((lx * g.gy + ly) * g.gz + lz);
+  };
+  // whole y planes of the brick per round of kBoxT particles: the next
+  // particle is a constant away (no division per particle)
+  const bool even = nloc % kBoxT == 0 && kBoxT % (cx * cz) == 0;
+  const unsigned pstep = even ? 12u * (unsigned)(kBoxT / (cx * cz)) * g.gz : 0u;
+  const bool kick = c.do_k2 || c.do_k1d;
+  const float* const Xl = (c.xin ? c.xin : X) + o0;
+  const float* const Pl = (c.pin ? c.pin : P) + o0;
+  const unsigned o_first = poff(tid);
+  unsigned on = o_first;
+  float xn[3], pn[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+  for (int e = 0; e < 3; ++e) xn[e] = ldo(Xl, on, e);
+  if (kick) {
+#pragma unroll
+    for (int e = 0; e < 3; ++e) pn[e] = ldo(Pl, on, e);
+  }
+  int lo[3], ext[3];  // first cell and extent of the brick's deposits
+  bool boxed;
+  if (META) {
+    const int* m = meta + 8LL * ((long long)b * g.nbricks + bid);
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      lo[e] = m[e];
+      ext[e] = m[3 + e];
+    }
+    boxed = ext[0] > 0;
+  } else {
+    int hi[3] = {INT_MIN, INT_MIN, INT_MIN};
+    lo[0] = lo[1] = lo[2] = INT_MAX;
+    for (int t = tid; t < nloc; t += kBoxT) {
+      const unsigned o = poff(t);
+      const float x[3] = {ldo(Xl, o, 0), ldo(Xl, o, 1), ldo(Xl, o, 2)};
+      if (!finite_pos(x[0], x[1], x[2])) continue;
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        const int f = (int)floorf(x[e]);
+        lo[e] = min(lo[e], f);
+        hi[e] = max(hi[e], f);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+#pragma unroll
+      for (int k = 32; k > 0; k >>= 1) {
+        lo[e] = min(lo[e], __shfl_xor(lo[e], k));
+        hi[e] = max(hi[e], __shfl_xor(hi[e], k));
+      }
+      if ((tid & 63) == 0) {
+        red[META ? 0 : tid >> 6][e] = lo[e];
+        red[META ? 0 : tid >> 6][3 + e] = hi[e];
+      }
+    }
+    __syncthreads();
+    boxed = true;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      int l = red[0][e], h = red[0][3 + e];
+#pragma unroll
+      for (int w = 1; w < (META ? 1 : kBoxT / 64); ++w) {
+        l = min(l, red[w][e]);
+        h = max(h, red[w][3 + e]);
+      }
+      l = __builtin_amdgcn_readfirstlane(l);
+      h = __builtin_amdgcn_readfirstlane(h);
+      // wider than the window in any case: not boxed
+      boxed = boxed && l <= h && (long long)h - l < 4096;
+      lo[e] = boxed ? l : 0;
+      ext[e] = boxed ? h - l + 2 : 0;
+    }
+  }
+  // the box of potential cells: 2 more on each side; in z from a multiple of
+  // 4 on, in whole quads, with an odd row pitch (the fill's rows start on other
+  // banks)
+  const int ez0 = (lo[2] - 2) & ~3;
+  const int nzq = (lo[2] + ext[2] + 2 - ez0 + 3) >> 2;  // quads per row
+  const int px = ext[0] + 4, py = ext[1] + 4, pz = 4 * nzq + 1;
+  // plane pitch 16 mod 64: the 4 planes a wave's 4 x 16 lanes read start 16
+  // banks apart
+  const int plane = ((py * pz + 47) & ~63) + 16;
+  // planes per window; a particle needs 6
+  const int hx = boxed && 6 * plane <= kBoxWin ? min(px, kBoxWin / plane) : 0;
+  // rows and planes wrap at most once (every box not longer than the sides)
+  const bool once = px <= d.nx && py <= d.ny;
+  const float* const pm =
+      phi + (long long)b * ((long long)d.nx * d.ny * d.nz);
+  const long long tot = (long long)d.B * d.N;
+  // without a box every particle reads the mesh, in one round
+  const int rounds = hx >= 6 ? px - 5 : 1, step = hx >= 6 ? hx - 5 : 1;
+  unsigned done = 0;
+  for (int s0 = 0; s0 < rounds; s0 += step) {
+    int nxw = 0;
+    if (hx >= 6) {
+      nxw = min(hx, px - s0);
+      const int x0 = imod(lo[0] - 2 + s0, d.nx), y0 = imod(lo[1] - 2, d.ny),
+                z0 = imod(ez0, d.nz);
+      const int rows = nxw * py;
+      const unsigned my = magic(py);
+      if (s0 > 0) __syncthreads();  // the window is reused
+      // 8 lanes of quads per row, kBoxT / 8 rows at a time
+      for (int zq = tid & 7; zq < nzq; zq += 8) {
+        int z = z0 + 4 * zq;
+        while (z >= d.nz) z -= d.nz;  // a box may be longer than the side
+        constexpr int U = 8;  // loads in flight per thread
+        for (int r0 = tid >> 3; r0 < rows; r0 += kBoxT / 8 * U) {
+          V4 v[U];
+          int at[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const unsigned r = min(r0 + u * (kBoxT / 8), rows - 1);
+            const unsigned xx = __umulhi(r, my);
+            unsigned y = r - xx * py, x = x0 + xx;
+            at[u] = (int)(xx * plane + y * pz);
+            y += y0;
+            if (once) {
+              y = min(y, y - (unsigned)d.ny);
+              x = min(x, x - (unsigned)d.nx);
+            } else {
+              y %= (unsigned)d.ny;
+              x %= (unsigned)d.nx;
+            }
+            // 32-bit byte offset: a member has at most 2^30 cells
+            const unsigned off = 4u * ((x * d.ny + y) * d.nz + (unsigned)z);
+            v[u] = *reinterpret_cast<const V4*>(
+                reinterpret_cast<const char*>(pm) + off);
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int r = r0 + u * (kBoxT / 8);
+            if (r < rows) {
+              float* const w = win + at[u] + 4 * zq;
+#pragma unroll
+              for (int q = 0; q < 4; ++q) w[q] = v[u][q];
+            }
+          }
+        }
+      }
+      __syncthreads();
+    }
+#pragma unroll 1
+    for (int u = 0; u < 4; ++u) {
+      const int t = tid + u * kBoxT;
+      const unsigned o = on;
+      float x[3], p[3];
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        x[e] = xn[e];
+        p[e] = pn[e];
+      }
+      // the next particle's loads (the first one's again for a next window)
+      on = u == 3 ? o_first : (even ? on + pstep : poff(t + kBoxT));
+#pragma unroll
+      for (int e = 0; e < 3; ++e) xn[e] = ldo(Xl, on, e);
+      if (kick) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e) pn[e] = ldo(Pl, on, e);
+      }
+      if (t >= nloc || (done >> u & 1)) continue;
+      float r[3] = {0.f, 0.f, 0.f};
+      if (finite_pos(x[0], x[1], x[2])) {
+        const int ix = (int)floorf(x[0]), iy = (int)floorf(x[1]),
+                  iz = (int)floorf(x[2]);
+        if (hx >= 6) {
+          const int i = ix - lo[0] - s0;
+          if (i < 0 || i + 5 >= nxw) continue;  // another window's
+          const float* const w =
+              win + i * plane + (iy - lo[1]) * pz + (iz - 2 - ez0);
+          grad_readout(
+              [&](int a, int bb, int cc) -> V2 {
+                return *reinterpret_cast<const V2u*>(
+                    w + (a + 2) * plane + (bb + 2) * pz + cc + 2);
+              },
+              x[0], x[1], x[2], r);
+        } else {
+          grad_readout(
+              [&](int a, int bb, int cc) -> V2 {
+                const float* const w =
+                    pm + ((unsigned)imod(ix + a, d.nx) * d.ny +
+                          (unsigned)imod(iy + bb, d.ny)) * d.nz;
+                return V2{w[imod(iz + cc, d.nz)], w[imod(iz + cc + 1, d.nz)]};
+              },
+              x[0], x[1], x[2], r);
+        }
+      }
+      done |= 1u << u;
+#pragma unroll
+      for (int e = 0; e < 3; ++e) r[e] *= c.fac;
+      auto store = [&](const float (&v)[3], float* q) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e) sto(v[e], q + o0, o, e);
+      };
+      if (!c.skip_f) store(r, F);
+      if (c.ckpt) {
+        store(x, c.ckpt);
+        store(r, c.ckpt + 6 * tot);
+      }
+      if (kick) {
+        if (c.do_k2) {
+#pragma unroll
+          for (int e = 0; e < 3; ++e) p[e] = p[e] + c.k2 * r[e];
+        }
+        if (c.ckpt) store(p, c.ckpt + 3 * tot);
+        if (c.do_k1d) {
+#pragma unroll
+          for (int e = 0; e < 3; ++e) {
+            p[e] = p[e] + c.k1 * r[e];
+            x[e] = x[e] + c.d * p[e];
+          }
+          store(x, c.xout ? c.xout : X);
+          if (c.xcopy) store(x, c.xcopy);
+        }
+        store(p, P);
+      }
+    }
+  }
+}
+
+bool readout_box_ok(const MeshDims& d, const KickDrift& c, const float* X,
+                    const float* P, const float* F, const float* phi) {
+  return c.f == 1.0f && c.gx == d.nx && c.gy == d.ny && c.gz == d.nz &&
+         d.nz % 4 == 0 && (long long)d.nx * d.ny * d.nz == d.N &&
+         reinterpret_cast<uintptr_t>(phi) % 16 == 0;
+}
+
+int launch_readout_box(float* X, float* P, float* F, const float* phi,
+                       const int* meta, const MeshDims& d, const KickDrift& c,
+                       hipStream_t s) {
+  if ((long long)d.B * d.N == 0) return kOk;
+  PMX_REQUIRE(readout_box_ok(d, c, X, P, F, phi),
+              "readout_box: one particle per cell, 16-byte aligned arrays");
+  ProfScope prof_(kProfReadoutKD, s);
+  const BrickGrid g = make_brick_grid(d.nx, d.ny, d.nz, 1);
+  auto kern = meta ? k_readout_box<true> : k_readout_box<false>;
+  hipLaunchKernelGGL(kern, dim3(g.nbricks, d.B), dim3(kBoxT), 0, s, X, P, F,
+                     phi, meta, d, g, c);
+  PMX_LAUNCH_CHECK();
+  return kOk;
+}
+
+}  // namespace pmx

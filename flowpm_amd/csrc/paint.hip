@@ -674,6 +674,18 @@ long long brick_work_floats(const MeshDims& d, const BrickGrid& g, int C) {
   return arena + meta + 16;
 }
 
+// 16-byte aligned, with at least 3 floats in front: the gather's 16-byte
+// loads may start 3 floats before a box (those values are dropped)
+static float* brick_arena(float* work) {
+  return reinterpret_cast<float*>(
+      (reinterpret_cast<uintptr_t>(work + 3) + 15) & ~uintptr_t(15));
+}
+const int* brick_meta(const MeshDims& d, const BrickGrid& g, int C,
+                      float* work) {
+  return reinterpret_cast<const int*>(
+      brick_arena(work) + (long long)d.B * g.nbricks * C * kBoxFloats);
+}
+
 int launch_brick_paint(float* const* mesh, int C, const float* X,
                        const float* w, int wstride, float wscale, float ps,
                        const MeshDims& d, const BrickGrid& g, float* work,
@@ -683,12 +695,8 @@ int launch_brick_paint(float* const* mesh, int C, const float* X,
   a.accum = accumulate ? 1 : 0;
   for (int c = 0; c < C; ++c) a.mesh[c] = mesh[c];
   a.slot = (long long)C * kBoxFloats;
-  // 16-byte aligned, with at least 3 floats in front: the gather's 16-byte
-  // loads may start 3 floats before a box (those values are dropped)
-  a.arena = reinterpret_cast<float*>(
-      (reinterpret_cast<uintptr_t>(work + 3) + 15) & ~uintptr_t(15));
-  const long long arena_floats = (long long)d.B * g.nbricks * a.slot;
-  a.meta = reinterpret_cast<int*>(a.arena + arena_floats);
+  a.arena = brick_arena(work);
+  a.meta = const_cast<int*>(brick_meta(d, g, C, work));
   a.ctr = a.meta + 8LL * d.B * g.nbricks;
   a.vec4 = d.nz % 4 == 0;
   for (int c = 0; c < C; ++c)

@@ -243,6 +243,7 @@ static int poisson_grad(const Plan& p, const float2* spec, int fwd,
 // (the reference's i g_d multiplier is the fourth-order central difference,
 // stencil.hip): one transform chain instead of three.  nc = 4: float4
 // cells (x, y, z, -), whose fourth slot the adjoint uses; nc = 3: packed.
+// nc = 0: the potential only.
 static int force_mesh_f4(const Plan& p, const float* rho, float2* w,
                          float* phi, float* f4, float rho_scale,
                          hipStream_t s, const PgdTerm* pgd, int nc = 4) {
@@ -267,7 +268,7 @@ static int force_mesh_f4(const Plan& p, const float* rho, float2* w,
   zj.n = 1;
   zj.j[0] = zc2r(w, phi, 1.0f, 0);
   PMX_TRY(launch_zpass_c2r(p, zj, s));
-  return launch_grad_mesh(p, phi, f4, nc, s);
+  return nc ? launch_grad_mesh(p, phi, f4, nc, s) : kOk;
 }
 
 // Three separate force meshes (the drop-in force / apply_longrange path).
@@ -797,10 +798,34 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
   auto force_k = [&](int k, const float* Xf, const NbodyWork& nw,
                      int nc) -> int {
     if (tape.phi_in)
-      return launch_grad_mesh(p, tape.phi_in + (long long)k * M, nw.f4, nc,
-                              s);
+      return nc ? launch_grad_mesh(p, tape.phi_in + (long long)k * M, nw.f4,
+                                   nc, s)
+                : kOk;
     return force_at(p, Xf, N, f, nw, s, nullptr, nc,
                     tape.phi ? tape.phi + (long long)k * M : nullptr);
+  };
+  // the force of slot k at Xf, its readout, kicks and drift (as kd says).
+  // fkeep: the tape's slot for the float4 force mesh, or null; without one
+  // the readout of one particle per cell takes the potential itself
+  auto force_readout = [&](int k, float* Xf, const float* Xforce,
+                           float* fkeep) -> int {
+    const NbodyWork nw = at(fkeep);
+    const float* phi = tape.phi_in ? tape.phi_in + (long long)k * M
+                       : tape.phi  ? tape.phi + (long long)k * M
+                                   : nw.rho;
+    if (!fkeep && readout_box_ok(md, kd, Xf, P, F, phi)) {
+      PMX_TRY(force_k(k, Xforce, nw, 0));
+      // the boxes of the paint just made, where there was one
+      const int* meta =
+          tape.phi_in
+              ? nullptr
+              : brick_meta(md, make_brick_grid(md.nx, md.ny, md.nz, 1), 1,
+                           nw.brick);
+      return launch_readout_box(Xf, P, F, phi, meta, md, kd, s);
+    }
+    const int nc = fkeep ? 4 : 3;
+    PMX_TRY(force_k(k, Xforce, nw, nc));
+    return launch_readout_kick_drift(Xf, P, F, mesh_nc(nw.f4, nc), md, kd, s);
   };
   // a force mesh the tape keeps is float4 (the reverse sweep stores the
   // density cotangent in its fourth slot); one only the readout reads is
@@ -808,9 +833,6 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
   if (jump) {
     const float* Xj = src ? src : X;  // the jump-start force's positions
     PMX_TRY(keep_x(tape.xj, Xj));
-    const NbodyWork nw = at(tape.fj);
-    const int nc = tape.fj ? 4 : 3;
-    PMX_TRY(force_k(0, Xj, nw, nc));
     kd.do_k2 = 0;
     kd.do_k1d = (b0 < b1);
     if (kd.do_k1d) {
@@ -820,8 +842,7 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
     }
     kd.xin = src;
     kd.pin = src ? src + BN3 : nullptr;
-    PMX_TRY(launch_readout_kick_drift(X, P, F, mesh_nc(nw.f4, nc), md,
-                                      kd, s));
+    PMX_TRY(force_readout(0, X, Xj, tape.fj));
     kd.xin = kd.pin = nullptr;
     if (kd.do_k1d && kd.xout) Xc = kd.xout;
   } else if (b0 < b1) {
@@ -859,9 +880,6 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
     } else if (!x_kept) {
       PMX_TRY(keep_x(xslot(i), Xc));
     }
-    const NbodyWork nw = at(tape.fs ? tape.fs + slot * 4 * M : nullptr);
-    const int nc = tape.fs ? 4 : 3;
-    PMX_TRY(force_k(1 + i, Xc, nw, nc));
     kd.do_k2 = 1;
     kd.k2 = (float)coef[3 * i + 2];
     kd.do_k1d = (i + 1 < b1);
@@ -877,8 +895,8 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
     kd.ckpt = (ck_out && kd.do_k1d && (i + 1 - b0) % ck_every == 0)
                   ? ck_out + (long long)((i + 1 - b0) / ck_every - 1) * 3 * BN3
                   : nullptr;
-    PMX_TRY(launch_readout_kick_drift(Xc, P, F, mesh_nc(nw.f4, nc), md,
-                                      kd, s));
+    PMX_TRY(force_readout(1 + i, Xc, Xc,
+                          tape.fs ? tape.fs + slot * 4 * M : nullptr));
     if (kd.do_k1d && kd.xout) Xc = kd.xout;
   }
   if (Xc != X && !tape.x_from_tape) {

@@ -271,6 +271,15 @@ int launch_readout_kick_drift(float* X, float* P, float* F, const Mesh3& m,
                               const MeshDims& d, const KickDrift& c,
                               hipStream_t s);
 
+// The same from the potential (boxread.hip), for one particle per cell
+// (c.f == 1, the particle grid the mesh's own) and 16-byte aligned arrays.
+bool readout_box_ok(const MeshDims& d, const KickDrift& c, const float* X,
+                    const float* P, const float* F, const float* phi);
+// meta: the boxes the paint of the same positions left (brick_meta), or null.
+int launch_readout_box(float* X, float* P, float* F, const float* phi,
+                       const int* meta, const MeshDims& d, const KickDrift& c,
+                       hipStream_t s);
+
 // out += scale * sum_p sum_c G[p][c] readout(m_c, X_p * f) (float64)
 int launch_readout_dot(const float* X, const float* G, const Mesh3& m,
                        const MeshDims& d, float f, double* out, double scale,
@@ -318,6 +327,9 @@ int launch_power_bins_adj(const Plan& p, float2* spec, const double* kx,
 // Lagrangian-brick paint (paint.hip).
 bool brick_paint_ok(const MeshDims& d, const BrickGrid& g);
 long long brick_work_floats(const MeshDims& d, const BrickGrid& g, int C);
+// where launch_brick_paint leaves the boxes of its bricks (8 ints each)
+const int* brick_meta(const MeshDims& d, const BrickGrid& g, int C,
+                      float* work);
 // mesh[c] = sum_p w[p*wstride+c]*wscale * CIC(X*ps) (every cell written;
 // accumulate: mesh[c] += instead)
 int launch_brick_paint(float* const* mesh, int C, const float* X,
