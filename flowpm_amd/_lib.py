@@ -83,6 +83,10 @@ _SIGS = {
                                     _i, _i, _f, _f, _f, _f, _f, _i, _vp]),
     "pmx_nbody_work_floats": (_ll, [_vp]),
     "pmx_nbody_run": (_i, [_vp, _vp, _ll, _f, _f, _dp, _i, _i, _i, _vp, _vp]),
+    "pmx_nbody_run_from": (_i, [_vp, _vp, _vp, _ll, _f, _f, _dp, _i, _vp, _i,
+                                _vp, _vp]),
+    "pmx_nbody_adjoint_from": (_i, [_vp, _vp, _i, _i, _ll, _f, _f, _dp, _vp,
+                                    _vp, _vp, _vp, _vp]),
     "pmx_nbody_run_noalloc": (_i, [_vp, _vp, _ll, _f, _f, _dp, _i, _i, _i,
                                    _vp]),
     "pmx_nbody_run_pgd": (_i, [_vp, _vp, _ll, _f, _f, _dp,

@@ -45,8 +45,9 @@ class _Group:
       # holds the cotangent of the final state, gstate receives the
       # cotangent of the initial state
       h = self.plan.handle
-      self.tape = torch.empty(L.pmx_nbody_tape_floats(h, self.N, self.nsteps),
-                              dtype=torch.float32, device=dev)
+      self.compact = tfpm._compact()
+      self.tape = tfpm._tape(self.plan, self.N, self.nsteps, self.compact,
+                             dev)
       self.adj_work = torch.empty(L.pmx_nbody_adj_work_floats(h, self.N, 0),
                                   dtype=torch.float32, device=dev)
       self.gfinal = torch.zeros_like(self.state)
@@ -61,16 +62,15 @@ class _Group:
 
   def run_grad(self, stream):
     """Taped forward run, then the hand-written reverse sweep of the
-    cotangent in gfinal (copied into gstate, which the sweep turns into the
-    initial state's cotangent)."""
-    _lib.call("pmx_nbody_run_taped", self.plan.handle, _lib.ptr(self.state),
-              self.N, self.f, self.fac, self.cptr, self.nsteps,
-              _lib.ptr(self.tape), _lib.ptr(self.work), stream)
-    self.gstate.copy_(self.gfinal)
-    _lib.call("pmx_nbody_adjoint_taped", self.plan.handle,
-              _lib.ptr(self.tape), self.nsteps, self.N, self.f, self.fac,
-              self.cptr, _lib.ptr(self.gstate), _lib.ptr(self.adj_work),
-              None, stream)
+    cotangent in gfinal into the initial state's, gstate."""
+    _lib.call("pmx_nbody_run_%staped" % ("compact_" if self.compact else ""),
+              self.plan.handle, _lib.ptr(self.state), self.N, self.f,
+              self.fac, self.cptr, self.nsteps, _lib.ptr(self.tape),
+              _lib.ptr(self.work), stream)
+    _lib.call("pmx_nbody_adjoint_from", self.plan.handle,
+              _lib.ptr(self.tape), 1 if self.compact else 0, self.nsteps,
+              self.N, self.f, self.fac, self.cptr, _lib.ptr(self.gfinal),
+              _lib.ptr(self.gstate), _lib.ptr(self.adj_work), None, stream)
 
 
 class BatchedNbody:

@@ -1,4 +1,5 @@
-// Force readout of the particle grid straight from the potential, for gfx950.
+// Force readout of the particle grid straight from the potential, for gfx950
+// (part of cic.hip).
 //
 // F = fac * readout(D phi), D the fourth-order central difference of
 // stencil.hip, phi the potential: the same values as the force mesh of
@@ -20,6 +21,7 @@
 // evaluation: 256^3 (a = 0.1 to 1) 327 -> 252 us, 512^3 (a = 0.5) 2760 ->
 // 1683, 16 x 64^3 73 -> 53; at 32^3 to 64^3 the two kernels took 8 to 11 us
 // against 11 here, but one launch less makes the run 1 to 3 % faster.
+#pragma once
 #include "pmx_internal.h"
 
 namespace pmx {
@@ -44,11 +46,12 @@ typedef float V4 __attribute__((ext_vector_type(4)));
 typedef float V2 __attribute__((ext_vector_type(2)));
 typedef float V2u __attribute__((ext_vector_type(2), aligned(4)));
 
-// Gradient readout at one particle.  pair(a, b, c) is the potential at the
-// lower corner + (a, b, c) and + (a, b, c + 1), a, b, c in -2 .. 3 with one
-// of a, b outside 0 .. 1 only where c = 0: 28 loads of two values for the 56
-// cells of the 8 corners' differences.  Each difference and the order of
-// their weighted sum are those of k_grad_mesh and k_readout_kick_drift.
+// Gradient readout at one particle: the differences at the 8 corners of its
+// cell and their weighted sum, in the corner order of cic.hip.
+// pair(a, b, c) is the potential at the lower corner + (a, b, c) and
+// + (a, b, c + 1), a, b, c in -2 .. 3 with one of a, b outside 0 .. 1 only
+// where c = 0: 28 loads of two values for the 56 cells of the differences,
+// which are those of k_grad_mesh, as the sum is k_readout_kick_drift's.
 template <class Pair>
 static __device__ __forceinline__ void grad_readout(const Pair& pair, float x,
                                                     float y, float z,
@@ -115,6 +118,119 @@ constexpr int kBoxT = 512;  // 4 particles per thread, one after the other
 // (80 VGPRs) the late boxes take two, 287 us against 262 at 256^3.
 constexpr int kBoxWin = 20224;
 
+// A box of mesh cells in the LDS window: planes of py rows of nzq quads, row
+// pitch pz floats, plane pitch plane floats.
+struct Box {
+  int z0, nzq, y0, py, x0, px;  // first cells (unwrapped) and lengths
+  int pz, plane;
+};
+// the cells lo - h .. lo + ext - 1 + h per axis (ext: lower corners and their
+// upper neighbours), in z widened to whole quads from a multiple of 4 on.
+// The row pitch is odd (the fill's rows start on other banks), the plane
+// pitch 16 mod 64: the 4 planes a wave's 4 x 16 lanes read start 16 banks
+// apart.
+static __device__ __forceinline__ Box make_box(const int (&lo)[3],
+                                               const int (&ext)[3], int h) {
+  Box q;
+  q.x0 = lo[0] - h;
+  q.px = ext[0] + 2 * h;
+  q.y0 = lo[1] - h;
+  q.py = ext[1] + 2 * h;
+  q.z0 = (lo[2] - h) & ~3;
+  q.nzq = (lo[2] + ext[2] + h - q.z0 + 3) >> 2;
+  q.pz = 4 * q.nzq + 1;
+  q.plane = ((q.py * q.pz + 47) & ~63) + 16;
+  return q;
+}
+
+// Planes s0 .. s0 + np - 1 of the box of mesh pm into win: 8 lanes of quads
+// per row, T / 8 rows at a time, U loads in flight per thread.
+template <int T>
+static __device__ __forceinline__ void fill_box(float* win, const float* pm,
+                                                const MeshDims& d,
+                                                const Box& q, int s0, int np) {
+  constexpr int U = 8;
+  const int x0 = imod(q.x0 + s0, d.nx), y0 = imod(q.y0, d.ny),
+            z0 = imod(q.z0, d.nz);
+  // rows and planes wrap at most once (the box is not longer than the sides)
+  const bool once = q.px <= d.nx && q.py <= d.ny;
+  const int rows = np * q.py;
+  const unsigned my = magic(q.py);
+  for (int zq = threadIdx.x & 7; zq < q.nzq; zq += 8) {
+    int z = z0 + 4 * zq;
+    while (z >= d.nz) z -= d.nz;  // a box may be longer than the side
+    for (int r0 = threadIdx.x >> 3; r0 < rows; r0 += T / 8 * U) {
+      V4 v[U];
+      int at[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const unsigned r = min(r0 + u * (T / 8), rows - 1);
+        const unsigned xx = __umulhi(r, my);
+        unsigned y = r - xx * q.py, x = x0 + xx;
+        at[u] = (int)(xx * q.plane + y * q.pz);
+        y += y0;
+        if (once) {
+          y = min(y, y - (unsigned)d.ny);
+          x = min(x, x - (unsigned)d.nx);
+        } else {
+          y %= (unsigned)d.ny;
+          x %= (unsigned)d.nx;
+        }
+        // 32-bit byte offset: a member has at most 2^30 cells
+        const unsigned off = 4u * ((x * d.ny + y) * d.nz + (unsigned)z);
+        v[u] = *reinterpret_cast<const V4*>(
+            reinterpret_cast<const char*>(pm) + off);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (r0 + u * (T / 8) < rows) {
+          float* const w = win + at[u] + 4 * zq;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[e] = v[u][e];
+        }
+      }
+    }
+  }
+}
+
+// potential pairs of the cell whose lower corner is (ix, iy, iz), from the
+// mesh itself: the wrapped offsets of the 6 planes, rows and cells, taken once
+struct MeshPair {
+  const float* pm;
+  unsigned ox[6], oy[6], oz[6];
+  __device__ __forceinline__ MeshPair(const float* pm_, int ix, int iy, int iz,
+                                      const MeshDims& d)
+      : pm(pm_) {
+    axis(ox, ix, d.nx, (unsigned)d.ny * d.nz);
+    axis(oy, iy, d.ny, (unsigned)d.nz);
+    axis(oz, iz, d.nz, 1u);
+  }
+  static __device__ __forceinline__ void axis(unsigned (&o)[6], int i, int n,
+                                              unsigned stride) {
+    // sides are 8 or more: - 2 .. 3 wraps at most once
+    const int w = imod(i, n);
+#pragma unroll
+    for (int e = 0; e < 6; ++e) {
+      int v = w + e - 2;
+      v = v < 0 ? v + n : (v >= n ? v - n : v);
+      o[e] = (unsigned)v * stride;
+    }
+  }
+  __device__ __forceinline__ V2 operator()(int a, int b, int c) const {
+    const unsigned r = ox[a + 2] + oy[b + 2];
+    return V2{pm[r + oz[c + 2]], pm[r + oz[c + 3]]};
+  }
+};
+// and from a window whose cell (ix - 2, iy - 2, iz - 2) is w
+struct WinPair {
+  const float* w;
+  int plane, pz;
+  __device__ __forceinline__ V2 operator()(int a, int b, int c) const {
+    return *reinterpret_cast<const V2u*>(w + (a + 2) * plane + (b + 2) * pz +
+                                         c + 2);
+  }
+};
+
 // META: the bricks' boxes are those the paint of the same positions stored
 // (paint.hip), so the potential and the particles are loaded together;
 // otherwise the workgroup finds the box first.
@@ -129,8 +245,7 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
   const int b = blockIdx.y;
   int q0[3], cnt[3];
   brick_block(g, bid, q0, cnt);
-  // z fastest, then x: the 4 rows of a wave read LDS rows a plane apart,
-  // whose pitch spreads them over the banks
+  // z fastest, then x: the 4 rows of a wave are a plane apart in LDS
   const int cx = cnt[0], cz = cnt[2], nloc = cx * cnt[1] * cz;
   // the brick's first particle (uniform); particle t of the brick is poff(t)
   // bytes from there
@@ -147,6 +262,7 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
   const bool even = nloc % kBoxT == 0 && kBoxT % (cx * cz) == 0;
   const unsigned pstep = even ? 12u * (unsigned)(kBoxT / (cx * cz)) * g.gz : 0u;
   const bool kick = c.do_k2 || c.do_k1d;
+  const bool useP = kick || c.copy_xp;
   const float* const Xl = (c.xin ? c.xin : X) + o0;
   const float* const Pl = (c.pin ? c.pin : P) + o0;
   const unsigned o_first = poff(tid);
@@ -154,7 +270,7 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
   float xn[3], pn[3] = {0.f, 0.f, 0.f};
 #pragma unroll
   for (int e = 0; e < 3; ++e) xn[e] = ldo(Xl, on, e);
-  if (kick) {
+  if (useP) {
 #pragma unroll
     for (int e = 0; e < 3; ++e) pn[e] = ldo(Pl, on, e);
   }
@@ -212,72 +328,22 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
       ext[e] = boxed ? h - l + 2 : 0;
     }
   }
-  // the box of potential cells: 2 more on each side; in z from a multiple of
-  // 4 on, in whole quads, with an odd row pitch (the fill's rows start on other
-  // banks)
-  const int ez0 = (lo[2] - 2) & ~3;
-  const int nzq = (lo[2] + ext[2] + 2 - ez0 + 3) >> 2;  // quads per row
-  const int px = ext[0] + 4, py = ext[1] + 4, pz = 4 * nzq + 1;
-  // plane pitch 16 mod 64: the 4 planes a wave's 4 x 16 lanes read start 16
-  // banks apart
-  const int plane = ((py * pz + 47) & ~63) + 16;
+  const Box q = make_box(lo, ext, 2);
   // planes per window; a particle needs 6
-  const int hx = boxed && 6 * plane <= kBoxWin ? min(px, kBoxWin / plane) : 0;
-  // rows and planes wrap at most once (every box not longer than the sides)
-  const bool once = px <= d.nx && py <= d.ny;
+  const int hx =
+      boxed && 6 * q.plane <= kBoxWin ? min(q.px, kBoxWin / q.plane) : 0;
   const float* const pm =
       phi + (long long)b * ((long long)d.nx * d.ny * d.nz);
   const long long tot = (long long)d.B * d.N;
   // without a box every particle reads the mesh, in one round
-  const int rounds = hx >= 6 ? px - 5 : 1, step = hx >= 6 ? hx - 5 : 1;
+  const int rounds = hx >= 6 ? q.px - 5 : 1, step = hx >= 6 ? hx - 5 : 1;
   unsigned done = 0;
   for (int s0 = 0; s0 < rounds; s0 += step) {
     int nxw = 0;
     if (hx >= 6) {
-      nxw = min(hx, px - s0);
-      const int x0 = imod(lo[0] - 2 + s0, d.nx), y0 = imod(lo[1] - 2, d.ny),
-                z0 = imod(ez0, d.nz);
-      const int rows = nxw * py;
-      const unsigned my = magic(py);
+      nxw = min(hx, q.px - s0);
       if (s0 > 0) __syncthreads();  // the window is reused
-      // 8 lanes of quads per row, kBoxT / 8 rows at a time
-      for (int zq = tid & 7; zq < nzq; zq += 8) {
-        int z = z0 + 4 * zq;
-        while (z >= d.nz) z -= d.nz;  // a box may be longer than the side
-        constexpr int U = 8;  // loads in flight per thread
-        for (int r0 = tid >> 3; r0 < rows; r0 += kBoxT / 8 * U) {
-          V4 v[U];
-          int at[U];
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const unsigned r = min(r0 + u * (kBoxT / 8), rows - 1);
-            const unsigned xx = __umulhi(r, my);
-            unsigned y = r - xx * py, x = x0 + xx;
-            at[u] = (int)(xx * plane + y * pz);
-            y += y0;
-            if (once) {
-              y = min(y, y - (unsigned)d.ny);
-              x = min(x, x - (unsigned)d.nx);
-            } else {
-              y %= (unsigned)d.ny;
-              x %= (unsigned)d.nx;
-            }
-            // 32-bit byte offset: a member has at most 2^30 cells
-            const unsigned off = 4u * ((x * d.ny + y) * d.nz + (unsigned)z);
-            v[u] = *reinterpret_cast<const V4*>(
-                reinterpret_cast<const char*>(pm) + off);
-          }
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const int r = r0 + u * (kBoxT / 8);
-            if (r < rows) {
-              float* const w = win + at[u] + 4 * zq;
-#pragma unroll
-              for (int q = 0; q < 4; ++q) w[q] = v[u][q];
-            }
-          }
-        }
-      }
+      fill_box<kBoxT>(win, pm, d, q, s0, nxw);
       __syncthreads();
     }
 #pragma unroll 1
@@ -294,7 +360,7 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
       on = u == 3 ? o_first : (even ? on + pstep : poff(t + kBoxT));
 #pragma unroll
       for (int e = 0; e < 3; ++e) xn[e] = ldo(Xl, on, e);
-      if (kick) {
+      if (useP) {
 #pragma unroll
         for (int e = 0; e < 3; ++e) pn[e] = ldo(Pl, on, e);
       }
@@ -306,23 +372,12 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
         if (hx >= 6) {
           const int i = ix - lo[0] - s0;
           if (i < 0 || i + 5 >= nxw) continue;  // another window's
-          const float* const w =
-              win + i * plane + (iy - lo[1]) * pz + (iz - 2 - ez0);
-          grad_readout(
-              [&](int a, int bb, int cc) -> V2 {
-                return *reinterpret_cast<const V2u*>(
-                    w + (a + 2) * plane + (bb + 2) * pz + cc + 2);
-              },
-              x[0], x[1], x[2], r);
+          grad_readout(WinPair{win + i * q.plane + (iy - lo[1]) * q.pz +
+                                   (iz - 2 - q.z0),
+                               q.plane, q.pz},
+                       x[0], x[1], x[2], r);
         } else {
-          grad_readout(
-              [&](int a, int bb, int cc) -> V2 {
-                const float* const w =
-                    pm + ((unsigned)imod(ix + a, d.nx) * d.ny +
-                          (unsigned)imod(iy + bb, d.ny)) * d.nz;
-                return V2{w[imod(iz + cc, d.nz)], w[imod(iz + cc + 1, d.nz)]};
-              },
-              x[0], x[1], x[2], r);
+          grad_readout(MeshPair(pm, ix, iy, iz, d), x[0], x[1], x[2], r);
         }
       }
       done |= 1u << u;
@@ -333,6 +388,11 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
         for (int e = 0; e < 3; ++e) sto(v[e], q + o0, o, e);
       };
       if (!c.skip_f) store(r, F);
+      if (c.xkeep) store(x, c.xkeep);
+      if (c.copy_xp) {
+        store(x, X);
+        store(p, P);
+      }
       if (c.ckpt) {
         store(x, c.ckpt);
         store(r, c.ckpt + 6 * tot);

@@ -683,7 +683,10 @@ __global__ __launch_bounds__(256) void k_force_vjp_finish(
   const bool full = tiled || p0 + 256 <= tot;
   const bool upd = u.mode == 1 || u.mode == 2;
   const bool gin_gp = u.gin_scale != 0.0f;  // readout cotangent from gP
-  const bool ldgp = upd || gin_gp;
+  const bool cpgp = u.gpin && !upd;       // gP is copied
+  const bool ldgp = upd || gin_gp || cpgp;
+  const float* const gXl = u.gxin ? u.gxin : gX;
+  const float* const gPl = u.gpin ? u.gpin : gP;
   // particle streams: non-temporal (read once, kept out of L2 where the
   // gathered mesh is re-read by neighbouring blocks); a full block stages
   // them through LDS so every load and store is a contiguous run
@@ -696,8 +699,8 @@ __global__ __launch_bounds__(256) void k_force_vjp_finish(
       const long long o = stage_off(tiled, p0, u.gz, t + 256 * k);
       v[0][k] = __builtin_nontemporal_load(X + o);
       v[1][k] = gin_gp ? 0.0f : __builtin_nontemporal_load(gin + o);
-      v[2][k] = __builtin_nontemporal_load(gX + o);
-      v[3][k] = ldgp ? __builtin_nontemporal_load(gP + o) : 0.0f;
+      v[2][k] = __builtin_nontemporal_load(gXl + o);
+      v[3][k] = ldgp ? __builtin_nontemporal_load(gPl + o) : 0.0f;
       if (CG) v[NQ - 1][k] = __builtin_nontemporal_load(Xprev + o);
     }
 #pragma unroll
@@ -722,8 +725,8 @@ __global__ __launch_bounds__(256) void k_force_vjp_finish(
     for (int c = 0; c < 3; ++c) {
       xv[c] = X[3 * q + c];
       gfv[c] = gin_gp ? 0.0f : gin[3 * q + c];
-      gxv[c] = gX[3 * q + c];
-      gpv[c] = ldgp ? gP[3 * q + c] : 0.0f;
+      gxv[c] = gXl[3 * q + c];
+      gpv[c] = ldgp ? gPl[3 * q + c] : 0.0f;
       xpv[c] = CG ? Xprev[3 * q + c] : 0.0f;
     }
   }
@@ -778,7 +781,7 @@ __global__ __launch_bounds__(256) void k_force_vjp_finish(
   for (int c = 0; c < 3; ++c) {
     g[c] = gxv[c] + f * s3[c];
     g[c] = g[c] + f * r3[c];
-    gp[c] = gpv[c] + u.d * g[c];
+    gp[c] = cpgp ? gpv[c] : gpv[c] + u.d * g[c];
     gf[c] = u.k1 * gp[c];
     if (u.mode == 2) gf[c] = gf[c] + u.k2prev * gp[c];
     if (u.mode == 3) gf[c] = 0.0f;
@@ -797,14 +800,15 @@ __global__ __launch_bounds__(256) void k_force_vjp_finish(
     for (int k = 0; k < 3; ++k) {
       const long long o = stage_off(tiled, p0, u.gz, t + 256 * k);
       __builtin_nontemporal_store(sh[0][t + 256 * k], gX + o);
-      if (upd) __builtin_nontemporal_store(sh[1][t + 256 * k], gP + o);
+      if (upd || cpgp)
+        __builtin_nontemporal_store(sh[1][t + 256 * k], gP + o);
       if (wgf) __builtin_nontemporal_store(sh[2][t + 256 * k], gF + o);
     }
   } else if (p < tot) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       gX[3 * p + c] = g[c];
-      if (upd) gP[3 * p + c] = gp[c];
+      if (upd || cpgp) gP[3 * p + c] = gp[c];
       if (wgf) gF[3 * p + c] = gf[c];
     }
   }
@@ -1059,3 +1063,5 @@ int launch_force_vjp_particles(float* gmx, float* gmy, float* gmz, float* dX,
 }
 
 }  // namespace pmx
+
+#include "box_readout.h"

@@ -492,6 +492,18 @@ __global__ void k_adj_update(float* __restrict__ gX, float* __restrict__ gP,
   }
 }
 
+// The state cotangent (gX, gP, gF + k2 gP) from another buffer.
+__global__ void k_adj_open(const float* __restrict__ src,
+                           float* __restrict__ dst, long long n, float k2) {
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
+       i += (long long)gridDim.x * blockDim.x) {
+    const float gp = src[n + i];
+    dst[i] = src[i];
+    dst[n + i] = gp;
+    dst[2 * n + i] = src[2 * n + i] + k2 * gp;
+  }
+}
+
 // Adjoint of k_lpt_assemble: per-component cotangent meshes of dx1 / dx2.
 __global__ void k_lpt_assemble_adj(const float* __restrict__ gstate,
                                    float* __restrict__ g1,
@@ -711,20 +723,29 @@ struct Tape {
   // numbers).  phi: the run stores them there; phi_in: the run takes its
   // force meshes from them (the gradient stencil) instead of painting and
   // transforming, as a checkpointed reverse sweep does when it recomputes
-  // a segment whose potentials the forward run kept.
+  // a segment whose potentials the forward run kept.  phi0: the slot that
+  // phi / phi_in point at.
   float* phi = nullptr;
   const float* phi_in = nullptr;
+  int phi0 = 0;
   // the caller reads the run's last positions from their slot: the state's
   // X is left as it is (a reverse sweep's scratch state)
   bool x_from_tape = false;
 };
 
+// One particle per cell in grid order: the readout and its adjoint work on
+// the potential itself (box_readout.h), so no force mesh is formed or kept.
+static bool box_run(const Plan& p, long long N, float f) {
+  return f == 1.0f && p.d.nz % 4 == 0 &&
+         N == (long long)p.d.nx * p.d.ny * p.d.nz;
+}
+
 // pgd (optional): (alpha, kl, ks) of every step; after the drift of step
 // i the positions move by the PGD displacement (tfpm.py:487-488).
-// src (optional, not with pgd, at least one step): the run starts from
-// this state (X, P, F) instead of the one in state, which it only writes:
-// the jump-start force and readout, or the first kick and drift, read src,
-// so no copy of it is needed.
+// src (optional, not with pgd, at least one step or the jump-start force):
+// the run starts from this state (X, P, F) instead of the one in state, which
+// it only writes: the jump-start force and readout, or the first kick and
+// drift, read src, so no copy of it is needed.
 // ck_out (optional, with ck_every >= 1; no PGD, no kept positions or force
 // meshes): the state after the closing kick of every step i with
 // (i + 1 - b0) % ck_every == 0 and i + 1 < b1 (the state a run ending at
@@ -736,9 +757,8 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
                      const Tape* tp = nullptr, const float* pgd = nullptr,
                      const float* src = nullptr, float* ck_out = nullptr,
                      int ck_every = 0) {
-  PMX_REQUIRE(!(src && (pgd || b0 >= b1)),
-              "nbody: a run from a separate state needs at least one step "
-              "and no PGD");
+  PMX_REQUIRE(!(src && (pgd || (b0 >= b1 && !jump))),
+              "nbody: a run from a separate state needs a force and no PGD");
   PMX_REQUIRE(!(ck_out && (ck_every < 1 || pgd ||
                            (tp && (tp->xs || tp->fs || tp->xp)))),
               "nbody: checkpoints are written by untaped runs without PGD "
@@ -773,6 +793,7 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
   kd.fac = fac;
   kd.f = f;
   particle_grid(p, N, f, &kd.gx, &kd.gy, &kd.gz);
+  const bool box = box_run(p, N, f);
   // slot of step i in the tape of the positions the drift produces (the
   // pre-correction ones with PGD), null when not kept
   auto xslot = [&](int i) -> float* {
@@ -797,12 +818,11 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
   // the potential when asked)
   auto force_k = [&](int k, const float* Xf, const NbodyWork& nw,
                      int nc) -> int {
+    const long long o = (long long)(k - tape.phi0) * M;
     if (tape.phi_in)
-      return nc ? launch_grad_mesh(p, tape.phi_in + (long long)k * M, nw.f4,
-                                   nc, s)
-                : kOk;
+      return nc ? launch_grad_mesh(p, tape.phi_in + o, nw.f4, nc, s) : kOk;
     return force_at(p, Xf, N, f, nw, s, nullptr, nc,
-                    tape.phi ? tape.phi + (long long)k * M : nullptr);
+                    tape.phi ? tape.phi + o : nullptr);
   };
   // the force of slot k at Xf, its readout, kicks and drift (as kd says).
   // fkeep: the tape's slot for the float4 force mesh, or null; without one
@@ -810,10 +830,11 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
   auto force_readout = [&](int k, float* Xf, const float* Xforce,
                            float* fkeep) -> int {
     const NbodyWork nw = at(fkeep);
-    const float* phi = tape.phi_in ? tape.phi_in + (long long)k * M
-                       : tape.phi  ? tape.phi + (long long)k * M
+    const long long o = (long long)(k - tape.phi0) * M;
+    const float* phi = tape.phi_in ? tape.phi_in + o
+                       : tape.phi  ? tape.phi + o
                                    : nw.rho;
-    if (!fkeep && readout_box_ok(md, kd, Xf, P, F, phi)) {
+    if (!fkeep && box) {
       PMX_TRY(force_k(k, Xforce, nw, 0));
       // the boxes of the paint just made, where there was one
       const int* meta =
@@ -832,7 +853,18 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
   // packed, 12 bytes per cell
   if (jump) {
     const float* Xj = src ? src : X;  // the jump-start force's positions
-    PMX_TRY(keep_x(tape.xj, Xj));
+    // the box readout keeps the positions and carries X and P of a run of
+    // no steps over itself
+    const bool carry = src && b0 >= b1;
+    if (box && !tape.fj) {
+      kd.xkeep = tape.xj;
+      kd.copy_xp = carry;
+    } else {
+      PMX_TRY(keep_x(tape.xj, Xj));
+      if (carry)
+        PMX_HIP_CHECK(hipMemcpyAsync(X, src, sizeof(float) * 2 * BN3,
+                                     hipMemcpyDeviceToDevice, s));
+    }
     kd.do_k2 = 0;
     kd.do_k1d = (b0 < b1);
     if (kd.do_k1d) {
@@ -844,6 +876,8 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
     kd.pin = src ? src + BN3 : nullptr;
     PMX_TRY(force_readout(0, X, Xj, tape.fj));
     kd.xin = kd.pin = nullptr;
+    kd.xkeep = nullptr;
+    kd.copy_xp = 0;
     if (kd.do_k1d && kd.xout) Xc = kd.xout;
   } else if (b0 < b1) {
     // opening kick + drift of the first step from the stored force
@@ -936,6 +970,9 @@ static int store_implicit_gf(float* gF, const float* gP, float* gf_scale,
 // the factor s with force cotangent s * gP (gF not stored).  On return it
 // says the same of the gF this update leaves: the grid path of the plain
 // (no PGD) force leaves it unstored.
+// phi (optional, no fm): the potential at X, from which the force mesh is
+// formed.  gsrc (optional, with box_run and update mode 3): gX, gP and gF are
+// read from this state and written to gX, gP, gF.
 static int force_vjp(const Plan& p, const float* X, float* gF, float* gX,
                      float* gP, long long N, float f, float fac,
                      const NbodyWork& nw, float* gm, float* fm,
@@ -943,19 +980,31 @@ static int force_vjp(const Plan& p, const float* X, float* gF, float* gX,
                      const PgdTerm* pgd = nullptr,
                      const float* gin = nullptr,
                      float* gf_scale = nullptr,
-                     const CoefDot* cd = nullptr, bool* cd_done = nullptr) {
+                     const CoefDot* cd = nullptr, bool* cd_done = nullptr,
+                     const float* phi = nullptr,
+                     const float* gsrc = nullptr) {
   const long long M = p.d.rows * p.d.nz;
   const long long Mb = (long long)p.d.nx * p.d.ny * p.d.nz;
   const long long BN3 = (long long)p.d.B * N * 3;
   if (gin || pgd) PMX_TRY(store_implicit_gf(gF, gP, gf_scale, BN3, s));
   const float gin_scale = gf_scale ? *gf_scale : 0.0f;
   // the readout's cotangent: gin, gF, or gin_scale * gP
-  const float* gc = gin ? gin : (gin_scale != 0.0f ? gP : gF);
+  const float* gc = gin     ? gin
+                    : gsrc  ? gsrc + 2 * BN3
+                    : gin_scale != 0.0f ? gP
+                                        : gF;
   const float wsc = gin_scale != 0.0f ? gin_scale * (fac / f) : fac / f;
   MeshDims md{p.d.B, p.d.nx, p.d.ny, p.d.nz, N};
   float* f4 = fm ? fm : nw.f4;
   const Mesh3 m = m3(f4);
-  if (!fm) PMX_TRY(force_at(p, X, N, f, nw, s, pgd));
+  if (pgd && !fm) PMX_TRY(force_at(p, X, N, f, nw, s, pgd));
+  if (!pgd && !fm && !phi) {
+    // the density buffer takes the potential's cotangent below, the second
+    // spectral buffer is free
+    float* const keep = reinterpret_cast<float*>(nw.w + p.d.S);
+    PMX_TRY(force_at(p, X, N, f, nw, s, nullptr, 0, keep));
+    phi = keep;
+  }
   float* gms[3] = {gm, gm + M, gm + 2 * M};
   const int rc3 = paint_meshes(p, gms, 3, X, gc, 3, wsc, N, f, nw.brick, s);
   if (rc3 != kOk && rc3 != kUnsupported) return rc3;
@@ -967,12 +1016,28 @@ static int force_vjp(const Plan& p, const float* X, float* gF, float* gX,
     // the density cotangent goes to the unused fourth component of the
     // force mesh, so the finish kernel gathers one float4 per corner
     // nw.rho is free here: it takes the potential's cotangent
-    PMX_TRY(force_meshes_adj(p, gm, gm + M, gm + 2 * M, nw.w, nullptr, sc,
-                             s, f4, pgd, nw.rho));
     AdjUpdate uu = u;
     uu.gin_scale = gin ? 0.0f : gin_scale;
     const bool upd = u.mode == 1 || u.mode == 2;
     uu.implicit_gf = (gf_scale && !pgd && !gin && upd) ? 1 : 0;
+    if (phi) {
+      // with the potential at hand the force mesh is formed here and takes
+      // the density cotangent along: the transform stores it contiguously
+      // (28 us at 256^3 against 105 into every fourth float) and the
+      // gradient pass, which writes whole 16-byte cells anyway, reads it
+      // (112 us); the forward run then keeps potentials only, and its
+      // readout reads them (gradient + readout 73 + 331 us -> 416 with the
+      // copies of the state in it).  A finish pass on boxes of the potential
+      // and of the density cotangent instead took 720 us against 112 + 505.
+      PMX_TRY(force_meshes_adj(p, gm, gm + M, gm + 2 * M, nw.w, nw.rho, sc, s,
+                               nullptr, nullptr, nw.rho));
+      PMX_TRY(launch_grad_mesh(p, phi, f4, 4, s, nw.rho));
+    } else {
+      PMX_TRY(force_meshes_adj(p, gm, gm + M, gm + 2 * M, nw.w, nullptr, sc,
+                               s, f4, pgd, nw.rho));
+    }
+    uu.gxin = gsrc;
+    uu.gpin = gsrc ? gsrc + BN3 : nullptr;
     // the step-coefficient dot products ride along (they need the update)
     const bool fuse = cd && m.f4 && upd;
     PMX_TRY(launch_force_vjp_finish(gX, gP, gF, gc, X, m, nullptr, md, f,
@@ -984,6 +1049,7 @@ static int force_vjp(const Plan& p, const float* X, float* gF, float* gX,
     return kOk;
   }
   PMX_REQUIRE(!pgd, "PGD adjoint: particles must form the Lagrangian grid");
+  if (phi) PMX_TRY(launch_grad_mesh(p, phi, f4, 4, s));
   PMX_TRY(store_implicit_gf(gF, gP, gf_scale, BN3, s));
   for (int c = 0; c < 3; ++c) PMX_TRY(launch_fill(gms[c], M, 0.0f, s));
   PMX_TRY(launch_force_vjp_particles(gm, gm + M, gm + 2 * M, gX, gF, X, m,
@@ -1022,8 +1088,13 @@ static long long tape_floats(const Plan& p, long long N, int nsteps) {
   return (long long)(nsteps + 1) * (BN3 + 4 * M);
 }
 
+static Tape compact_tape_of(const Plan& p, float* tape, long long N,
+                            int nsteps);
+// A run that works on the potential itself lays its tape out like the
+// compact one, in the same allocation.
 static Tape tape_of(const Plan& p, float* tape, long long N, int nsteps,
-                    bool pgd = false) {
+                    float f, bool pgd = false) {
+  if (!pgd && box_run(p, N, f)) return compact_tape_of(p, tape, N, nsteps);
   const long long BN3 = 3LL * p.d.B * N;
   const long long M4 = 4 * p.d.rows * p.d.nz;
   Tape t;
@@ -1153,23 +1224,22 @@ static int reverse_steps(const Plan& p, const Tape& tp, int b0, int b1,
     particle_grid(p, N, f, &u.gx, &u.gy, &u.gz);
     const long long slot = i - tp.first;
     if (!pgd) {
-      // the step's float4 force mesh: taped, or (compact tape) from its
-      // potential into the force-mesh scratch
-      float* fm = tp.fs ? tp.fs + slot * 4 * M : nw.f4;
-      if (!tp.fs)
-        PMX_TRY(launch_grad_mesh(p, tp.phi_in + (long long)(1 + i) * M, fm,
-                                 4, s));
+      // the step's float4 force mesh, taped; or its potential, from which
+      // the VJP forms the mesh
+      float* fm = tp.fs ? tp.fs + slot * 4 * M : nullptr;
+      const float* phi =
+          fm ? nullptr : tp.phi_in + (long long)(1 + i - tp.phi0) * M;
       const float* xprev = i > b0 ? tp.xs + (slot - 1) * BN3 : cg.xb0;
       const CoefDot cd{xprev, coef_scratch(nw), cg.out, i, cg.nsteps + i};
       bool fused = false;
       PMX_TRY(force_vjp(p, tp.xs + slot * BN3, gF, gX, gP, N, f, fac, nw, gm,
                         fm, u, s, nullptr, nullptr, gsc,
-                        cg.out ? &cd : nullptr, &fused));
+                        cg.out ? &cd : nullptr, &fused, phi));
       if (cg.out && !fused)
         PMX_TRY(launch_coef_dot(
             tp.xs + slot * BN3, nullptr, xprev, gX, gP,
-            reinterpret_cast<const float4*>(fm), md, f, fac, u.d,
-            coef_scratch(nw), cg.out, i, cg.nsteps + i, s));
+            reinterpret_cast<const float4*>(fm ? fm : nw.f4), md, f, fac,
+            u.d, coef_scratch(nw), cg.out, i, cg.nsteps + i, s));
       continue;
     }
     PMX_TRY(store_implicit_gf(gF, gP, gsc, BN3, s));
@@ -1203,11 +1273,19 @@ static int reverse_steps(const Plan& p, const Tape& tp, int b0, int b1,
 }
 
 // First update of the reverse sweep: the closing kick of the last step.
+// gsrc (optional): the cotangent of the final state, read there.
 static int adjoint_open(const Plan& p, long long N, int nsteps,
-                        const double* coef, float* gstate, hipStream_t s) {
+                        const double* coef, float* gstate, hipStream_t s,
+                        const float* gsrc = nullptr) {
   if (nsteps <= 0) return kOk;
   const long long BN3 = (long long)p.d.B * N * 3;
   ProfScope prof_(kProfAdjUpdate, s);
+  if (gsrc) {
+    hipLaunchKernelGGL(k_adj_open, dim3(gridfor(BN3)), dim3(256), 0, s, gsrc,
+                       gstate, BN3, (float)coef[3 * (nsteps - 1) + 2]);
+    PMX_LAUNCH_CHECK();
+    return kOk;
+  }
   hipLaunchKernelGGL(k_adj_update, dim3(gridfor(BN3)), dim3(256), 0, s,
                      gstate, gstate + BN3, gstate + 2 * BN3, BN3, 0.f, 0.f,
                      (float)coef[3 * (nsteps - 1) + 2], 0);
@@ -1215,20 +1293,52 @@ static int adjoint_open(const Plan& p, long long N, int nsteps,
   return kOk;
 }
 
+// The end of a reverse sweep: the jump-start force at the initial positions X
+// (the initial F is discarded), from its float4 force mesh or its potential
+// phi, and the dot product of its coefficient.  gsrc: see force_vjp.
+static int jump_vjp(const Plan& p, const float* X, float* fm,
+                    const float* phi, float* gstate, int nsteps, long long N,
+                    float f, float fac, const NbodyWork& nw, float* gm,
+                    float* gsc, double* gcoef, hipStream_t s,
+                    const float* gsrc = nullptr) {
+  const long long BN3 = (long long)p.d.B * N * 3;
+  AdjUpdate u{0.f, 0.f, 0.f, 3, 0, 0, 0};
+  particle_grid(p, N, f, &u.gx, &u.gy, &u.gz);
+  PMX_TRY(force_vjp(p, X, gstate + 2 * BN3, gstate, gstate + BN3, N, f, fac,
+                    nw, gm, fm, u, s, nullptr, nullptr, gsc, nullptr, nullptr,
+                    phi, gsrc));
+  if (!gcoef || nsteps <= 0) return kOk;
+  if (!fm) fm = nw.f4;  // the VJP formed it there
+  return launch_coef_dot(X, nullptr, nullptr, gstate, gstate + BN3,
+                         reinterpret_cast<const float4*>(fm),
+                         MeshDims{p.d.B, p.d.nx, p.d.ny, p.d.nz, N}, f, fac,
+                         0.0f, coef_scratch(nw), gcoef, 2 * nsteps, -1, s);
+}
+
 // The recomputation tape of a checkpointed reverse sweep (inside its
 // workspace): X and the force meshes of the steps of one segment, and the
 // jump-start force.
 static Tape segment_tape(const Plan& p, long long N, int every, float* work,
-                         int b0) {
+                         int b0, float f, bool phi_kept) {
   const long long M = p.d.rows * p.d.nz;
   const long long BN3 = (long long)p.d.B * N * 3;
   float* gm = work + nbody_work_floats(p);
   float* st = gm + 3 * M;            // scratch state (3, B, N, 3)
   Tape tp;
   tp.xs = st + 3 * BN3;              // every * BN3
-  tp.fs = tp.xs + (long long)every * BN3;  // every * 4M
-  tp.fj = tp.fs + (long long)every * 4 * M;
   tp.first = b0;
+  float* const fs = tp.xs + (long long)every * BN3;  // every * 4M, then 4M
+  if (box_run(p, N, f)) {
+    // potentials instead of force meshes (the forward run's where kept):
+    // slots b0 (the jump start of the first segment) .. b0 + every
+    if (!phi_kept) {
+      tp.phi = fs;
+      tp.phi0 = b0;
+    }
+    return tp;
+  }
+  tp.fs = fs;
+  tp.fj = tp.fs + (long long)every * 4 * M;
   return tp;
 }
 
@@ -1254,8 +1364,8 @@ static int nbody_adjoint(const Plan& p, const float* ckpt, int every,
   PMX_TRY(adjoint_open(p, N, nsteps, coef, gstate, s));
   for (int sg = nseg - 1; sg >= 0; --sg) {
     const int b0 = sg * every, b1 = std::min(nsteps, b0 + every);
-    Tape tp = segment_tape(p, N, every, work, b0);
-    tp.phi_in = phi;
+    Tape tp = segment_tape(p, N, every, work, b0, f, phi != nullptr);
+    if (phi) tp.phi_in = phi;
     tp.x_from_tape = true;  // the sweep reads every position from the tape
     if (!(last_taped && sg == nseg - 1)) {
       const float* ck = ckpt + (long long)sg * 3 * BN3;
@@ -1270,6 +1380,10 @@ static int nbody_adjoint(const Plan& p, const float* ckpt, int every,
       PMX_TRY(nbody_run(p, st, N, f, fac, coef, b0, b1, sg == 0, work, s,
                         &tp, nullptr, b0 >= b1 ? nullptr : ck));
     }
+    if (!tp.fs && !tp.phi_in) {  // the segment's own potentials
+      tp.phi_in = tp.phi;
+      tp.phi = nullptr;
+    }
     CoefGrad cg;
     cg.out = gcoef;
     cg.nsteps = nsteps;
@@ -1277,65 +1391,50 @@ static int nbody_adjoint(const Plan& p, const float* ckpt, int every,
     PMX_TRY(reverse_steps(p, tp, b0, b1, N, f, fac, coef, gstate, nw, gm, s,
                           &gsc, nullptr, nullptr, cg));
   }
-  float* fjump = segment_tape(p, N, every, work, 0).fj;
   // jump-start force at the initial positions; the initial F is discarded
-  AdjUpdate u0{0.f, 0.f, 0.f, 3, 0, 0, 0};
-  particle_grid(p, N, f, &u0.gx, &u0.gy, &u0.gz);
-  PMX_TRY(force_vjp(p, ckpt, gstate + 2 * BN3, gstate, gstate + BN3, N, f,
-                    fac, nw, gm, nsteps > 0 ? fjump : nullptr, u0, s, nullptr,
-                    nullptr, &gsc));
-  if (gcoef && nsteps > 0)
-    PMX_TRY(launch_coef_dot(ckpt, nullptr, nullptr, gstate, gstate + BN3,
-                            reinterpret_cast<const float4*>(fjump),
-                            MeshDims{p.d.B, p.d.nx, p.d.ny, p.d.nz, N}, f,
-                            fac, 0.0f, coef_scratch(nw), gcoef, 2 * nsteps,
-                            -1, s));
-  return kOk;
+  const Tape t0 = segment_tape(p, N, every, work, 0, f, phi != nullptr);
+  const float* phij = nsteps <= 0 ? nullptr : phi ? phi : t0.phi;
+  float* fjump = nsteps > 0 ? t0.fj : nullptr;
+  return jump_vjp(p, ckpt, fjump, fjump ? nullptr : phij, gstate, nsteps, N,
+                  f, fac, nw, gm, &gsc, gcoef, s);
 }
 
 // Reverse sweep over a tape recorded by the forward run (no recomputation).
+// gsrc (optional): the cotangent of the final state, read there and left as
+// it is; gstate is then only written.
 static int nbody_adjoint_taped(const Plan& p, float* tape, int nsteps,
                                long long N, float f, float fac,
                                const double* coef, float* gstate,
                                float* work, hipStream_t s,
-                               double* gcoef = nullptr,
-                               bool compact = false) {
+                               double* gcoef = nullptr, bool compact = false,
+                               const float* gsrc = nullptr) {
   const long long BN3 = (long long)p.d.B * N * 3;
   NbodyWork nw = nbody_work(p, work);
   float* gm = work + nbody_work_floats(p);
   Tape tp = compact ? compact_tape_of(p, tape, N, nsteps)
-                    : tape_of(p, tape, N, nsteps);
-  if (compact) {
-    // the reverse sweep reads the potentials, and forms each force mesh
+                    : tape_of(p, tape, N, nsteps, f);
+  if (tp.phi) {
+    // the reverse sweep reads the potentials (and forms each force mesh)
     tp.phi_in = tp.phi;
     tp.phi = nullptr;
     PMX_REQUIRE(grad_stencil_ok(p),
                 "compact tape: nz must be a multiple of 4, sides >= 4");
   }
   float gsc = 0.0f;  // 0: gF stored; else the force cotangent is gsc * gP
-  PMX_TRY(adjoint_open(p, N, nsteps, coef, gstate, s));
+  if (gsrc && nsteps == 0 && !box_run(p, N, f)) {
+    PMX_HIP_CHECK(hipMemcpyAsync(gstate, gsrc, sizeof(float) * 3 * BN3,
+                                 hipMemcpyDeviceToDevice, s));
+    gsrc = nullptr;
+  }
+  PMX_TRY(adjoint_open(p, N, nsteps, coef, gstate, s, gsrc));
   CoefGrad cg;
   cg.out = gcoef;
   cg.nsteps = nsteps;
   cg.xb0 = tp.xj;
   PMX_TRY(reverse_steps(p, tp, 0, nsteps, N, f, fac, coef, gstate, nw, gm,
                         s, &gsc, nullptr, nullptr, cg));
-  AdjUpdate u0{0.f, 0.f, 0.f, 3, 0, 0, 0};
-  particle_grid(p, N, f, &u0.gx, &u0.gy, &u0.gz);
-  float* fj = tp.fj;
-  if (compact) {
-    fj = nw.f4;
-    PMX_TRY(launch_grad_mesh(p, tp.phi_in, fj, 4, s));
-  }
-  PMX_TRY(force_vjp(p, tp.xj, gstate + 2 * BN3, gstate, gstate + BN3, N, f,
-                    fac, nw, gm, fj, u0, s, nullptr, nullptr, &gsc));
-  if (gcoef && nsteps > 0)
-    PMX_TRY(launch_coef_dot(tp.xj, nullptr, nullptr, gstate, gstate + BN3,
-                            reinterpret_cast<const float4*>(fj),
-                            MeshDims{p.d.B, p.d.nx, p.d.ny, p.d.nz, N}, f,
-                            fac, 0.0f, coef_scratch(nw), gcoef, 2 * nsteps,
-                            -1, s));
-  return kOk;
+  return jump_vjp(p, tp.xj, tp.fj, tp.phi_in, gstate, nsteps, N, f, fac, nw,
+                  gm, &gsc, gcoef, s, nsteps == 0 ? gsrc : nullptr);
 }
 
 static int nbody_adjoint_pgd_taped(const Plan& p, float* tape, int nsteps,
@@ -1346,7 +1445,7 @@ static int nbody_adjoint_pgd_taped(const Plan& p, float* tape, int nsteps,
   const long long BN3 = (long long)p.d.B * N * 3;
   NbodyWork nw = nbody_work(p, work);
   float* gm = work + nbody_work_floats(p);
-  const Tape tp = tape_of(p, tape, N, nsteps, true);
+  const Tape tp = tape_of(p, tape, N, nsteps, f, true);
   if (gpgd && nsteps > 0) {
     hipLaunchKernelGGL(k_zero_dbl, dim3((3 * nsteps + 255) / 256), dim3(256),
                        0, s, gpgd, 3 * nsteps);
@@ -1360,17 +1459,8 @@ static int nbody_adjoint_pgd_taped(const Plan& p, float* tape, int nsteps,
   cg.xb0 = tp.xj;
   PMX_TRY(reverse_steps(p, tp, 0, nsteps, N, f, fac, coef, gstate, nw, gm, s,
                         &gsc, pgd, gpgd, cg));
-  AdjUpdate u0{0.f, 0.f, 0.f, 3, 0, 0, 0};
-  particle_grid(p, N, f, &u0.gx, &u0.gy, &u0.gz);
-  PMX_TRY(force_vjp(p, tp.xj, gstate + 2 * BN3, gstate, gstate + BN3, N, f,
-                    fac, nw, gm, tp.fj, u0, s));
-  if (gcoef && nsteps > 0)
-    PMX_TRY(launch_coef_dot(tp.xj, nullptr, nullptr, gstate, gstate + BN3,
-                            reinterpret_cast<const float4*>(tp.fj),
-                            MeshDims{p.d.B, p.d.nx, p.d.ny, p.d.nz, N}, f,
-                            fac, 0.0f, coef_scratch(nw), gcoef, 2 * nsteps,
-                            -1, s));
-  return kOk;
+  return jump_vjp(p, tp.xj, tp.fj, nullptr, gstate, nsteps, N, f, fac, nw, gm,
+                  nullptr, gcoef, s);
 }
 
 }  // namespace pmx
@@ -2081,6 +2171,37 @@ int pmx_nbody_run(const pmx_plan* plan, float* state, long long N, float f,
                    S(stream));
 }
 
+int pmx_nbody_run_from(const pmx_plan* plan, const float* src, float* state,
+                       long long N, float f, float fac, const double* coef,
+                       int nsteps, float* tape, int compact, float* work,
+                       void* stream) {
+  PMX_REQUIRE(plan && src && state && work && src != state,
+              "pmx_nbody_run_from: null pointer, or one state");
+  PMX_REQUIRE(N >= 1, "pmx_nbody_run_from: need at least one particle");
+  PMX_REQUIRE(nsteps >= 0 && (coef || nsteps == 0),
+              "pmx_nbody_run_from: bad steps");
+  const Plan& p = P(plan);
+  Tape tp;
+  if (tape)
+    tp = compact ? compact_tape_of(p, tape, N, nsteps)
+                 : tape_of(p, tape, N, nsteps, f);
+  return nbody_run(p, state, N, f, fac, coef, 0, nsteps, 1, work, S(stream),
+                   tape ? &tp : nullptr, nullptr, src);
+}
+
+int pmx_nbody_adjoint_from(const pmx_plan* plan, float* tape, int compact,
+                           int nsteps, long long N, float f, float fac,
+                           const double* coef, const float* gsrc,
+                           float* gstate, float* work, double* gcoef,
+                           void* stream) {
+  PMX_REQUIRE(plan && tape && gsrc && gstate && work && gsrc != gstate,
+              "pmx_nbody_adjoint_from: null pointer, or one state");
+  PMX_REQUIRE(N >= 1 && nsteps >= 0 && (coef || nsteps == 0),
+              "pmx_nbody_adjoint_from: bad steps");
+  return nbody_adjoint_taped(P(plan), tape, nsteps, N, f, fac, coef, gstate,
+                             work, S(stream), gcoef, compact != 0, gsrc);
+}
+
 int pmx_nbody_run_noalloc(const pmx_plan* plan, float* state, long long N,
                           float f, float fac, const double* coef, int b0,
                           int b1, int jump, void* stream) {
@@ -2164,7 +2285,7 @@ int pmx_nbody_run_taped(const pmx_plan* plan, float* state, long long N,
   PMX_REQUIRE(N >= 1, "pmx_nbody_run_taped: need at least one particle");
   PMX_REQUIRE(nsteps >= 0 && (coef || nsteps == 0),
               "pmx_nbody_run_taped: bad steps");
-  const Tape tp = tape_of(P(plan), tape, N, nsteps);
+  const Tape tp = tape_of(P(plan), tape, N, nsteps, f);
   return nbody_run(P(plan), state, N, f, fac, coef, 0, nsteps, 1, work,
                    S(stream), &tp);
 }
@@ -2222,7 +2343,7 @@ int pmx_nbody_run_pgd_taped(const pmx_plan* plan, float* state, long long N,
   for (int i = 0; i < nsteps; ++i)
     PMX_REQUIRE(pgd[3 * i + 1] != 0.0f && pgd[3 * i + 2] != 0.0f,
                 "pmx_nbody_run_pgd_taped: kl and ks must be nonzero");
-  const Tape tp = tape_of(P(plan), tape, N, nsteps, true);
+  const Tape tp = tape_of(P(plan), tape, N, nsteps, f, true);
   return nbody_run(P(plan), state, N, f, fac, coef, 0, nsteps, 1, work,
                    S(stream), &tp, pgd);
 }
@@ -2275,7 +2396,7 @@ int pmx_nbody_run_last_segment(const pmx_plan* plan, float* state,
               "every >= 1");
   const int nseg = (nsteps + every - 1) / every;
   const int b0 = (nseg - 1) * every;
-  const Tape tp = segment_tape(P(plan), N, every, work, b0);
+  const Tape tp = segment_tape(P(plan), N, every, work, b0, f, false);
   return nbody_run(P(plan), state, N, f, fac, coef, b0, nsteps, nseg == 1,
                    work, S(stream), &tp);
 }
@@ -2344,7 +2465,7 @@ int pmx_nbody_run_last_segment_phi(const pmx_plan* plan, float* state,
               "every >= 1");
   const int nseg = (nsteps + every - 1) / every;
   const int b0 = (nseg - 1) * every;
-  Tape tp = segment_tape(P(plan), N, every, work, b0);
+  Tape tp = segment_tape(P(plan), N, every, work, b0, f, true);
   tp.phi = phi;
   return nbody_run(P(plan), state, N, f, fac, coef, b0, nsteps, nseg == 1,
                    work, S(stream), &tp);

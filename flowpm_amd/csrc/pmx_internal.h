@@ -218,8 +218,9 @@ int launch_fill(float* p, long long n, float v, hipStream_t s);
 // first three packed (nc = 3), and the adjoint
 // out = -(D_x gx + D_y gy + D_z gz).  Needs nz % 4 == 0.
 bool grad_stencil_ok(const Plan& p);
+// (w4, with nc = 4: a mesh for the fourth component instead of 0)
 int launch_grad_mesh(const Plan& p, const float* phi, float* fm, int nc,
-                     hipStream_t s);
+                     hipStream_t s, const float* w4 = nullptr);
 int launch_grad_adj(const Plan& p, const float* gx, const float* gy,
                     const float* gz, float* out, hipStream_t s);
 int launch_paint(float* mesh, const float* pos, const float* w, float wscale,
@@ -257,6 +258,10 @@ struct KickDrift {
   // or xout and to P)
   const float* xin;
   const float* pin;
+  // readout_box only.  xkeep: the positions as read are also stored here.
+  // copy_xp (no kicks, xin / pin set): X and P as read are stored to X and P.
+  float* xkeep;
+  int copy_xp;
 };
 // The three force meshes: separate (x, y, z), interleaved float4 (f4) or
 // interleaved packed (x, y, z) floats (f3).
@@ -271,7 +276,7 @@ int launch_readout_kick_drift(float* X, float* P, float* F, const Mesh3& m,
                               const MeshDims& d, const KickDrift& c,
                               hipStream_t s);
 
-// The same from the potential (boxread.hip), for one particle per cell
+// The same from the potential (box_readout.h), for one particle per cell
 // (c.f == 1, the particle grid the mesh's own) and 16-byte aligned arrays.
 bool readout_box_ok(const MeshDims& d, const KickDrift& c, const float* X,
                     const float* P, const float* F, const float* phi);
@@ -349,6 +354,10 @@ struct AdjUpdate {
   // 1: the update does not store gF = (k1 [+ k2prev]) gP; the next force
   // VJP reads it as gin_scale * gP
   int implicit_gf;
+  // if set: gX and gP are read here instead of from the arrays that take the
+  // result (a gP that is not updated is then copied)
+  const float* gxin;
+  const float* gpin;
 };
 // Step-coefficient cotangents taken in the same pass: out[ia] += a and
 // out[ib] += b (see launch_coef_dot, with Xd = X), via part (2 doubles per

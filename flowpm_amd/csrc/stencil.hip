@@ -116,7 +116,7 @@ static __device__ __forceinline__ Nbr nbr_of(const Cell& c, const GridDims& g) {
   return n;
 }
 
-// NC = 4: fm[cell] = (D_x phi, D_y phi, D_z phi, 0) as one float4;
+// NC = 4: fm[cell] = (D_x phi, D_y phi, D_z phi, w4 or 0) as one float4;
 // NC = 3: (D_x phi, D_y phi, D_z phi) packed, 12 bytes per cell (the
 // forward step's mesh: a quarter fewer bytes written here and gathered by
 // the readout).  A thread's 4 cells are consecutive, so its own stores
@@ -126,11 +126,13 @@ static __device__ __forceinline__ Nbr nbr_of(const Cell& c, const GridDims& g) {
 template <int NC>
 __global__ __launch_bounds__(256) void k_grad_mesh(const float* __restrict__ phi,
                                                    float* __restrict__ fm,
+                                                   const float* __restrict__ w4,
                                                    GridDims g) {
   const Cell c = cell_of(g);
-  float4 gx = make_float4(0.f, 0.f, 0.f, 0.f), gy = gx, gz = gx;
+  float4 gx = make_float4(0.f, 0.f, 0.f, 0.f), gy = gx, gz = gx, gw = gx;
   if (c.ok) {
     const Nbr n = nbr_of(c, g);
+    if (NC == 4 && w4) gw = ld4(w4 + n.c + c.z0);
     const int z0 = c.z0;
     gz = dz_row(phi + n.c, z0, g.nz);
     gy = dvec(ld4(phi + n.ym2 + z0), ld4(phi + n.ym1 + z0),
@@ -141,10 +143,10 @@ __global__ __launch_bounds__(256) void k_grad_mesh(const float* __restrict__ phi
   __shared__ float4 st[256 * NC];
   const int t = threadIdx.x;
   if (NC == 4) {
-    st[4 * t] = make_float4(gx.x, gy.x, gz.x, 0.0f);
-    st[4 * t + 1] = make_float4(gx.y, gy.y, gz.y, 0.0f);
-    st[4 * t + 2] = make_float4(gx.z, gy.z, gz.z, 0.0f);
-    st[4 * t + 3] = make_float4(gx.w, gy.w, gz.w, 0.0f);
+    st[4 * t] = make_float4(gx.x, gy.x, gz.x, gw.x);
+    st[4 * t + 1] = make_float4(gx.y, gy.y, gz.y, gw.y);
+    st[4 * t + 2] = make_float4(gx.z, gy.z, gz.z, gw.z);
+    st[4 * t + 3] = make_float4(gx.w, gy.w, gz.w, gw.w);
   } else {
     // cells 0..3 of the thread: x0 y0 z0 x1 | y1 z1 x2 y2 | z2 x3 y3 z3
     st[3 * t] = make_float4(gx.x, gy.x, gz.x, gx.y);
@@ -219,7 +221,7 @@ bool grad_stencil_ok(const Plan& p) {
 }
 
 int launch_grad_mesh(const Plan& p, const float* phi, float* fm, int nc,
-                     hipStream_t s) {
+                     hipStream_t s, const float* w4) {
   PMX_REQUIRE(grad_stencil_ok(p),
               "gradient stencil: nz % 4 != 0, a side below 4 (nz below 8) "
               "or B * cells >= 2^33");
@@ -228,10 +230,10 @@ int launch_grad_mesh(const Plan& p, const float* phi, float* fm, int nc,
   ProfScope prof_(kProfGrad, s);
   if (nc == 4)
     hipLaunchKernelGGL(k_grad_mesh<4>, dim3(nblocks(g)), dim3(256), 0, s, phi,
-                       fm, g);
+                       fm, w4, g);
   else
     hipLaunchKernelGGL(k_grad_mesh<3>, dim3(nblocks(g)), dim3(256), 0, s, phi,
-                       fm, g);
+                       fm, nullptr, g);
   PMX_LAUNCH_CHECK();
   return kOk;
 }

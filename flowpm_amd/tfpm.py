@@ -48,8 +48,8 @@ def set_checkpoint_every(k):
   k >= 1: keep the state every k steps and recompute each segment in the
   backward pass; k = 0: record the positions and force meshes of every step
   in the forward pass (no recomputation; or the positions and potentials,
-  see set_compact_tape); None: automatic (k = 0 when the tape, full or
-  compact, fits in half of the free device memory, else k = 8)."""
+  see set_compact_tape); None: automatic (k = 0 when the tape fits in half
+  of the free device memory, else k = 8)."""
   if k is not None and int(k) < 0:
     raise ValueError("checkpoint interval must be >= 0 (or None)")
   _CKPT_EVERY[0] = None if k is None else int(k)
@@ -83,9 +83,10 @@ def set_compact_tape(compact):
   """Whether a taped differentiable nbody run (checkpoint interval 0) keeps
   the potential of every force evaluation instead of its float4 force mesh
   (about half the memory: at 256^3 x 40 steps 11 GB against 18.8 GB; the
-  backward pass forms each force mesh again with the gradient stencil, the
-  same gradients): True, False, or None (automatic: compact only when the
-  full tape does not fit in half of the free device memory)."""
+  backward pass forms each force mesh from it together with the density
+  cotangent; the same gradients): True, False, or None (automatic: True).
+  With one particle per cell (pm_nc_factor 1) either tape keeps potentials:
+  the forward pass reads the potential itself."""
   _COMPACT[0] = None if compact is None else bool(compact)
 
 
@@ -94,22 +95,17 @@ def _tape_fits(plan, N, nsteps, device, name):
   return need <= _TAPE_FRACTION * torch.cuda.mem_get_info(device)[0]
 
 
-def _compact(plan, N, nsteps, device):
-  if _COMPACT[0] is not None:
-    return _COMPACT[0]
-  return not _tape_fits(plan, N, nsteps, device, "pmx_nbody_tape_floats")
+def _compact():
+  return _COMPACT[0] is not False
 
 
 def _resolve_every(plan, N, nsteps, every, device):
-  """Checkpoint interval of the automatic policy: 0 (a tape: the full one,
-  or the compact one when only that fits in half of the free device
-  memory), else segments of 8 steps."""
+  """Checkpoint interval of the automatic policy: 0 (a tape, when it fits in
+  half of the free device memory), else segments of 8 steps."""
   if every is not None:
     return int(every)
-  if _tape_fits(plan, N, nsteps, device, "pmx_nbody_tape_floats"):
-    return 0
-  if _COMPACT[0] is not False and _tape_fits(
-      plan, N, nsteps, device, "pmx_nbody_compact_tape_floats"):
+  if _tape_fits(plan, N, nsteps, device, "pmx_nbody_%stape_floats" %
+                ("compact_" if _compact() else "")):
     return 0
   return _AUTO_SEGMENT
 
@@ -754,24 +750,52 @@ def _work(plan):
                      dtype=torch.float32, device=plan.device)
 
 
+def _tape(plan, N, nsteps, compact, device):
+  return torch.empty(
+      getattr(_lib.lib(), "pmx_nbody_%stape_floats" %
+              ("compact_" if compact else ""))(plan.handle, N, nsteps),
+      dtype=torch.float32, device=device)
+
+
+def _run_from(plan, x0, N, f, fac, cptr, nsteps, work, tape=None,
+              compact=False):
+  """The state after ``nsteps`` steps (and the jump-start force) from x0,
+  which is only read (pmx_nbody_run_from)."""
+  st = torch.empty_like(x0)
+  _lib.call("pmx_nbody_run_from", plan.handle, _lib.ptr(x0), _lib.ptr(st), N,
+            f, fac, cptr, nsteps, _lib.ptr(tape), 1 if compact else 0,
+            _lib.ptr(work), _lib.stream_of(st))
+  return st
+
+
+def _adjoint_from(plan, tape, compact, g, N, f, fac, cptr, nsteps, gcoef=None):
+  """The cotangent of the initial state from that of the final one, g, which
+  is only read (pmx_nbody_adjoint_from)."""
+  gs = torch.empty_like(g)
+  work = torch.empty(_lib.lib().pmx_nbody_adj_work_floats(plan.handle, N, 0),
+                     dtype=torch.float32, device=gs.device)
+  _lib.call("pmx_nbody_adjoint_from", plan.handle, _lib.ptr(tape),
+            1 if compact else 0, nsteps, N, f, fac, cptr, _lib.ptr(g),
+            _lib.ptr(gs), _lib.ptr(work), _lib.ptr(gcoef), _lib.stream_of(gs))
+  return gs
+
+
 class _Force(torch.autograd.Function):
   """F = force(X) (tfpm.py:317-366) as a taped run of zero steps: the
-  forward keeps X and the force mesh, the backward is the jump-start force
-  VJP of the nbody reverse sweep (gX += J^T gF, gF = 0).  The reverse
-  sweep rewrites only the fourth (density cotangent) component of the
-  taped force mesh, so the tape also serves a second backward pass
+  forward keeps X and the potential or force mesh, the backward is the
+  jump-start force VJP of the nbody reverse sweep (gX += J^T gF, gF = 0).
+  The reverse sweep leaves the tape's positions, potentials and forces as
+  they are, so the tape also serves a second backward pass
   (retain_graph=True); it is released with the graph otherwise."""
 
   @staticmethod
   def forward(ctx, state, plan, N, f, fac, fac_t=None):
-    st = _f32(state).clone()
-    tape = torch.empty(_lib.lib().pmx_nbody_tape_floats(plan.handle, N, 0),
-                       dtype=torch.float32, device=st.device)
-    _lib.call("pmx_nbody_run_taped", plan.handle, _lib.ptr(st), N, f, fac,
-              None, 0, _lib.ptr(tape), _lib.ptr(_work(plan)),
-              _lib.stream_of(st))
+    x0 = _f32(state)
+    compact = _compact()
+    tape = _tape(plan, N, 0, compact, x0.device)
+    st = _run_from(plan, x0, N, f, fac, None, 0, _work(plan), tape, compact)
     ctx.save_for_backward(tape)
-    ctx.args = (plan, N, f, fac)
+    ctx.args = (plan, N, f, fac, compact)
     # F = fac G(X): d L / d fac = gF . F / fac
     ctx.f_out = st[2].clone() if (len(ctx.needs_input_grad) > 5 and
                                   ctx.needs_input_grad[5]) else None
@@ -779,7 +803,7 @@ class _Force(torch.autograd.Function):
 
   @staticmethod
   def backward(ctx, g):
-    plan, N, f, fac = ctx.args
+    plan, N, f, fac, compact = ctx.args
     (tape,) = ctx.saved_tensors
     g = _f32(g)
     gfac = None
@@ -787,13 +811,7 @@ class _Force(torch.autograd.Function):
       gfac = torch.tensor(
           float((g[2].double() * ctx.f_out.double()).sum()) / fac,
           dtype=torch.float64)
-    gs = g.clone()
-    work = torch.empty(_lib.lib().pmx_nbody_adj_work_floats(plan.handle, N,
-                                                            0),
-                       dtype=torch.float32, device=gs.device)
-    _lib.call("pmx_nbody_adjoint_taped", plan.handle, _lib.ptr(tape), 0, N,
-              f, fac, None, _lib.ptr(gs), _lib.ptr(work), None,
-              _lib.stream_of(gs))
+    gs = _adjoint_from(plan, tape, compact, g, N, f, fac, None, 0)
     return (gs, None, None, None, None, gfac)[:len(ctx.needs_input_grad)]
 
 
@@ -807,10 +825,7 @@ def force(cosmo, state, nc, pm_nc_factor=1, dtype=torch.float32, name="Force",
   fac_t = _coef_tensor(cosmo, lambda c: 1.5 * c.Omega_m)
   if torch.is_grad_enabled() and (state.requires_grad or fac_t is not None):
     return _Force.apply(state, plan, N, f, fac, fac_t)
-  st = _f32(state).clone()
-  _lib.call("pmx_nbody_run", plan.handle, _lib.ptr(st), N, f, fac, None, 0, 0,
-            1, _lib.ptr(_work(plan)), _lib.stream_of(st))
-  return st
+  return _run_from(plan, _f32(state), N, f, fac, None, 0, _work(plan))
 
 
 def step_coefficients(cosmo, stages):
@@ -874,10 +889,7 @@ class _Nbody(torch.autograd.Function):
     cptr = _lib.dbl(coef)
     stream = _lib.stream_of(x0)
     if not need_grad:
-      st = x0.clone()
-      _lib.call("pmx_nbody_run", plan.handle, _lib.ptr(st), N, f, fac, cptr,
-                0, nsteps, 1, _lib.ptr(work), stream)
-      return st
+      return _run_from(plan, x0, N, f, fac, cptr, nsteps, work)
     ctx.want_c = len(ctx.needs_input_grad) > 8 and ctx.needs_input_grad[8]
     st = _Nbody._run_for_grad(ctx, x0, plan, N, f, fac, coef, every, work,
                               cptr, stream)
@@ -892,16 +904,12 @@ class _Nbody(torch.autograd.Function):
     B = plan.B
     nsteps = len(coef) // 3
     if every == 0:
-      st = x0.clone()
-      # the full tape (X and the float4 force mesh of every force), or the
-      # compact one (X and the potential)
-      ctx.compact = _compact(plan, N, nsteps, x0.device)
-      kind = "compact_" if ctx.compact else ""
-      tape = torch.empty(getattr(_lib.lib(), "pmx_nbody_%stape_floats" %
-                                 kind)(plan.handle, N, nsteps),
-                         dtype=torch.float32, device=x0.device)
-      _lib.call("pmx_nbody_run_%staped" % kind, plan.handle, _lib.ptr(st), N,
-                f, fac, cptr, nsteps, _lib.ptr(tape), _lib.ptr(work), stream)
+      # the compact tape (X and the potential of every force), or the full
+      # one (X and the float4 force mesh)
+      ctx.compact = _compact()
+      tape = _tape(plan, N, nsteps, ctx.compact, x0.device)
+      st = _run_from(plan, x0, N, f, fac, cptr, nsteps, work, tape,
+                     ctx.compact)
       # released with the graph; the reverse sweep rewrites only the fourth
       # (density cotangent) component of its force meshes, so a second
       # backward pass (retain_graph=True) reads an intact tape
@@ -965,25 +973,20 @@ class _Nbody(torch.autograd.Function):
     plan, N, f, fac, coef, every = ctx.args
     nsteps = len(coef) // 3
     g = _f32(g)
-    gs = g.clone()
     gcoef = gfin = None
     if ctx.want_c:
       gcoef = torch.zeros(2 * nsteps + 1, dtype=torch.float64,
-                          device=gs.device)
+                          device=g.device)
       # the final force's own cotangent
       gfin = float((g[2].double() * ctx.f_final.double()).sum())
     gptr = _lib.ptr(gcoef) if gcoef is not None else None
     if every == 0:
       (tape,) = ctx.saved_tensors
-      work = torch.empty(_lib.lib().pmx_nbody_adj_work_floats(plan.handle, N,
-                                                              0),
-                         dtype=torch.float32, device=gs.device)
-      kind = "compact_" if ctx.compact else ""
-      _lib.call("pmx_nbody_adjoint_%staped" % kind, plan.handle,
-                _lib.ptr(tape), nsteps, N, f, fac, _lib.dbl(coef),
-                _lib.ptr(gs), _lib.ptr(work), gptr, _lib.stream_of(gs))
+      gs = _adjoint_from(plan, tape, ctx.compact, g, N, f, fac,
+                         _lib.dbl(coef), nsteps, gcoef)
     else:
       ckpt, adj, phi = ctx.saved_tensors
+      gs = g.clone()
       k = min(every, max(nsteps, 1))
       if phi is not None:
         # the last segment's tape is used once; a second backward pass

@@ -325,6 +325,24 @@ int pmx_nbody_run(const pmx_plan* plan, float* state, long long N, float f,
                   float fac, const double* coef, int step_begin, int step_end,
                   int jump_start, float* work, void* stream);
 
+/* Steps [0, nsteps) with the jump-start force from the state src, which is
+ * left as it is; state (another buffer) is only written: no copy of the input
+ * is made.  tape (may be NULL): the run is taped, like pmx_nbody_run_taped, or
+ * with compact != 0 like pmx_nbody_run_compact_taped (below). */
+int pmx_nbody_run_from(const pmx_plan* plan, const float* src, float* state,
+                       long long N, float f, float fac, const double* coef,
+                       int nsteps, float* tape, int compact, float* work,
+                       void* stream);
+
+/* pmx_nbody_adjoint_taped (compact != 0: pmx_nbody_adjoint_compact_taped)
+ * from the cotangent gsrc of the final state, which is left as it is; gstate
+ * (another buffer) is only written. */
+int pmx_nbody_adjoint_from(const pmx_plan* plan, float* tape, int compact,
+                           int nsteps, long long N, float f, float fac,
+                           const double* coef, const float* gsrc,
+                           float* gstate, float* work, double* gcoef,
+                           void* stream);
+
 /* pmx_nbody_run without a workspace argument.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code
  * under HIP stream/graph capture, tight serving loops).  The workspace is a
