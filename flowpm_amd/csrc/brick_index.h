@@ -20,13 +20,24 @@ struct BrickGrid {
   int nbx, nby, nbz;  // bricks per dimension
   int nbricks;
   int f;              // mesh cells per particle spacing (pm_nc_factor)
+  unsigned my, mz;    // div_magic of nby and nbz
 };
 
-constexpr int kBoxFloats = 16384;  // largest brick box: its arena slot (64 KB)
+constexpr int kBoxFloats = 16384;  // the arena's floats per brick (64 KB)
 constexpr int kTile = 16;          // gather tile side
 
 PMX_HD int imin(int a, int b) { return a < b ? a : b; }
 PMX_HD int imax(int a, int b) { return a > b ? a : b; }
+
+// n / d by one high multiplication with m = div_magic(d) = ceil(2^32 / d), for
+// n d < 2^32 (a scalar division is some 30 instructions of the scalar unit the
+// whole CU shares)
+PMX_HD unsigned div_magic(unsigned d) {
+  return d > 1 ? 0xffffffffu / d + 1u : 0u;
+}
+PMX_HD unsigned div_by(unsigned n, unsigned m) {
+  return m ? (unsigned)(((unsigned long long)n * m) >> 32) : n;
+}
 
 PMX_HD int imod(int a, int n) {
   int r = a % n;
@@ -57,14 +68,18 @@ PMX_HD BrickGrid make_brick_grid(int gx, int gy, int gz, int f) {
   g.nby = (gy + g.ey - 1) / g.ey;
   g.nbz = (gz + g.ez - 1) / g.ez;
   g.nbricks = g.nbx * g.nby * g.nbz;
+  g.my = div_magic((unsigned)g.nby);
+  g.mz = div_magic((unsigned)g.nbz);
   return g;
 }
 
 // Particle block of brick bid: first particle (q0) and counts (cnt) per
 // axis.
 PMX_HD void brick_block(const BrickGrid& g, int bid, int q0[3], int cnt[3]) {
-  const int kz = bid % g.nbz, ky = (bid / g.nbz) % g.nby,
-            kx = bid / (g.nbz * g.nby);
+  // (at most 1024 bricks per axis and 2^22 in all: the products stay in range)
+  const int kxy = (int)div_by((unsigned)bid, g.mz),
+            kx = (int)div_by((unsigned)kxy, g.my);
+  const int kz = bid - kxy * g.nbz, ky = kxy - kx * g.nby;
   q0[0] = kx * g.ex;
   q0[1] = ky * g.ey;
   q0[2] = kz * g.ez;

@@ -10,13 +10,17 @@
 //   exceeds the 39.5 KB window) as 32-bit fixed point
 //   (integer LDS atomics run several times faster than float ones on
 //   gfx950, and integer sums do not depend on their order), and stores the
-//   dense box, converted back to float, to its own arena slot; the C
-//   channels are deposited one after the other through the same box.  The
-//   fixed-point scale is a power of two chosen per brick and channel from
+//   dense box, converted back to float, to a piece of the arena of its own.
+//   The fixed-point scale is a power of two chosen per brick and channel from
 //   the sum S of the channel's |weights| so no cell can overflow: the scale
 //   is 2^(30 - ex) with S = m 2^ex, m in [0.5, 1), so one deposit is rounded
 //   by at most half a unit, 2^(ex - 31) <= 2^-30 S.
-//   A brick whose box exceeds its 64 KB arena slot falls back to
+//   Every brick has a 56 KB piece of the arena per channel; a larger box, up
+//   to 128 KB, goes to a pool of 8 KB per brick (where a box lies does not
+//   change what is in it).  Without the pool (64 KB pieces) the late boxes
+//   beyond them spilled: at 256^3, a = 1, 100 us of float atomics per density
+//   paint and 231 per three-channel one.
+//   A brick whose box is larger still, or finds the pool full, falls back to
 //   device-scope float atomics into the finished mesh (k_brick_spill, after
 //   phase 2).
 // phase 2 (k_brick_gather): one workgroup per mesh tile (4, 8 or 16 x planes
@@ -30,6 +34,8 @@
 // memory transaction per deposit; here the mesh sees none in the common
 // case.  C = 1 is the density paint, C = 3 the weighted paint of the force
 // VJP (three mesh cotangents at once).
+#include <type_traits>
+
 #include "pmx_internal.h"
 
 namespace pmx {
@@ -37,13 +43,13 @@ namespace pmx {
 struct BrickArgs {
   float* mesh[3];        // C output meshes [B][nx][ny][nz] (overwritten)
   float* arena;          // box arena
-  long long slot;        // arena floats per brick
   int accum;             // gather adds to the mesh instead of overwriting
   int vec4;              // the gather may store the mesh 16 bytes at a time
   int* meta;             // 8 ints per brick: lo[3], ext[3], R (how far the
-                         // box reaches past the brick), overflow flag
-  int* ctr;              // [2] overflow count, [3] box radius (written by
-                         // k_brick_reduce between the two phases)
+                         // box reaches past the brick), where its box lies in
+                         // the arena (16-float units; kNoBox: it spills)
+  int* ctr;              // [kCtrPool] the pool's fill count, [kCtrR] the
+                         // largest R; zero before and after every paint
   const float* X;        // positions [B][N][3]
   const float* w;        // weights [B][N][wstride] or null
   int wstride;
@@ -53,15 +59,53 @@ struct BrickArgs {
   BrickGrid g;
 };
 
+constexpr int kNoBox = -1;
+// The arena: a piece of kSlot floats per brick and channel, and the rest of
+// kBoxFloats per brick and channel as a pool for the boxes beyond that, handed
+// out by a fill count.  (Every brick taking what it needs from the count would
+// pack the arena, but 8192 returning device-scope atomics on one line take
+// 400 us.)
+constexpr int kSlot = kBoxFloats - 2048;
+constexpr int kCtrPool = 0, kCtrR = 2, kCtrInts = 8;  // (the count: 64 bits)
+
+// Reductions along a wave by DPP moves (no LDS traffic): the result of the
+// first 8 << k lanes of a row ends up in the last of them; wave_* in lane 63.
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ int dpp_from(int old, int v) {
+  return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xf, false);
+}
+// (lanes without a source take the identity, so that each step is one
+// instruction with a DPP operand)
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ int dpp_min(int v) {
+  return min(v, dpp_from<CTRL, ROWS>(INT_MAX, v));
+}
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ int dpp_max(int v) {
+  return max(v, dpp_from<CTRL, ROWS>(INT_MIN, v));
+}
+__device__ __forceinline__ int min8(int v) {
+  return dpp_min<0x114>(dpp_min<0x112>(dpp_min<0x111>(v)));  // row_shr
+}
+__device__ __forceinline__ int max8(int v) {
+  return dpp_max<0x114>(dpp_max<0x112>(dpp_max<0x111>(v)));
+}
 __device__ __forceinline__ int wave_min(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
-  return v;
+  // then row_shr 8, row_bcast 15, row_bcast 31
+  return dpp_min<0x143, 0xc>(dpp_min<0x142, 0xa>(dpp_min<0x118>(min8(v))));
 }
 __device__ __forceinline__ int wave_max(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
-  return v;
+  return dpp_max<0x143, 0xc>(dpp_max<0x142, 0xa>(dpp_max<0x118>(max8(v))));
+}
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __int_as_float(dpp_from<CTRL, ROWS>(0, __float_as_int(v)));
+}
+__device__ __forceinline__ float sum8(float v) {
+  return dpp_add<0x114>(dpp_add<0x112>(dpp_add<0x111>(v)));
+}
+__device__ __forceinline__ float wave_sum(float v) {
+  return dpp_add<0x143, 0xc>(dpp_add<0x142, 0xa>(dpp_add<0x118>(sum8(v))));
 }
 
 __device__ __forceinline__ bool ok_pos(float x, float y, float z) {
@@ -70,312 +114,301 @@ __device__ __forceinline__ bool ok_pos(float x, float y, float z) {
 
 // deposit workgroup: 512 threads (8 waves; four workgroups per CU give 32
 // waves to hide the loads and the LDS atomics), 4 particles per thread;
-// bricks hold <= 2048 particles.  A box (<= kBoxFloats, its arena slot) is
-// accumulated through an LDS window of kWinFloats ints: four windows and
-// the workgroups' other LDS fit a CU's 160 KB; a larger box is deposited
-// in slabs of whole x planes, one pass over the particles per slab.
+// bricks hold <= 2048 particles.  A box is accumulated through an LDS window
+// of kWinFloats ints: four windows and the workgroups' other LDS fit a CU's
+// 160 KB; a larger box is deposited in slabs of whole x planes, one pass over
+// the particles per slab and channel.
 constexpr int kDT = 512;
 constexpr int kWinFloats = 10112;
 constexpr int kDW = kDT / 64;
 constexpr int kPPT = 2048 / kDT;
+// largest box: the arena holds kBoxFloats per brick and channel on average
+constexpr long long kBoxMax = 2 * kBoxFloats;
+static_assert(kDW == 8, "the workgroup reductions take 8 waves");
 
-// one brick's particles in registers, kPPT per thread (raw positions and
-// weights; lanes past the brick's end hold ok = false)
-template <int C>
-struct BrickRegs {
-  float px[kPPT], py[kPPT], pz[kPPT], wc[kPPT][C];
-  bool ok[kPPT];
-};
+// four consecutive floats of a box row, at any dword
+typedef float Vec4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// every load issued up front, branch-free: lanes past the brick's end load
-// its first particle and drop it; the weight test is one uniform branch
+// A deposit is bound by its VALU work, then the LDS atomics (8 per particle
+// and channel).  Particles a constant stride apart instead of two divisions
+// each, DPP instead of permute reductions, the box set up by every wave from
+// one LDS read instead of by one thread between two barriers, clearing and
+// storing 16 bytes at a time, and the three channels unrolled: density at
+// 256^3 105 -> 92 us, 16 x 64^3 28.4 -> 24.7, three channels at a = 1 in 256^3
+// 296 (a twelfth of the boxes not among them) -> 271, 128 x 160 x 96 31 -> 22.
+// (The three channels in one pass, so that the corner weights are formed once,
+// leave each a third of the window and take 381 us; the loop over them not
+// unrolled takes 360.)
 template <int C>
-__device__ __forceinline__ void load_brick(const BrickArgs& a, int bid, int b,
-                                           int tid, BrickRegs<C>& r) {
+// (launch bounds: at least 8 waves per SIMD, i.e. at most 64 VGPRs, so that
+// four 512-thread workgroups share a CU; their LDS windows fit its 160 KB)
+__global__ __launch_bounds__(kDT, 8) void k_brick_deposit(BrickArgs a) {
+  __shared__ __align__(16) int box[kWinFloats];  // fixed-point accumulators
+  __shared__ int red[6 * kDW];
+  __shared__ float redw[C * kDW];
+  __shared__ int sh_off;
   const BrickGrid& g = a.g;
+  // XCD-aware: each XCD deposits one contiguous run of bricks, so the
+  // cache lines that z-neighbouring bricks share are fetched into one L2
+  const int bid = xcd_block32(blockIdx.x, gridDim.x);
+  const int b = blockIdx.y;
+  const int tid = threadIdx.x, ln = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const float ps = a.ps;
   int q0[3], cnt[3];
   brick_block(g, bid, q0, cnt);
-  const int cy = cnt[1], cz = cnt[2];
-  const int nloc = cnt[0] * cy * cz;
-  const long long pb = (long long)b * a.d.N;
-  long long pidx[kPPT];
+  const int cy = cnt[1], cz = cnt[2], nloc = cnt[0] * cy * cz;
+  // the brick's first particle (uniform) and each particle's offset from it;
+  // in bricks of whole rounds of kDT particles a constant apart
+  const long long p0 = (long long)b * a.d.N +
+                       ((long long)q0[0] * g.gy + q0[1]) * g.gz + q0[2];
+  const bool even = nloc == kDT * kPPT && kDT % (cy * cz) == 0;
+  const unsigned pstep =
+      even ? (unsigned)(kDT / (cy * cz)) * g.gy * g.gz : 0u;
+  const float rz = 1.0f / (float)cz, ry = 1.0f / (float)cy;
+  auto part = [&](int t) {
+    // exact divisions: t < 2048, and (t + 1/2) / c is 1 / 2c off a whole
+    // number
+    const int q = (int)(((float)t + 0.5f) * rz), lz = t - q * cz,
+              lx = (int)(((float)q + 0.5f) * ry), ly = q - lx * cy;
+    return (unsigned)((lx * g.gy + ly) * g.gz + lz);
+  };
+  const float* const X0 = a.X + 3 * p0;
+  const float* const w0 = a.w ? a.w + p0 * a.wstride : nullptr;
+  // every load issued up front, branch-free: lanes past the brick's end load
+  // its first particle and drop it; the weight test is one uniform branch
+  float px[kPPT], py[kPPT], pz[kPPT], wc[kPPT][C];
+  unsigned q[kPPT];
+  bool ok[kPPT];
+  q[0] = part(tid < nloc ? tid : 0);
 #pragma unroll
   for (int u = 0; u < kPPT; ++u) {
     const int t = tid + u * kDT;
-    r.ok[u] = t < nloc;
-    const int tt = r.ok[u] ? t : 0;
-    const int lz = tt % cz, q = tt / cz, ly = q % cy, lx = q / cy;
-    pidx[u] = pb + ((long long)(q0[0] + lx) * g.gy + (q0[1] + ly)) * g.gz +
-              q0[2] + lz;
-    r.px[u] = a.X[3 * pidx[u]];
-    r.py[u] = a.X[3 * pidx[u] + 1];
-    r.pz[u] = a.X[3 * pidx[u] + 2];
+    ok[u] = t < nloc;
+    if (u > 0) q[u] = even ? q[u - 1] + pstep : part(ok[u] ? t : 0);
+    px[u] = X0[3 * q[u]];
+    py[u] = X0[3 * q[u] + 1];
+    pz[u] = X0[3 * q[u] + 2];
   }
   if (a.w) {
 #pragma unroll
     for (int u = 0; u < kPPT; ++u)
 #pragma unroll
-      for (int c = 0; c < C; ++c) r.wc[u][c] = a.w[pidx[u] * a.wstride + c];
+      for (int c = 0; c < C; ++c) wc[u][c] = w0[q[u] * a.wstride + c];
   }
-}
-
-template <int C>
-// (launch bounds: at least 8 waves per SIMD, i.e. at most 64 VGPRs, so that
-// four 512-thread workgroups share a CU; their LDS windows fit its 160 KB)
-__global__ __launch_bounds__(kDT, 8) void k_brick_deposit(BrickArgs a) {
-  __shared__ int box[kWinFloats];  // fixed-point accumulators
-  __shared__ int red[kDW][6];
-  __shared__ float redw[kDW][C];
-  __shared__ int sh[10];
-  __shared__ float shs[C][2];
-  const BrickGrid& g = a.g;
-  // XCD-aware: each XCD deposits one contiguous run of bricks, so the
-  // cache lines that z-neighbouring bricks share are fetched into one L2
-  const int bid = (int)xcd_block(blockIdx.x, gridDim.x);
-  const int b = blockIdx.y;
-  const int tid = threadIdx.x;
-  const float ps = a.ps;
-  BrickRegs<C> cur;
-  load_brick<C>(a, bid, b, tid, cur);
-  {
-    int q0[3], cnt[3];
-    brick_block(g, bid, q0, cnt);
-    // the brick's registers, modified in place
-    float(&px)[kPPT] = cur.px;
-    float(&py)[kPPT] = cur.py;
-    float(&pz)[kPPT] = cur.pz;
-    float(&wc)[kPPT][C] = cur.wc;
-    bool(&ok)[kPPT] = cur.ok;
+  // bounds and sums of |weight|
+  int mn[3] = {INT_MAX, INT_MAX, INT_MAX}, mx[3] = {INT_MIN, INT_MIN, INT_MIN};
+  float sw[C];
 #pragma unroll
-    for (int u = 0; u < kPPT; ++u) {
-      px[u] = ok[u] ? px[u] : 0.0f;
-      py[u] = ok[u] ? py[u] : 0.0f;
-      pz[u] = ok[u] ? pz[u] : 0.0f;
+  for (int c = 0; c < C; ++c) sw[c] = 0.0f;
 #pragma unroll
-      for (int c = 0; c < C; ++c)
-        wc[u][c] = ok[u] ? (a.w ? wc[u][c] * a.wscale : a.wscale) : 0.0f;
-    }
-    int mn[3] = {INT_MAX, INT_MAX, INT_MAX},
-        mx[3] = {INT_MIN, INT_MIN, INT_MIN};
-    float sw[C];  // per channel: sum over particles of |weight|
-#pragma unroll
-    for (int c = 0; c < C; ++c) sw[c] = 0.0f;
-#pragma unroll
-    for (int u = 0; u < kPPT; ++u) {
-      px[u] *= ps;
-      py[u] *= ps;
-      pz[u] *= ps;
-      ok[u] = ok[u] && ok_pos(px[u], py[u], pz[u]);
-      if (ok[u]) {
-        const int f[3] = {(int)floorf(px[u]), (int)floorf(py[u]),
-                          (int)floorf(pz[u])};
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          mn[d] = min(mn[d], f[d]);
-          mx[d] = max(mx[d], f[d]);
-        }
-#pragma unroll
-        for (int c = 0; c < C; ++c) sw[c] += fabsf(wc[u][c]);
-      }
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      mn[d] = wave_min(mn[d]);
-      mx[d] = wave_max(mx[d]);
-    }
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) sw[c] += __shfl_xor(sw[c], o);
-    const int wv = tid >> 6;
-    if ((tid & 63) == 0) {
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        red[wv][d] = mn[d];
-        red[wv][3 + d] = mx[d];
-      }
-#pragma unroll
-      for (int c = 0; c < C; ++c) redw[wv][c] = sw[c];
-    }
-    __syncthreads();
-    if (tid == 0) {
-      int lo[3], hi[3];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        lo[d] = red[0][d];
-        hi[d] = red[0][3 + d];
-        for (int w = 1; w < kDW; ++w) {
-          lo[d] = min(lo[d], red[w][d]);
-          hi[d] = max(hi[d], red[w][3 + d]);
-        }
-      }
-      const int n[3] = {a.d.nx, a.d.ny, a.d.nz};
-      const long long off = ((long long)b * g.nbricks + bid) * a.slot;
-      // fixed-point scale 2^e with (sum of |weights|) * 2^e < 2^30: no cell
-      // total (nor a partial sum) can leave the int32 range
-      bool wfin = true;
-      for (int c = 0; c < C; ++c) {
-        float swt = redw[0][c];
-        for (int w = 1; w < kDW; ++w) swt += redw[w][c];
-        int e = 0;
-        wfin = wfin && swt <= 3.0e38f;  // false for inf / nan weights
-        if (swt <= 3.0e38f && swt > 0.0f) {
-          int ex;
-          frexpf(swt, &ex);  // swt = m 2^ex, m in [0.5, 1)
-          e = min(max(30 - ex, -120), 120);
-        }
-        shs[c][0] = ldexpf(1.0f, e);
-        shs[c][1] = ldexpf(1.0f, -e);
-      }
-      // every brick owns a fixed arena slot: no shared allocator, and no
-      // shared counter either (k_brick_reduce takes the radius maximum)
-      const BrickBox bx = brick_box(lo, hi, n, q0, cnt, g.f, wfin, kBoxFloats);
-      const int mode = bx.mode;
-      const int* ext = bx.ext;
-      const long long vol = bx.vol;
-      int* m = a.meta + 8LL * ((long long)b * g.nbricks + bid);
-      m[0] = lo[0];
-      m[1] = lo[1];
-      m[2] = lo[2];
-      m[3] = ext[0];
-      m[4] = ext[1];
-      m[5] = ext[2];
-      m[6] = bx.R;
-      m[7] = mode == 2 ? 1 : 0;
-      sh[0] = mode;
-      sh[1] = lo[0];
-      sh[2] = lo[1];
-      sh[3] = lo[2];
-      sh[4] = ext[0];
-      sh[5] = ext[1];
-      sh[6] = ext[2];
-      sh[7] = (int)vol;
-      sh[8] = (int)(off & 0x7fffffff);
-      sh[9] = (int)(off >> 31);
-    }
-    __syncthreads();
-    const int mode = sh[0];
-    const int lo0 = sh[1], lo1 = sh[2], lo2 = sh[3];
-    const int e0 = sh[4], e1 = sh[5], e2 = sh[6], vol = sh[7];
-    const long long off = (long long)sh[8] | ((long long)sh[9] << 31);
-    // mode 0: no particles; mode 2: k_brick_spill adds it after the gather
-    if (mode != 1) return;
-    constexpr int OX[8] = {0, 1, 0, 0, 1, 1, 0, 1};
-    constexpr int OY[8] = {0, 0, 1, 0, 1, 0, 1, 1};
-    constexpr int OZ[8] = {0, 0, 0, 1, 0, 1, 1, 1};
-    // x planes of the box per LDS window: boxes larger than the window are
-    // deposited in several passes over x slabs
-    const int plane = e1 * e2;
-    const int hx = kWinFloats / plane;  // >= 1: plane <= vol / 2 <= 8192
-    const bool clip = hx < e0;
-    // clears the window and deposits channel c of the brick's particles
-    // whose corners fall in x planes [x0, x0 + nxw) of the box
-    auto deposit = [&](int c, float fxs, int x0, int nxw) {
-      const int wv = nxw * plane;
-      for (int i = tid; i < wv; i += kDT) box[i] = 0;
-      __syncthreads();
-      // the positions are opaque here, so the corner weights are computed
-      // per pass instead of being kept live across the passes and channels
-#pragma unroll
-      for (int u = 0; u < kPPT; ++u)
-        asm volatile("" : "+v"(px[u]), "+v"(py[u]), "+v"(pz[u]));
-#pragma unroll
-      for (int u = 0; u < kPPT; ++u) {
-        if (!ok[u]) continue;
-        const float x = px[u], y = py[u], z = pz[u];
-        const float flx = floorf(x), fly = floorf(y), flz = floorf(z);
-        const float w0x = 1.0f - fabsf(x - flx), w1x = 1.0f - fabsf(x - (flx + 1.0f));
-        const float w0y = 1.0f - fabsf(y - fly), w1y = 1.0f - fabsf(y - (fly + 1.0f));
-        const float w0z = 1.0f - fabsf(z - flz), w1z = 1.0f - fabsf(z - (flz + 1.0f));
-        const int bx = (int)flx - lo0 - x0, by = (int)fly - lo1, bz = (int)flz - lo2;
-        const float wq = wc[u][c] * fxs;
-        if (!clip) {  // the whole box in one window: no x test
-#pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            const float kw = ((OX[k] ? w1x : w0x) * (OY[k] ? w1y : w0y)) *
-                             (OZ[k] ? w1z : w0z);
-            const int li =
-                ((bx + OX[k]) * e1 + (by + OY[k])) * e2 + bz + OZ[k];
-            atomicAdd(&box[li], __float2int_rn(wq * kw));
-          }
-        } else {
-#pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            const int xx = bx + OX[k];
-            if ((unsigned)xx >= (unsigned)nxw) continue;
-            const float kw = ((OX[k] ? w1x : w0x) * (OY[k] ? w1y : w0y)) *
-                             (OZ[k] ? w1z : w0z);
-            const int li = (xx * e1 + (by + OY[k])) * e2 + bz + OZ[k];
-            atomicAdd(&box[li], __float2int_rn(wq * kw));
-          }
-        }
-      }
-      __syncthreads();
-    };
+  for (int u = 0; u < kPPT; ++u) {
+    px[u] *= ps;
+    py[u] *= ps;
+    pz[u] *= ps;
+    ok[u] = ok[u] && ok_pos(px[u], py[u], pz[u]);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-      const float fxinv = shs[c][1];
-      for (int x0 = 0; x0 < e0; x0 += hx) {
-        const int nxw = min(hx, e0 - x0);
-        deposit(c, shs[c][0], x0, nxw);
-        float* dst = a.arena + off + (long long)c * vol + (long long)x0 * plane;
-        const int wv = nxw * plane;
-        for (int i = tid; i < wv; i += kDT) dst[i] = (float)box[i] * fxinv;
-        if (c + 1 < C || x0 + hx < e0) __syncthreads();  // window reused
+      wc[u][c] = ok[u] ? (a.w ? wc[u][c] * a.wscale : a.wscale) : 0.0f;
+      sw[c] += fabsf(wc[u][c]);
+    }
+    if (ok[u]) {
+      const float p[3] = {px[u], py[u], pz[u]};
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const int f = (int)floorf(p[d]);
+        mn[d] = min(mn[d], f);
+        mx[d] = max(mx[d], f);
+      }
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const int l = wave_min(mn[d]), h = wave_max(mx[d]);
+    if (ln == 63) {
+      red[d * kDW + wv] = l;
+      red[(3 + d) * kDW + wv] = h;
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const float m = wave_sum(sw[c]);
+    if (ln == 63) redw[c * kDW + wv] = m;
+  }
+  __syncthreads();
+  // every wave finishes the reductions: 8 lanes per bound, 8 per channel
+  const int rv = red[ln < 6 * kDW ? ln : 0];
+  const int rmin = min8(rv), rmax = max8(rv);
+  const float rw = sum8(redw[ln < C * kDW ? ln : 0]);
+  int lo[3], hi[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    lo[d] = __builtin_amdgcn_readlane(rmin, 8 * d + 7);
+    hi[d] = __builtin_amdgcn_readlane(rmax, 8 * d + 31);
+  }
+  // fixed-point scale 2^e with (sum of |weights|) * 2^e < 2^30: no cell
+  // total (nor a partial sum) can leave the int32 range
+  float fxs[C], fxinv[C];
+  bool wfin = true;
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const float swt = __int_as_float(
+        __builtin_amdgcn_readlane(__float_as_int(rw), 8 * c + 7));
+    int e = 0;
+    wfin = wfin && swt <= 3.0e38f;  // false for inf / nan weights
+    if (swt <= 3.0e38f && swt > 0.0f) {
+      int ex;
+      frexpf(swt, &ex);  // swt = m 2^ex, m in [0.5, 1)
+      e = min(max(30 - ex, -120), 120);
+    }
+    // 2^e and 2^-e (|e| <= 120), uniform
+    const int es = __builtin_amdgcn_readfirstlane(e);
+    fxs[c] = __int_as_float((127 + es) << 23);
+    fxinv[c] = __int_as_float((127 - es) << 23);
+  }
+  const int n[3] = {a.d.nx, a.d.ny, a.d.nz};
+  BrickBox bx = brick_box(lo, hi, n, q0, cnt, g.f, wfin, kBoxMax);
+  // (the window has to hold a plane of the deposits' two)
+  if (bx.mode == 1 && 2LL * bx.ext[1] * bx.ext[2] > kWinFloats) bx.mode = 2;
+  int* const m = a.meta + 8LL * ((long long)b * g.nbricks + bid);
+  const bool box_ok = bx.mode == 1;
+  const int e0 = bx.ext[0], e1 = bx.ext[1], e2 = bx.ext[2];
+  const int vol4 = (int)((bx.vol + 3) & ~3LL);  // channel stride in the arena
+  // where the box goes, in 16-float units; a piece of the pool is asked for
+  // by thread 0, and its answer used after the first pass
+  const long long nb = (long long)gridDim.x * gridDim.y;
+  constexpr int kPiece = C * kSlot / 16, kPool = C * kBoxFloats / 16 - kPiece;
+  const bool pooled = vol4 > kSlot;
+  const int units = (C * vol4 + 15) / 16;
+  unsigned long long got = 0;
+  if (tid == 0 && box_ok && pooled)
+    got = atomicAdd(reinterpret_cast<unsigned long long*>(a.ctr + kCtrPool),
+                    (unsigned long long)units);
+  if (!box_ok) {
+    if (tid == 0) {
+      m[3] = m[4] = m[5] = m[6] = 0;
+      m[7] = bx.mode == 2 ? kNoBox : 0;
+    }
+    return;
+  }
+  constexpr int OX[8] = {0, 1, 0, 0, 1, 1, 0, 1};
+  constexpr int OY[8] = {0, 0, 1, 0, 1, 0, 1, 1};
+  constexpr int OZ[8] = {0, 0, 0, 1, 0, 1, 1, 1};
+  const int plane = e1 * e2, hx = kWinFloats / plane;  // planes per pass
+  const bool clip = hx < e0;
+  float* dst = nullptr;
+  // deposits channel c of the particles; with CLIP those whose corners fall
+  // in x planes [x0, x0 + nxw) of the box, else all
+  auto deposit = [&](auto clip_, int c, int x0, int nxw) {
+    constexpr bool CLIP = decltype(clip_)::value;
+    // the positions are opaque here, so the corner weights are computed
+    // per pass instead of being kept live across the passes and channels
+#pragma unroll
+    for (int u = 0; u < kPPT; ++u)
+      asm volatile("" : "+v"(px[u]), "+v"(py[u]), "+v"(pz[u]));
+#pragma unroll
+    for (int u = 0; u < kPPT; ++u) {
+      const float x = px[u], y = py[u], z = pz[u];
+      const float flx = floorf(x), fly = floorf(y), flz = floorf(z);
+      const int ix = (int)flx - lo[0] - x0;
+      if (!ok[u] || (CLIP && !(ix >= -1 && ix < nxw))) continue;
+      const float w0x = 1.0f - fabsf(x - flx), w1x = 1.0f - fabsf(x - (flx + 1.0f));
+      const float w0y = 1.0f - fabsf(y - fly), w1y = 1.0f - fabsf(y - (fly + 1.0f));
+      const float w0z = 1.0f - fabsf(z - flz), w1z = 1.0f - fabsf(z - (flz + 1.0f));
+      const int at = (ix * e1 + ((int)fly - lo[1])) * e2 + ((int)flz - lo[2]);
+      const float wq = wc[u][c] * fxs[c];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        if (CLIP && (unsigned)(ix + OX[k]) >= (unsigned)nxw) continue;
+        const float kw = ((OX[k] ? w1x : w0x) * (OY[k] ? w1y : w0y)) *
+                         (OZ[k] ? w1z : w0z);
+        atomicAdd(box + at + ((OX[k] * e1 + OY[k]) * e2 + OZ[k]),
+                  __float2int_rn(wq * kw));
+      }
+    }
+  };
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    for (int x0 = 0; x0 < e0; x0 += hx) {
+      const int nxw = min(hx, e0 - x0), nw = nxw * plane;
+      const bool first_pass = c == 0 && x0 == 0;
+      if (!first_pass) __syncthreads();  // the window is reused
+      for (int i = tid; 4 * i < nw; i += kDT)
+        reinterpret_cast<int4*>(box)[i] = make_int4(0, 0, 0, 0);
+      __syncthreads();
+      if (clip)
+        deposit(std::true_type{}, c, x0, nxw);
+      else
+        deposit(std::false_type{}, c, 0, nxw);
+      if (first_pass && tid == 0) {
+        const bool fits = !pooled || (long long)got + units <= nb * kPool;
+        const long long at =
+            pooled ? nb * kPiece + (long long)got
+                   : ((long long)b * g.nbricks + bid) * kPiece;
+        const int off = fits ? (int)(unsigned)at : kNoBox;
+        sh_off = off;
+        m[0] = lo[0];
+        m[1] = lo[1];
+        m[2] = lo[2];
+        m[3] = fits ? e0 : 0;
+        m[4] = fits ? e1 : 0;
+        m[5] = fits ? e2 : 0;
+        m[6] = fits ? bx.R : 0;
+        m[7] = off;
+      }
+      __syncthreads();
+      if (first_pass) {
+        const int off = sh_off;
+        if (off == kNoBox) return;
+        dst = a.arena + 16LL * (unsigned)off;
+      }
+      const float fi = fxinv[c];
+      float* const o = dst + c * vol4 + x0 * plane;
+      for (int i = tid; 4 * i < nw; i += kDT) {
+        const int4 v = reinterpret_cast<const int4*>(box)[i];
+        const Vec4u r = {(float)v.x * fi, (float)v.y * fi, (float)v.z * fi,
+                         (float)v.w * fi};
+        if (4 * i + 4 <= nw) {
+          *reinterpret_cast<Vec4u*>(o + 4 * i) = r;
+        } else {
+          o[4 * i] = r.x;
+          if (4 * i + 1 < nw) o[4 * i + 1] = r.y;
+          if (4 * i + 2 < nw) o[4 * i + 2] = r.z;
+        }
       }
     }
   }
 }
 
-// Radius maximum and overflow count over all bricks (one workgroup), read by
-// the gather: ctr[2] = bricks that went to device atomics, ctr[3] = max R.
-__global__ __launch_bounds__(1024) void k_brick_reduce(const int* __restrict__ meta,
-                                                       long long nb,
-                                                       int* __restrict__ ctr) {
-  __shared__ int smax[16], ssum[16];
-  int r = 0, o = 0;
-  // (R, overflow) of 8 bricks per thread and round, all loads issued before
-  // the first is used (indices past the end reload the last brick and are
-  // dropped)
+// The largest R of the paint, read by the gather (one workgroup).
+__global__ __launch_bounds__(1024) void k_brick_reduce(
+    const int* __restrict__ meta, long long nb, int* __restrict__ ctr) {
+  __shared__ int smax[16];
+  int r = 0;
+  // 8 bricks per thread and round, all loads issued before the first is used
+  // (indices past the end reload the last brick)
   constexpr int U = 8;
   for (long long i0 = threadIdx.x; i0 < nb; i0 += 1024LL * U) {
-    int vr[U], vo[U];
+    int v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const long long i = min(i0 + 1024LL * u, nb - 1);
-      vr[u] = meta[8 * i + 6];
-      vo[u] = meta[8 * i + 7];
-    }
+    for (int u = 0; u < U; ++u) v[u] = meta[8 * min(i0 + 1024LL * u, nb - 1) + 6];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bool in = i0 + 1024LL * u < nb;
-      r = max(r, in ? vr[u] : 0);
-      o += in ? vo[u] : 0;
-    }
+    for (int u = 0; u < U; ++u) r = max(r, v[u]);
   }
 #pragma unroll
-  for (int k = 32; k > 0; k >>= 1) {
-    r = max(r, __shfl_xor(r, k));
-    o += __shfl_xor(o, k);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    smax[threadIdx.x >> 6] = r;
-    ssum[threadIdx.x >> 6] = o;
-  }
+  for (int k = 32; k > 0; k >>= 1) r = max(r, __shfl_xor(r, k));
+  if ((threadIdx.x & 63) == 0) smax[threadIdx.x >> 6] = r;
   __syncthreads();
   if (threadIdx.x == 0) {
-    int rr = 0, oo = 0;
-    for (int w = 0; w < 16; ++w) {
-      rr = max(rr, smax[w]);
-      oo += ssum[w];
-    }
-    ctr[2] = oo;
-    ctr[3] = rr;
+    for (int w = 1; w < 16; ++w) r = max(r, smax[w]);
+    ctr[kCtrR] = max(r, smax[0]);
   }
 }
 
-// four consecutive floats of a box row, at any dword
-typedef float Vec4u __attribute__((ext_vector_type(4), aligned(4)));
+// the counters of a workspace that no paint has used
+__global__ void k_brick_init(int* __restrict__ ctr) {
+  if (threadIdx.x < kCtrInts) ctr[threadIdx.x] = 0;
+}
 
 // One workgroup of 4 waves per mesh tile of 4 PX x 16 x 16 cells: wave w owns
 // the x planes w PX .. w PX + PX - 1, a lane 4 consecutive z cells of one y
@@ -409,7 +442,7 @@ __global__ __launch_bounds__(256) void k_brick_gather(BrickArgs a) {
   const int t0x = tx * TX, t0y = ty * kTile, t0z = tz * kTile;
   const int Tx = min(TX, d.nx - t0x), Ty = min(kTile, d.ny - t0y),
             Tz = min(kTile, d.nz - t0z);
-  const int R = a.ctr[3];
+  const int R = a.ctr[kCtrR];
   // candidate bricks per dimension (wave w builds list w)
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), ln = tid & 63;
   if (wv < 3) {
@@ -465,7 +498,7 @@ __global__ __launch_bounds__(256) void k_brick_gather(BrickArgs a) {
         ok = box_meets(a0, e0, t0x, Tx, d.nx) &&
              box_meets(a1, e1, t0y, Ty, d.ny) &&
              box_meets(a2, e2, t0z, Tz, d.nz);
-        rec[0] = bid;
+        rec[0] = mb.w;
         rec[1] = a0;
         rec[2] = a1;
         rec[3] = a2;
@@ -512,9 +545,8 @@ __global__ __launch_bounds__(256) void k_brick_gather(BrickArgs a) {
           };
           const int a0 = rd(1), a1 = rd(2), a2 = rd(3), e0 = rd(4), e1 = rd(5),
                     e2 = rd(6);
-          const int vol = e0 * e1 * e2, pl = e1 * e2;
-          const float* src =
-              a.arena + ((long long)b * g.nbricks + rd(0)) * a.slot;
+          const int vol = (e0 * e1 * e2 + 3) & ~3, pl = e1 * e2;
+          const float* src = a.arena + 16LL * (unsigned)rd(0);
           const int oy = wrap_off(cy, a1, d.ny);
           const bool yin = any && yz_ok && oy < e1;
           const int o = cz - a2;
@@ -610,75 +642,91 @@ __global__ __launch_bounds__(256) void k_brick_gather(BrickArgs a) {
   }
 }
 
-// Bricks whose box did not fit (box over its 64 KB arena slot, positions spread
-// over more than the mesh, non-finite weights) are added to the gathered
-// mesh with device-scope float atomics, one thread per particle.  Without
-// such bricks (k_brick_reduce counted none) every workgroup returns after
-// one load.
 template <int C>
-__global__ __launch_bounds__(256) void k_brick_spill(BrickArgs a) {
-  if (a.ctr[2] == 0) return;
+__device__ __forceinline__ void spill_brick(const BrickArgs& a, long long q) {
   const BrickGrid& g = a.g;
   const MeshDims& d = a.d;
-  const long long nq = (long long)d.B * g.nbricks;
-  for (long long q = blockIdx.x; q < nq; q += gridDim.x) {
-    if (a.meta[8 * q + 7] == 0) continue;
-    const int b = (int)(q / g.nbricks), bid = (int)(q % g.nbricks);
-    int q0[3], cnt[3];
-    brick_block(g, bid, q0, cnt);
-    const int cy = cnt[1], cz = cnt[2];
-    const int nloc = cnt[0] * cy * cz;
-    for (int t = threadIdx.x; t < nloc; t += blockDim.x) {
-      const int lz = t % cz, r = t / cz, ly = r % cy, lx = r / cy;
-      const long long pi = (long long)b * d.N +
-                           ((long long)(q0[0] + lx) * g.gy + (q0[1] + ly)) *
-                               g.gz +
-                           q0[2] + lz;
-      const float x = a.X[3 * pi] * a.ps, y = a.X[3 * pi + 1] * a.ps,
-                  z = a.X[3 * pi + 2] * a.ps;
-      if (!ok_pos(x, y, z)) continue;
-      float wc[C];
+  const int b = (int)(q / g.nbricks), bid = (int)(q % g.nbricks);
+  int q0[3], cnt[3];
+  brick_block(g, bid, q0, cnt);
+  const int cy = cnt[1], cz = cnt[2];
+  const int nloc = cnt[0] * cy * cz;
+  for (int t = threadIdx.x; t < nloc; t += blockDim.x) {
+    const int lz = t % cz, r = t / cz, ly = r % cy, lx = r / cy;
+    const long long pi =
+        (long long)b * d.N +
+        ((long long)(q0[0] + lx) * g.gy + (q0[1] + ly)) * g.gz + q0[2] + lz;
+    const float x = a.X[3 * pi] * a.ps, y = a.X[3 * pi + 1] * a.ps,
+                z = a.X[3 * pi + 2] * a.ps;
+    if (!ok_pos(x, y, z)) continue;
+    float wc[C];
 #pragma unroll
-      for (int c = 0; c < C; ++c)
-        wc[c] = a.w ? a.w[pi * a.wstride + c] * a.wscale : a.wscale;
-      const float flx = floorf(x), fly = floorf(y), flz = floorf(z);
-      const float wx[2] = {1.0f - fabsf(x - flx), 1.0f - fabsf(x - (flx + 1.0f))};
-      const float wy[2] = {1.0f - fabsf(y - fly), 1.0f - fabsf(y - (fly + 1.0f))};
-      const float wz[2] = {1.0f - fabsf(z - flz), 1.0f - fabsf(z - (flz + 1.0f))};
-      const int ix = (int)flx, iy = (int)fly, iz = (int)flz;
+    for (int c = 0; c < C; ++c)
+      wc[c] = a.w ? a.w[pi * a.wstride + c] * a.wscale : a.wscale;
+    const float flx = floorf(x), fly = floorf(y), flz = floorf(z);
+    const float wx[2] = {1.0f - fabsf(x - flx), 1.0f - fabsf(x - (flx + 1.0f))};
+    const float wy[2] = {1.0f - fabsf(y - fly), 1.0f - fabsf(y - (fly + 1.0f))};
+    const float wz[2] = {1.0f - fabsf(z - flz), 1.0f - fabsf(z - (flz + 1.0f))};
+    const int ix = (int)flx, iy = (int)fly, iz = (int)flz;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int ox = k & 1, oy = (k >> 1) & 1, oz = k >> 2;
-        const float kw = (wx[ox] * wy[oy]) * wz[oz];
-        const long long cell =
-            (((long long)b * d.nx + imod(ix + ox, d.nx)) * d.ny +
-             imod(iy + oy, d.ny)) * d.nz + imod(iz + oz, d.nz);
+    for (int k = 0; k < 8; ++k) {
+      const int ox = k & 1, oy = (k >> 1) & 1, oz = k >> 2;
+      const float kw = (wx[ox] * wy[oy]) * wz[oz];
+      const long long cell =
+          (((long long)b * d.nx + imod(ix + ox, d.nx)) * d.ny +
+           imod(iy + oy, d.ny)) * d.nz + imod(iz + oz, d.nz);
 #pragma unroll
-        for (int c = 0; c < C; ++c) atomicAdd(a.mesh[c] + cell, wc[c] * kw);
-      }
+      for (int c = 0; c < C; ++c) atomicAdd(a.mesh[c] + cell, wc[c] * kw);
+    }
+  }
+}
+
+// Bricks whose box did not fit (too large, or the arena was full; positions
+// spread over more than the mesh; non-finite weights) are added to the
+// gathered mesh with device-scope float atomics, one thread per particle.
+// Every workgroup looks through the flags of its own bricks at once; without
+// a marked one it returns after that load.  The counters are left zero.
+template <int C>
+__global__ __launch_bounds__(256) void k_brick_spill(BrickArgs a) {
+  if (blockIdx.x == 0 && threadIdx.x < kCtrInts) a.ctr[threadIdx.x] = 0;
+  const long long nq = (long long)a.d.B * a.g.nbricks;
+  for (long long k0 = blockIdx.x; k0 < nq; k0 += 256LL * gridDim.x) {
+    const long long mine = k0 + (long long)threadIdx.x * gridDim.x;
+    const bool hit = mine < nq && a.meta[8 * mine + 7] == kNoBox;
+    if (!__syncthreads_or(hit)) continue;
+    for (int w = 0; w < 256; ++w) {
+      const long long q = k0 + (long long)w * gridDim.x;
+      if (q >= nq) break;
+      if (a.meta[8 * q + 7] == kNoBox) spill_brick<C>(a, q);
     }
   }
 }
 
 bool brick_paint_ok(const MeshDims& d, const BrickGrid& g) {
+  // (the limits on the bricks: brick_block's divisions, the candidate lists)
   return g.ex * g.ey * g.ez <= kDT * kPPT && g.gx * g.f == d.nx &&
+         (long long)g.nbx * g.nby * g.nbz < (1LL << 22) &&
          g.gy * g.f == d.ny && g.gz * g.f == d.nz &&
          (long long)g.gx * g.gy * g.gz == d.N && g.nbx <= 1024 &&
          g.nby <= 1024 && g.nbz <= 1024;
 }
 
 long long brick_work_floats(const MeshDims& d, const BrickGrid& g, int C) {
-  // one arena slot of C boxes per brick
+  // kBoxFloats per brick and channel; counters and alignment take the rest
   const long long arena = (long long)d.B * g.nbricks * C * kBoxFloats;
   const long long meta = 8LL * d.B * g.nbricks;
   return arena + meta + 16;
 }
 
-// 16-byte aligned, with at least 3 floats in front: the gather's 16-byte
-// loads may start 3 floats before a box (those values are dropped)
+// The counters come first, at a place that does not depend on C, and the
+// arena is 16-byte aligned with at least 3 floats in front: the gather's
+// 16-byte loads may start 3 floats before a box (those values are dropped).
+static int* brick_ctr(float* work) {
+  return reinterpret_cast<int*>(
+      (reinterpret_cast<uintptr_t>(work) + 15) & ~uintptr_t(15));
+}
 static float* brick_arena(float* work) {
-  return reinterpret_cast<float*>(
-      (reinterpret_cast<uintptr_t>(work + 3) + 15) & ~uintptr_t(15));
+  return reinterpret_cast<float*>(brick_ctr(work) + kCtrInts);
 }
 const int* brick_meta(const MeshDims& d, const BrickGrid& g, int C,
                       float* work) {
@@ -689,15 +737,19 @@ const int* brick_meta(const MeshDims& d, const BrickGrid& g, int C,
 int launch_brick_paint(float* const* mesh, int C, const float* X,
                        const float* w, int wstride, float wscale, float ps,
                        const MeshDims& d, const BrickGrid& g, float* work,
-                       hipStream_t s, bool accumulate) {
+                       hipStream_t s, bool accumulate, bool* ready) {
   if ((long long)d.B * d.N == 0) return kOk;
   BrickArgs a{};
   a.accum = accumulate ? 1 : 0;
   for (int c = 0; c < C; ++c) a.mesh[c] = mesh[c];
-  a.slot = (long long)C * kBoxFloats;
   a.arena = brick_arena(work);
   a.meta = const_cast<int*>(brick_meta(d, g, C, work));
-  a.ctr = a.meta + 8LL * d.B * g.nbricks;
+  a.ctr = brick_ctr(work);
+  if (!ready || !*ready) {
+    hipLaunchKernelGGL(k_brick_init, dim3(1), dim3(64), 0, s, a.ctr);
+    PMX_LAUNCH_CHECK();
+    if (ready) *ready = true;
+  }
   a.vec4 = d.nz % 4 == 0;
   for (int c = 0; c < C; ++c)
     if (reinterpret_cast<uintptr_t>(mesh[c]) % 16 != 0) a.vec4 = 0;

@@ -623,6 +623,7 @@ struct NbodyWork {
   float* f4;  // force meshes, interleaved (x, y, z, -) per cell
   float2* w;
   float* brick;  // brick-paint arena (C = 1 and C = 3 share it)
+  bool* ready = nullptr;  // see launch_brick_paint
 };
 // Brick paint needs the particle grid: the mesh divided by pm_nc_factor.
 static MeshDims paint_dims(const Plan& p, long long N) {
@@ -662,7 +663,7 @@ static long long nbody_work_floats(const Plan& p) {
 static int paint_meshes(const Plan& p, float* const* mesh, int C,
                         const float* X, const float* w, int wstride,
                         float wscale, long long N, float f, float* brick,
-                        hipStream_t s) {
+                        bool* ready, hipStream_t s) {
   const long long M = p.d.rows * p.d.nz;
   const int fi = (int)f;
   const MeshDims md = paint_dims(p, N);
@@ -672,7 +673,7 @@ static int paint_meshes(const Plan& p, float* const* mesh, int C,
         make_brick_grid(p.d.nx / fi, p.d.ny / fi, p.d.nz / fi, fi);
     if (brick_paint_ok(md, g) && brick_work_floats(md, g, C) <= brick_floats(p))
       return launch_brick_paint(mesh, C, X, w, wstride, wscale, f, md, g,
-                                brick, s);
+                                brick, s, false, ready);
   }
   if (C != 1) return kUnsupported;  // C = 3 only arises on the grid path
   PMX_TRY(launch_fill(mesh[0], M, 0.0f, s));
@@ -691,7 +692,8 @@ static int force_at(const Plan& p, const float* X, long long N, float f,
   (void)M;
   {
     float* r[1] = {nw.rho};
-    PMX_TRY(paint_meshes(p, r, 1, X, nullptr, 1, 1.0f, N, f, nw.brick, s));
+    PMX_TRY(paint_meshes(p, r, 1, X, nullptr, 1, 1.0f, N, f, nw.brick,
+                         nw.ready, s));
   }
   // rho * (1/nbar) with nbar = N / Mb (tfpm.py:346-351), then r2c / Mb
   const double inv_nbar = (double)Mb / (double)N;
@@ -782,7 +784,9 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
   float* P = state + BN3;
   float* F = state + 2 * BN3;
   MeshDims md{p.d.B, p.d.nx, p.d.ny, p.d.nz, N};
-  const NbodyWork nw0 = nbody_work(p, work);
+  NbodyWork nw0 = nbody_work(p, work);
+  bool ready = false;
+  nw0.ready = &ready;
   auto at = [&](float* dst) {
     NbodyWork w = nw0;
     if (dst)
@@ -1006,7 +1010,8 @@ static int force_vjp(const Plan& p, const float* X, float* gF, float* gX,
     phi = keep;
   }
   float* gms[3] = {gm, gm + M, gm + 2 * M};
-  const int rc3 = paint_meshes(p, gms, 3, X, gc, 3, wsc, N, f, nw.brick, s);
+  const int rc3 = paint_meshes(p, gms, 3, X, gc, 3, wsc, N, f, nw.brick,
+                               nw.ready, s);
   if (rc3 != kOk && rc3 != kUnsupported) return rc3;
   const bool grid = rc3 == kOk;
   const double inv_nbar = (double)Mb / (double)N;
@@ -1197,8 +1202,9 @@ struct CoefGrad {
   int nsteps = 0;
   const float* xb0 = nullptr;
 };
+// (past the counters of the brick paint)
 static double* coef_scratch(const NbodyWork& nw) {
-  const uintptr_t a = reinterpret_cast<uintptr_t>(nw.brick);
+  const uintptr_t a = reinterpret_cast<uintptr_t>(nw.brick + 64);
   return reinterpret_cast<double*>((a + 7) & ~uintptr_t(7));
 }
 
@@ -1357,6 +1363,8 @@ static int nbody_adjoint(const Plan& p, const float* ckpt, int every,
   const long long M = p.d.rows * p.d.nz;
   const long long BN3 = (long long)p.d.B * N * 3;
   NbodyWork nw = nbody_work(p, work);
+  bool ready = false;
+  nw.ready = &ready;
   float* gm = work + nbody_work_floats(p);
   float* st = gm + 3 * M;            // scratch state (3, B, N, 3)
   const int nseg = (nsteps + every - 1) / every;
@@ -1410,6 +1418,8 @@ static int nbody_adjoint_taped(const Plan& p, float* tape, int nsteps,
                                const float* gsrc = nullptr) {
   const long long BN3 = (long long)p.d.B * N * 3;
   NbodyWork nw = nbody_work(p, work);
+  bool ready = false;
+  nw.ready = &ready;
   float* gm = work + nbody_work_floats(p);
   Tape tp = compact ? compact_tape_of(p, tape, N, nsteps)
                     : tape_of(p, tape, N, nsteps, f);
@@ -1444,6 +1454,8 @@ static int nbody_adjoint_pgd_taped(const Plan& p, float* tape, int nsteps,
                                    hipStream_t s, double* gcoef = nullptr) {
   const long long BN3 = (long long)p.d.B * N * 3;
   NbodyWork nw = nbody_work(p, work);
+  bool ready = false;
+  nw.ready = &ready;
   float* gm = work + nbody_work_floats(p);
   const Tape tp = tape_of(p, tape, N, nsteps, f, true);
   if (gpgd && nsteps > 0) {

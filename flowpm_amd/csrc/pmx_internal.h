@@ -113,6 +113,12 @@ __device__ __forceinline__ long long xcd_block(long long i, long long nb) {
   return c * q + (c < r ? c : r) + slot;
 }
 
+// The same in 32 bits, for the kernels that walk bricks.
+__device__ __forceinline__ int xcd_block32(unsigned i, unsigned nb) {
+  const unsigned q = nb >> 3, r = nb & 7, c = i & 7;
+  return (int)(c * q + (c < r ? c : r) + (i >> 3));
+}
+
 // ------------------------------------------------------ plan (device) ------
 // Per-axis tables, computed on the host in float64 and uploaded once.
 struct AxisTab {
@@ -336,11 +342,13 @@ long long brick_work_floats(const MeshDims& d, const BrickGrid& g, int C);
 const int* brick_meta(const MeshDims& d, const BrickGrid& g, int C,
                       float* work);
 // mesh[c] = sum_p w[p*wstride+c]*wscale * CIC(X*ps) (every cell written;
-// accumulate: mesh[c] += instead)
+// accumulate: mesh[c] += instead).  ready (optional, in / out): whether a paint
+// has left this workspace's counters zero since anything else wrote there.
 int launch_brick_paint(float* const* mesh, int C, const float* X,
                        const float* w, int wstride, float wscale, float ps,
                        const MeshDims& d, const BrickGrid& g, float* work,
-                       hipStream_t s, bool accumulate = false);
+                       hipStream_t s, bool accumulate = false,
+                       bool* ready = nullptr);
 
 // Force VJP pieces.
 // KDK cotangent update applied after a force VJP (see k_force_vjp_finish)
