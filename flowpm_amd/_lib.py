@@ -41,6 +41,9 @@ _SIGS = {
                                _f, _vp]),
     "pmx_cic_readout_adj": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _ll, _i, _i, _i,
                                  _f, _vp]),
+    "pmx_cic_readout_adj_work_floats": (_ll, [_i, _ll, _i, _i, _i]),
+    "pmx_cic_readout_adj_ws": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _ll, _i, _i,
+                                    _i, _f, _vp, _ll, _vp]),
     "pmx_fft_r2c": (_i, [_vp, _vp, _vp, _f, _vp]),
     "pmx_fft_c2r": (_i, [_vp, _vp, _vp, _f, _vp]),
     "pmx_spec_to_full": (_i, [_vp, _vp, _vp, _vp]),

@@ -803,3 +803,5 @@ int launch_brick_paint(float* const* mesh, int C, const float* X,
 }
 
 }  // namespace pmx
+
+#include "bin_paint.h"

@@ -1619,7 +1619,7 @@ int pmx_cic_paint(float* mesh, const float* pos, const float* weight, int B,
 // Particles that number one per mesh cell are painted with the brick paint
 // (their grid order, when it is the Lagrangian one, keeps every brick's
 // box small; any order is painted correctly, scattered bricks spill to
-// atomics).
+// atomics).  Other numbers of particles: bin_paint_ok.
 static bool grid_paint(int B, long long N, int nx, int ny, int nz, float ps,
                        BrickGrid* g) {
   if (ps != 1.0f || N != (long long)nx * ny * nz) return false;
@@ -1631,10 +1631,10 @@ static bool grid_paint(int B, long long N, int nx, int ny, int nz, float ps,
 long long pmx_cic_paint_work_floats(int B, long long N, int nx, int ny,
                                     int nz, float ps) {
   BrickGrid g;
-  if (B < 1 || nx < 1 || ny < 1 || nz < 1 ||
-      !grid_paint(B, N, nx, ny, nz, ps, &g))
-    return 0;
-  return brick_work_floats(MeshDims{B, nx, ny, nz, N}, g, 1);
+  if (B < 1 || nx < 1 || ny < 1 || nz < 1 || ps != 1.0f) return 0;
+  const MeshDims d{B, nx, ny, nz, N};
+  if (grid_paint(B, N, nx, ny, nz, ps, &g)) return brick_work_floats(d, g, 1);
+  return bin_paint_ok(d) ? bin_work_floats(d) : 0;
 }
 
 int pmx_cic_paint_ws(float* mesh, const float* pos, const float* weight,
@@ -1650,6 +1650,10 @@ int pmx_cic_paint_ws(float* mesh, const float* pos, const float* weight,
     return launch_brick_paint(m, 1, pos, weight, 1, 1.0f, ps, d, g, work,
                               S(stream), true);
   }
+  if (work && ps == 1.0f && bin_paint_ok(d) &&
+      work_floats >= bin_work_floats(d))
+    return launch_bin_paint(mesh, pos, weight, ps, d, false, work,
+                            kProfPaint, S(stream));
   return launch_paint(mesh, pos, weight, 1.0f, d, ps, 0, S(stream));
 }
 
@@ -1685,6 +1689,35 @@ int pmx_cic_readout_adj(float* gmesh, float* dpos, const float* gout,
               "pmx_cic_readout_adj: position gradient needs the mesh");
   if (!gmesh && !dpos) return kOk;  // no cotangent asked for
   MeshDims d{B, nx, ny, nz, N};
+  return launch_readout_adj(gmesh, dpos, gout, mesh, pos, d, ps, 0,
+                            S(stream));
+}
+
+long long pmx_cic_readout_adj_work_floats(int B, long long N, int nx, int ny,
+                                          int nz) {
+  if (B < 1 || nx < 1 || ny < 1 || nz < 1) return 0;
+  const MeshDims d{B, nx, ny, nz, N};
+  return bin_paint_ok(d) ? bin_work_floats(d) : 0;
+}
+
+int pmx_cic_readout_adj_ws(float* gmesh, float* dpos, const float* gout,
+                           const float* mesh, const float* pos, int B,
+                           long long N, int nx, int ny, int nz, float ps,
+                           float* work, long long work_floats, void* stream) {
+  CHECK_MESH(B, N, nx, ny, nz);
+  PMX_REQUIRE((gout && pos) || N == 0,
+              "pmx_cic_readout_adj_ws: null pointer");
+  PMX_REQUIRE(dpos == nullptr || mesh != nullptr,
+              "pmx_cic_readout_adj_ws: position gradient needs the mesh");
+  MeshDims d{B, nx, ny, nz, N};
+  if (gmesh && work && bin_paint_ok(d) && work_floats >= bin_work_floats(d)) {
+    PMX_TRY(launch_bin_paint(gmesh, pos, gout, ps, d, true, work,
+                             kProfAdjCic, S(stream)));
+    gmesh = nullptr;
+  } else if (gmesh) {
+    PMX_TRY(launch_fill(gmesh, (long long)B * nx * ny * nz, 0.0f, S(stream)));
+  }
+  if ((!gmesh && !dpos) || N == 0) return kOk;
   return launch_readout_adj(gmesh, dpos, gout, mesh, pos, d, ps, 0,
                             S(stream));
 }

@@ -350,6 +350,13 @@ int launch_brick_paint(float* const* mesh, int C, const float* X,
                        hipStream_t s, bool accumulate = false,
                        bool* ready = nullptr);
 
+// Paint of particles in any order by mesh tiles (bin_paint.h).
+bool bin_paint_ok(const MeshDims& d);
+long long bin_work_floats(const MeshDims& d);
+int launch_bin_paint(float* mesh, const float* pos, const float* w, float ps,
+                     const MeshDims& d, bool overwrite, float* work,
+                     ProfKind kind, hipStream_t s);
+
 // Force VJP pieces.
 // KDK cotangent update applied after a force VJP (see k_force_vjp_finish)
 struct AdjUpdate {

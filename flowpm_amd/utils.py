@@ -53,7 +53,8 @@ class _CicPaint(torch.autograd.Function):
     w = None if weight is None else _f32(weight).reshape(B, N)
     out = _f32(mesh).clone()
     # one particle per cell (the final paint of an nbody run): the time
-    # loop's atomic-free brick paint, on a workspace; else the scatter
+    # loop's atomic-free brick paint, on a workspace; other numbers sorted by
+    # mesh tiles on one, or the scatter
     nw = _lib.lib().pmx_cic_paint_work_floats(B, N, nx, ny, nz, 1.0)
     work = torch.empty(nw, dtype=torch.float32, device=out.device) \
         if nw > 0 else None
@@ -117,12 +118,16 @@ class _CicReadout(torch.autograd.Function):
     m, pos = ctx.saved_tensors
     B, N, nx, ny, nz = ctx.dims
     g = _f32(g)
-    gm = torch.zeros_like(m) if ctx.needs_input_grad[0] else None
+    gm = torch.empty_like(m) if ctx.needs_input_grad[0] else None
     dpos = torch.empty_like(pos) if ctx.needs_input_grad[1] else None
     if gm is not None or dpos is not None:
-      _lib.call("pmx_cic_readout_adj", _lib.ptr(gm), _lib.ptr(dpos),
+      nw = 0 if gm is None else _lib.lib().pmx_cic_readout_adj_work_floats(
+          B, N, nx, ny, nz)
+      work = torch.empty(nw, dtype=torch.float32, device=g.device) \
+          if nw > 0 else None
+      _lib.call("pmx_cic_readout_adj_ws", _lib.ptr(gm), _lib.ptr(dpos),
                 _lib.ptr(g), _lib.ptr(m), _lib.ptr(pos), B, N, nx, ny, nz,
-                1.0, _lib.stream_of(g))
+                1.0, _lib.ptr(work), nw, _lib.stream_of(g))
     if dpos is not None:
       dpos = dpos.reshape(ctx.part_shape)
     return gm, dpos

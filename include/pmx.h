@@ -68,8 +68,9 @@ int pmx_cic_paint(float* mesh, const float* pos, const float* weight, int B,
 /* pmx_cic_paint with a workspace: particles that number one per mesh cell
  * (N = nx*ny*nz, pos_scale 1: the final paint of an nbody run) go through
  * the brick paint of the time loop, which writes the mesh without atomics
- * (mesh += paint, as pmx_cic_paint); others through pmx_cic_paint's
- * scatter.  work: pmx_cic_paint_work_floats() floats (0: not applicable;
+ * (mesh += paint, as pmx_cic_paint); others, from some tens of thousands
+ * on, are sorted by mesh tiles, which are painted without atomics; the rest
+ * goes through pmx_cic_paint's scatter.  work: pmx_cic_paint_work_floats() floats (0: not applicable;
  * work may then be NULL). */
 long long pmx_cic_paint_work_floats(int B, long long N, int nx, int ny,
                                     int nz, float pos_scale);
@@ -93,6 +94,17 @@ int pmx_cic_readout_adj(float* gmesh, float* dpos, const float* gout,
                         const float* mesh, const float* pos, int B,
                         long long N, int nx, int ny, int nz, float pos_scale,
                         void* stream);
+/* The same with gmesh overwritten (it need not be cleared) and a workspace of
+ * pmx_cic_readout_adj_work_floats() floats, in which the particles are sorted
+ * by mesh tiles, so that the mesh is written without atomics (0: not
+ * applicable; work may then be NULL). */
+long long pmx_cic_readout_adj_work_floats(int B, long long N, int nx, int ny,
+                                          int nz);
+int pmx_cic_readout_adj_ws(float* gmesh, float* dpos, const float* gout,
+                           const float* mesh, const float* pos, int B,
+                           long long N, int nx, int ny, int nz,
+                           float pos_scale, float* work,
+                           long long work_floats, void* stream);
 
 /* ---- FFT: flowpm/utils.py:213-241 (r2c3d), :244-272 (c2r3d) ---- */
 /* spec = fft3d(in) * scale, half spectrum (r2c3d with scale = 1/norm) */
