@@ -9,18 +9,16 @@
 // reach into LDS, and every particle forms the gradient at its 8 corners
 // there; closing kick, opening kick and drift follow in registers.
 //
-// What bounds it: the LDS reads (56 potential values per particle as 28
-// two-float reads; late positions spread them unevenly over the banks, 10
-// clocks a read instead of 4) and the VALU work (about 230 operations per
-// particle and 120 per thread for the fill), each about 140 of the 252 us it
-// takes at 256^3, then the particle streams (48 bytes per particle).  The
-// gradient mesh it replaces costs 12 bytes per cell written and 8 scattered
-// 12-byte gathers per particle; the potential boxes overlap (about 2.7 times
-// the mesh at a = 0.5) but are a third of the bytes and come from the 256 MB
-// cache in rows of whole quads.  Gradient + readout before -> here, one force
-// evaluation: 256^3 (a = 0.1 to 1) 327 -> 252 us, 512^3 (a = 0.5) 2760 ->
-// 1683, 16 x 64^3 73 -> 53; at 32^3 to 64^3 the two kernels took 8 to 11 us
-// against 11 here, but one launch less makes the run 1 to 3 % faster.
+// What bounds it: memory, 48 bytes of state per particle and step and about 11
+// of potential (the boxes overlap, about 2.7 times the mesh at a = 0.5), 210
+// of the 255 us it takes at 256^3 at the rate of a large copy; then the LDS
+// reads (56 potential values per particle as 28 two-float reads; late
+// positions spread them unevenly over the banks, 10 clocks a read instead of
+// 4) and the VALU work, each about 130 us.  The gradient mesh it replaces
+// costs 12 bytes per cell written and 8 scattered 12-byte gathers per
+// particle.  Gradient + readout before -> here, one force evaluation: 256^3
+// (a = 0.1 to 1) 327 -> 255 us, 512^3 (a = 0.5, with the copies of a first
+// step) 2760 -> 2290, 16 x 64^3 73 -> 55, 64^3 10.5 -> 9.6, 32^3 8 -> 6.7.
 #pragma once
 #include "pmx_internal.h"
 
@@ -143,51 +141,58 @@ static __device__ __forceinline__ Box make_box(const int (&lo)[3],
   return q;
 }
 
-// Planes s0 .. s0 + np - 1 of the box of mesh pm into win: 8 lanes of quads
-// per row, T / 8 rows at a time, U loads in flight per thread.
-template <int T>
+// i modulo n, of an i that is mostly in range or one side off (a scalar
+// division is some 40 instructions of the scalar unit the whole CU shares)
+static __device__ __forceinline__ int near_mod(int i, int n) {
+  if (i < 0) i += n;
+  if (i >= n) i -= n;
+  if ((unsigned)i >= (unsigned)n) i = imod(i, n);
+  return i;
+}
+
+// Planes s0 .. s0 + np - 1 of the box of mesh pm into win: the quads of all
+// rows in one sequence, T at a time, U loads in flight per thread.
+// ONCE: rows and planes wrap at most once (the box is not longer than the
+// sides).
+template <int T, bool ONCE>
 static __device__ __forceinline__ void fill_box(float* win, const float* pm,
                                                 const MeshDims& d,
                                                 const Box& q, int s0, int np) {
-  constexpr int U = 8;
-  const int x0 = imod(q.x0 + s0, d.nx), y0 = imod(q.y0, d.ny),
-            z0 = imod(q.z0, d.nz);
-  // rows and planes wrap at most once (the box is not longer than the sides)
-  const bool once = q.px <= d.nx && q.py <= d.ny;
-  const int rows = np * q.py;
-  const unsigned my = magic(q.py);
-  for (int zq = threadIdx.x & 7; zq < q.nzq; zq += 8) {
-    int z = z0 + 4 * zq;
-    while (z >= d.nz) z -= d.nz;  // a box may be longer than the side
-    for (int r0 = threadIdx.x >> 3; r0 < rows; r0 += T / 8 * U) {
-      V4 v[U];
-      int at[U];
+  constexpr int U = 4;
+  const unsigned x0 = near_mod(q.x0 + s0, d.nx), y0 = near_mod(q.y0, d.ny),
+                 z0 = near_mod(q.z0, d.nz);
+  const unsigned nx = d.nx, ny = d.ny, nz = d.nz;
+  const int quads = np * q.py * q.nzq;
+  const unsigned my = magic(q.py), mz = magic(q.nzq);
+  for (int i0 = threadIdx.x; i0 < quads; i0 += T * U) {
+    V4 v[U];
+    int at[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const unsigned r = min(r0 + u * (T / 8), rows - 1);
-        const unsigned xx = __umulhi(r, my);
-        unsigned y = r - xx * q.py, x = x0 + xx;
-        at[u] = (int)(xx * q.plane + y * q.pz);
-        y += y0;
-        if (once) {
-          y = min(y, y - (unsigned)d.ny);
-          x = min(x, x - (unsigned)d.nx);
-        } else {
-          y %= (unsigned)d.ny;
-          x %= (unsigned)d.nx;
-        }
-        // 32-bit byte offset: a member has at most 2^30 cells
-        const unsigned off = 4u * ((x * d.ny + y) * d.nz + (unsigned)z);
-        v[u] = *reinterpret_cast<const V4*>(
-            reinterpret_cast<const char*>(pm) + off);
+    for (int u = 0; u < U; ++u) {
+      const unsigned i = min(i0 + u * T, quads - 1);
+      const unsigned r = __umulhi(i, mz), zq = i - r * q.nzq;
+      const unsigned xx = __umulhi(r, my), yy = r - xx * q.py;
+      at[u] = (int)(xx * q.plane + yy * q.pz + 4 * zq);
+      unsigned x = x0 + xx, y = y0 + yy, z = z0 + 4 * zq;
+      if (ONCE) {
+        x = min(x, x - nx);
+        y = min(y, y - ny);
+        z = min(z, z - nz);
+      } else {
+        x %= nx;
+        y %= ny;
+        z %= nz;
       }
+      // 32-bit byte offset: a member has at most 2^30 cells
+      v[u] = *reinterpret_cast<const V4*>(reinterpret_cast<const char*>(pm) +
+                                          4u * ((x * ny + y) * nz + z));
+    }
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (r0 + u * (T / 8) < rows) {
-          float* const w = win + at[u] + 4 * zq;
+    for (int u = 0; u < U; ++u) {
+      if (i0 + u * T < quads) {
+        float* const w = win + at[u];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) w[e] = v[u][e];
-        }
+        for (int e = 0; e < 4; ++e) w[e] = v[u][e];
       }
     }
   }
@@ -234,15 +239,19 @@ struct WinPair {
 // META: the bricks' boxes are those the paint of the same positions stored
 // (paint.hip), so the potential and the particles are loaded together;
 // otherwise the workgroup finds the box first.
-template <bool META>
+// PLAIN: none of the copies of a tape, of a first step or of kept positions.
+template <bool META, bool PLAIN>
 __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
     float* X, float* P, float* F, const float* __restrict__ phi,
-    const int* __restrict__ meta, MeshDims d, BrickGrid g, KickDrift c) {
+    const int* __restrict__ meta, MeshDims d, BrickGrid g, KickDrift c,
+    int rounds_each) {
   __shared__ float win[kBoxWin];
   __shared__ int red[META ? 1 : kBoxT / 64][6];
   const int tid = threadIdx.x;
-  const int bid = (int)xcd_block(blockIdx.x, gridDim.x);
+  const int bid = xcd_block32(blockIdx.x, gridDim.x);
   const int b = blockIdx.y;
+  // this workgroup's rounds of kBoxT particles
+  const int ua = blockIdx.z * rounds_each, ub = ua + rounds_each;
   int q0[3], cnt[3];
   brick_block(g, bid, q0, cnt);
   // z fastest, then x: the 4 rows of a wave are a plane apart in LDS
@@ -252,9 +261,13 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
   const long long o0 =
       3 * ((long long)b * d.N +
            ((long long)q0[0] * g.gy + q0[1]) * g.gz + q0[2]);
+  const float rz = 1.0f / (float)cz, rx = 1.0f / (float)cx;
   auto poff = [&](int t) {
     const int tt = t < nloc ? t : 0;
-    const int lz = tt % cz, q = tt / cz, lx = q % cx, ly = q / cx;
+    // exact divisions: tt < 2048, and (tt + 1/2) / c is 1 / 2c off a whole
+    // number
+    const int q = (int)(((float)tt + 0.5f) * rz), lz = tt - q * cz,
+              ly = (int)(((float)q + 0.5f) * rx), lx = q - ly * cx;
     return 12u * (unsigned)((lx * g.gy + ly) * g.gz + lz);
   };
   // whole y planes of the brick per round of kBoxT particles: the next
@@ -262,10 +275,10 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
   const bool even = nloc % kBoxT == 0 && kBoxT % (cx * cz) == 0;
   const unsigned pstep = even ? 12u * (unsigned)(kBoxT / (cx * cz)) * g.gz : 0u;
   const bool kick = c.do_k2 || c.do_k1d;
-  const bool useP = kick || c.copy_xp;
+  const bool useP = kick || (!PLAIN && c.copy_xp);
   const float* const Xl = (c.xin ? c.xin : X) + o0;
   const float* const Pl = (c.pin ? c.pin : P) + o0;
-  const unsigned o_first = poff(tid);
+  const unsigned o_first = poff(tid + ua * kBoxT);
   unsigned on = o_first;
   float xn[3], pn[3] = {0.f, 0.f, 0.f};
 #pragma unroll
@@ -343,11 +356,14 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
     if (hx >= 6) {
       nxw = min(hx, q.px - s0);
       if (s0 > 0) __syncthreads();  // the window is reused
-      fill_box<kBoxT>(win, pm, d, q, s0, nxw);
+      if (q.px <= d.nx && q.py <= d.ny && 4 * q.nzq <= d.nz)
+        fill_box<kBoxT, true>(win, pm, d, q, s0, nxw);
+      else
+        fill_box<kBoxT, false>(win, pm, d, q, s0, nxw);
       __syncthreads();
     }
 #pragma unroll 1
-    for (int u = 0; u < 4; ++u) {
+    for (int u = ua; u < ub; ++u) {
       const int t = tid + u * kBoxT;
       const unsigned o = on;
       float x[3], p[3];
@@ -357,7 +373,7 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
         p[e] = pn[e];
       }
       // the next particle's loads (the first one's again for a next window)
-      on = u == 3 ? o_first : (even ? on + pstep : poff(t + kBoxT));
+      on = u == ub - 1 ? o_first : (even ? on + pstep : poff(t + kBoxT));
 #pragma unroll
       for (int e = 0; e < 3; ++e) xn[e] = ldo(Xl, on, e);
       if (useP) {
@@ -388,21 +404,23 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
         for (int e = 0; e < 3; ++e) sto(v[e], q + o0, o, e);
       };
       if (!c.skip_f) store(r, F);
-      if (c.xkeep) store(x, c.xkeep);
-      if (c.copy_xp) {
-        store(x, X);
-        store(p, P);
-      }
-      if (c.ckpt) {
-        store(x, c.ckpt);
-        store(r, c.ckpt + 6 * tot);
+      if (!PLAIN) {
+        if (c.xkeep) store(x, c.xkeep);
+        if (c.copy_xp) {
+          store(x, X);
+          store(p, P);
+        }
+        if (c.ckpt) {
+          store(x, c.ckpt);
+          store(r, c.ckpt + 6 * tot);
+        }
       }
       if (kick) {
         if (c.do_k2) {
 #pragma unroll
           for (int e = 0; e < 3; ++e) p[e] = p[e] + c.k2 * r[e];
         }
-        if (c.ckpt) store(p, c.ckpt + 3 * tot);
+        if (!PLAIN && c.ckpt) store(p, c.ckpt + 3 * tot);
         if (c.do_k1d) {
 #pragma unroll
           for (int e = 0; e < 3; ++e) {
@@ -410,7 +428,7 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
             x[e] = x[e] + c.d * p[e];
           }
           store(x, c.xout ? c.xout : X);
-          if (c.xcopy) store(x, c.xcopy);
+          if (!PLAIN && c.xcopy) store(x, c.xcopy);
         }
         store(p, P);
       }
@@ -433,9 +451,18 @@ int launch_readout_box(float* X, float* P, float* F, const float* phi,
               "readout_box: one particle per cell, 16-byte aligned arrays");
   ProfScope prof_(kProfReadoutKD, s);
   const BrickGrid g = make_brick_grid(d.nx, d.ny, d.nz, 1);
-  auto kern = meta ? k_readout_box<true> : k_readout_box<false>;
-  hipLaunchKernelGGL(kern, dim3(g.nbricks, d.B), dim3(kBoxT), 0, s, X, P, F,
-                     phi, meta, d, g, c);
+  const bool plain = !c.xkeep && !c.copy_xp && !c.ckpt && !c.xcopy;
+  auto kern = meta ? (plain ? k_readout_box<true, true>
+                            : k_readout_box<true, false>)
+                   : (plain ? k_readout_box<false, true>
+                            : k_readout_box<false, false>);
+  // few bricks, which leave most of the chip idle: their particles by several
+  // workgroups, each with the whole box: 32 bricks (32^3) 10.8 us by one, 7.9
+  // by two, 6.7 by four; 128 (64^3) 12.8 / 9.6 / 11.2; 2048 55 / 68 / 96
+  const long long nb = (long long)g.nbricks * d.B;
+  const int parts = nb <= 64 ? 4 : (nb <= 128 ? 2 : 1);
+  hipLaunchKernelGGL(kern, dim3(g.nbricks, d.B, parts), dim3(kBoxT), 0, s, X,
+                     P, F, phi, meta, d, g, c, 4 / parts);
   PMX_LAUNCH_CHECK();
   return kOk;
 }
