@@ -36,6 +36,8 @@ _SIGS = {
     "pmx_cic_paint_work_floats": (_ll, [_i, _ll, _i, _i, _i, _f]),
     "pmx_cic_paint_ws": (_i, [_vp, _vp, _vp, _i, _ll, _i, _i, _i, _f, _vp,
                               _ll, _vp]),
+    "pmx_cic_paint_from": (_i, [_vp, _vp, _vp, _vp, _i, _ll, _i, _i, _i, _f,
+                                _vp, _ll, _vp]),
     "pmx_cic_readout": (_i, [_vp, _vp, _vp, _i, _ll, _i, _i, _i, _f, _vp]),
     "pmx_cic_paint_adj": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _ll, _i, _i, _i,
                                _f, _vp]),

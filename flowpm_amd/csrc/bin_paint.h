@@ -38,6 +38,7 @@ constexpr long long kBinMin = 19 * 2048, kBinSparse = 80;
 
 struct BinArgs {
   float* mesh;
+  const float* base;  // added to, or null; may be the mesh itself
   const float* pos;
   const float* w;  // or null (ones)
   float ps;
@@ -268,7 +269,6 @@ __device__ __forceinline__ long long bin_cell(const BinArgs& a, int tile,
 // atomics) and the tiles' unequal loads: 512 threads with two entries each in
 // flight take 40 us for 2 x 96^3 particles, 256 threads with one 55, with two
 // 45, 1024 with two 43.
-template <bool OVER>
 __global__ __launch_bounds__(kBinPT) void k_bin_paint(BinArgs a) {
   __shared__ BinLds l;
   const int b = blockIdx.y;
@@ -281,12 +281,12 @@ __global__ __launch_bounds__(kBinPT) void k_bin_paint(BinArgs a) {
     h[1] = b;
     h[2] = (int)((n - 1) / kBinShare);  // further workgroups' shares
   }
-  if (!OVER && n == 0) return;
+  if (a.base == a.mesh && n == 0) return;
   __syncthreads();
   for (int i = threadIdx.x; i < kBinCells; i += kBinPT) {
     const long long c = bin_cell(a, tile, b, i);
     if (c >= 0)
-      a.mesh[c] = OVER ? (float)l.box[i] : (float)((double)a.mesh[c] + l.box[i]);
+      a.mesh[c] = (float)(a.base ? (double)a.base[c] + l.box[i] : l.box[i]);
   }
 }
 
@@ -346,12 +346,13 @@ long long bin_work_floats(const MeshDims& d) {
          4 + 4LL * d.B * a.ntiles;
 }
 
-// mesh (+)= CIC(pos * ps, w); the caller has asked bin_paint_ok
-int launch_bin_paint(float* mesh, const float* pos, const float* w, float ps,
-                     const MeshDims& d, bool overwrite, float* work,
+// (the caller has asked bin_paint_ok)
+int launch_bin_paint(float* mesh, const float* base, const float* pos,
+                     const float* w, float ps, const MeshDims& d, float* work,
                      ProfKind kind, hipStream_t s) {
   BinArgs a = bin_args(d);
   a.mesh = mesh;
+  a.base = base;
   a.pos = pos;
   a.w = w;
   a.ps = ps;
@@ -362,12 +363,7 @@ int launch_bin_paint(float* mesh, const float* pos, const float* w, float ps,
   hipLaunchKernelGGL(k_bin_sort, dim3(a.nchunk, d.B), dim3(kBinT),
                      a.ntiles * sizeof(unsigned), s, a);
   PMX_LAUNCH_CHECK();
-  if (overwrite)
-    hipLaunchKernelGGL(k_bin_paint<true>, dim3(a.ntiles, d.B), dim3(kBinPT), 0,
-                       s, a);
-  else
-    hipLaunchKernelGGL(k_bin_paint<false>, dim3(a.ntiles, d.B), dim3(kBinPT),
-                       0, s, a);
+  hipLaunchKernelGGL(k_bin_paint, dim3(a.ntiles, d.B), dim3(kBinPT), 0, s, a);
   PMX_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_bin_tail, dim3(kBinTail), dim3(kBinPT), 0, s, a);
   PMX_LAUNCH_CHECK();

@@ -673,7 +673,7 @@ static int paint_meshes(const Plan& p, float* const* mesh, int C,
         make_brick_grid(p.d.nx / fi, p.d.ny / fi, p.d.nz / fi, fi);
     if (brick_paint_ok(md, g) && brick_work_floats(md, g, C) <= brick_floats(p))
       return launch_brick_paint(mesh, C, X, w, wstride, wscale, f, md, g,
-                                brick, s, false, ready);
+                                brick, s, nullptr, ready);
   }
   if (C != 1) return kUnsupported;  // C = 3 only arises on the grid path
   PMX_TRY(launch_fill(mesh[0], M, 0.0f, s));
@@ -1637,24 +1637,36 @@ long long pmx_cic_paint_work_floats(int B, long long N, int nx, int ny,
   return bin_paint_ok(d) ? bin_work_floats(d) : 0;
 }
 
-int pmx_cic_paint_ws(float* mesh, const float* pos, const float* weight,
-                     int B, long long N, int nx, int ny, int nz, float ps,
-                     float* work, long long work_floats, void* stream) {
+int pmx_cic_paint_from(float* out, const float* mesh, const float* pos,
+                       const float* weight, int B, long long N, int nx, int ny,
+                       int nz, float ps, float* work, long long work_floats,
+                       void* stream) {
   CHECK_MESH(B, N, nx, ny, nz);
-  PMX_REQUIRE(mesh && (pos || N == 0), "pmx_cic_paint_ws: null pointer");
+  PMX_REQUIRE(out && mesh && (pos || N == 0),
+              "pmx_cic_paint_from: null pointer");
   MeshDims d{B, nx, ny, nz, N};
   BrickGrid g;
   if (work && grid_paint(B, N, nx, ny, nz, ps, &g) &&
       work_floats >= brick_work_floats(d, g, 1)) {
-    float* m[1] = {mesh};
+    float* m[1] = {out};
     return launch_brick_paint(m, 1, pos, weight, 1, 1.0f, ps, d, g, work,
-                              S(stream), true);
+                              S(stream), mesh);
   }
   if (work && ps == 1.0f && bin_paint_ok(d) &&
       work_floats >= bin_work_floats(d))
-    return launch_bin_paint(mesh, pos, weight, ps, d, false, work,
-                            kProfPaint, S(stream));
-  return launch_paint(mesh, pos, weight, 1.0f, d, ps, 0, S(stream));
+    return launch_bin_paint(out, mesh, pos, weight, ps, d, work, kProfPaint,
+                            S(stream));
+  if (out != mesh)
+    PMX_HIP_CHECK(hipMemcpyAsync(out, mesh, sizeof(float) * B * nx * ny * nz,
+                                 hipMemcpyDeviceToDevice, S(stream)));
+  return launch_paint(out, pos, weight, 1.0f, d, ps, 0, S(stream));
+}
+
+int pmx_cic_paint_ws(float* mesh, const float* pos, const float* weight,
+                     int B, long long N, int nx, int ny, int nz, float ps,
+                     float* work, long long work_floats, void* stream) {
+  return pmx_cic_paint_from(mesh, mesh, pos, weight, B, N, nx, ny, nz, ps,
+                            work, work_floats, stream);
 }
 
 int pmx_cic_readout(float* out, const float* mesh, const float* pos, int B,
@@ -1711,7 +1723,7 @@ int pmx_cic_readout_adj_ws(float* gmesh, float* dpos, const float* gout,
               "pmx_cic_readout_adj_ws: position gradient needs the mesh");
   MeshDims d{B, nx, ny, nz, N};
   if (gmesh && work && bin_paint_ok(d) && work_floats >= bin_work_floats(d)) {
-    PMX_TRY(launch_bin_paint(gmesh, pos, gout, ps, d, true, work,
+    PMX_TRY(launch_bin_paint(gmesh, nullptr, pos, gout, ps, d, work,
                              kProfAdjCic, S(stream)));
     gmesh = nullptr;
   } else if (gmesh) {

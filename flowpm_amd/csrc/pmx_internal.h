@@ -341,20 +341,21 @@ long long brick_work_floats(const MeshDims& d, const BrickGrid& g, int C);
 // where launch_brick_paint leaves the boxes of its bricks (8 ints each)
 const int* brick_meta(const MeshDims& d, const BrickGrid& g, int C,
                       float* work);
-// mesh[c] = sum_p w[p*wstride+c]*wscale * CIC(X*ps) (every cell written;
-// accumulate: mesh[c] += instead).  ready (optional, in / out): whether a paint
+// mesh[c] = sum_p w[p*wstride+c]*wscale * CIC(X*ps) (every cell written), plus
+// base, if given (C = 1; it may be the mesh itself).  ready (optional, in / out): whether a paint
 // has left this workspace's counters zero since anything else wrote there.
 int launch_brick_paint(float* const* mesh, int C, const float* X,
                        const float* w, int wstride, float wscale, float ps,
                        const MeshDims& d, const BrickGrid& g, float* work,
-                       hipStream_t s, bool accumulate = false,
+                       hipStream_t s, const float* base = nullptr,
                        bool* ready = nullptr);
 
 // Paint of particles in any order by mesh tiles (bin_paint.h).
 bool bin_paint_ok(const MeshDims& d);
 long long bin_work_floats(const MeshDims& d);
-int launch_bin_paint(float* mesh, const float* pos, const float* w, float ps,
-                     const MeshDims& d, bool overwrite, float* work,
+// mesh = base (null: 0) + CIC(pos * ps, w)
+int launch_bin_paint(float* mesh, const float* base, const float* pos,
+                     const float* w, float ps, const MeshDims& d, float* work,
                      ProfKind kind, hipStream_t s);
 
 // Force VJP pieces.

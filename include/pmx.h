@@ -78,6 +78,11 @@ int pmx_cic_paint_ws(float* mesh, const float* pos, const float* weight,
                      int B, long long N, int nx, int ny, int nz,
                      float pos_scale, float* work, long long work_floats,
                      void* stream);
+/* pmx_cic_paint_ws into another mesh: out = mesh + paint. */
+int pmx_cic_paint_from(float* out, const float* mesh, const float* pos,
+                       const float* weight, int B, long long N, int nx, int ny,
+                       int nz, float pos_scale, float* work,
+                       long long work_floats, void* stream);
 /* out[b][p] = sum_corners mesh * w(pos * pos_scale) */
 int pmx_cic_readout(float* out, const float* mesh, const float* pos, int B,
                     long long N, int nx, int ny, int nz, float pos_scale,
