@@ -734,6 +734,117 @@ __global__ __launch_bounds__(T) void k_xpass(XJob J, PlanDev p) {
   }
 }
 
+// ---------------------------------------------------------- planes ------
+// The z and y passes of a whole y-z plane (square, sides up to kPlaneN) in one
+// launch: the plane stays in LDS between them.  The same operations in the
+// same order as the two passes, and the same results.  Small passes are bound
+// by their launch and its chain of loads, stages and stores, so one of them is
+// nearly saved: forward + inverse, four passes -> two planes, 32^3 15.2 -> 9.1
+// us, 64^3 18.9 -> 10.8, 16 x 64^3 39.2 -> 22.4 (half the traffic).  With 256
+// threads 9.6, 12.6 and 23.9, with 128 10.5, 16.8 and 25.1.  The limit is a
+// plane's two tiles, 34 KB at 64, for four workgroups per CU.
+template <int N, int T>
+__global__ __launch_bounds__(T) void k_plane_r2c(ZJobs jobs, PlanDev p) {
+  constexpr int H = N / 2, TZ = N / 2, TY = H + 1;
+  constexpr int P = Pitch<TZ>::P, PY = Pitch<TY>::P;
+  __shared__ float2 s[N * P];   // z lines: row pairs as re / im
+  __shared__ float2 w[N * PY];  // y lines: columns kz = 0 .. H
+  __shared__ float2 tw[N];
+  const ZJob J = blockIdx.y == 0 ? jobs.j[0]
+                 : (blockIdx.y == 1 ? jobs.j[1] : jobs.j[2]);
+  load_twiddles<N, T>(tw, p.ax[2].tw);
+  const long long r0 = (long long)blockIdx.x * N;
+  const float* __restrict__ src = J.rin + r0 * N;
+  float* sf = reinterpret_cast<float*>(s);
+  {
+    constexpr int E = (N * N + T - 1) / T;
+    float v[E];
+#pragma unroll
+    for (int u = 0; u < E; ++u) v[u] = src[min((int)threadIdx.x + u * T, N * N - 1)];
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      const int q = threadIdx.x + u * T;
+      const int row = q / N, z = q % N;
+      if ((N * N) % T == 0 || q < N * N)
+        sf[2 * (z * P + (row >> 1)) + (row & 1)] = v[u];
+    }
+  }
+  __syncthreads();
+  fft_tile<N, TZ, T, -1>(s, tw);
+  const float sc = J.scale;
+  for (int q = threadIdx.x; q < N * H; q += T) {
+    const int row = q / H, k = q % H;
+    const float2 zk = s[k * P + (row >> 1)];
+    const float2 zn = s[((N - k) % N) * P + (row >> 1)];
+    float2 v;
+    if (row & 1)
+      v = make_float2(0.5f * (zk.y + zn.y), -0.5f * (zk.x - zn.x));
+    else
+      v = make_float2(0.5f * (zk.x + zn.x), 0.5f * (zk.y - zn.y));
+    w[row * PY + k] = cscale(v, sc);
+  }
+  for (int row = threadIdx.x; row < N; row += T) {
+    const float2 zk = s[H * P + (row >> 1)];
+    float2 v = (row & 1) ? make_float2(zk.y, 0.0f) : make_float2(zk.x, 0.0f);
+    w[row * PY + H] = cscale(v, sc);
+  }
+  __syncthreads();
+  fft_tile<N, TY, T, -1>(w, tw);
+  float2* __restrict__ dst = J.cout + r0 * H;
+  for (int q = threadIdx.x; q < N * H; q += T)
+    dst[q] = w[q / H * PY + q % H];
+  for (int row = threadIdx.x; row < N; row += T)
+    J.cout[p.nyq0 + r0 + row] = w[row * PY + H];
+}
+
+template <int N, int T>
+__global__ __launch_bounds__(T) void k_plane_c2r(ZJob J, PlanDev p) {
+  constexpr int H = N / 2, TZ = N / 2, TY = H + 1;
+  constexpr int P = Pitch<TZ>::P, PY = Pitch<TY>::P;
+  __shared__ float2 s[N * P];
+  __shared__ float2 w[N * PY];
+  __shared__ float2 tw[N];
+  load_twiddles<N, T>(tw, p.ax[2].tw);
+  const long long r0 = (long long)blockIdx.x * N;
+  const float2* __restrict__ src = J.cin + r0 * H;
+  {
+    constexpr int E = (N * H + T - 1) / T;
+    float2 v[E];
+#pragma unroll
+    for (int u = 0; u < E; ++u) v[u] = src[min((int)threadIdx.x + u * T, N * H - 1)];
+    const float2 ny = J.cin[p.nyq0 + r0 + min((int)threadIdx.x, N - 1)];
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      const int q = threadIdx.x + u * T;
+      if ((N * H) % T == 0 || q < N * H) w[q / H * PY + q % H] = v[u];
+    }
+    static_assert(T >= N, "one Nyquist column entry per thread");
+    if (threadIdx.x < N) w[threadIdx.x * PY + H] = ny;
+  }
+  __syncthreads();
+  fft_tile<N, TY, T, +1>(w, tw);
+  for (int q = threadIdx.x; q < TZ * (H + 1); q += T) {
+    const int l = q / (H + 1), k = q % (H + 1);
+    float2 a = w[2 * l * PY + k], b = w[(2 * l + 1) * PY + k];
+    if (k == 0 || k == H) {
+      a.y = 0.0f;
+      b.y = 0.0f;
+    }
+    s[k * P + l] = make_float2(a.x - b.y, a.y + b.x);
+    if (k > 0 && k < H)  // conj(X1) + i conj(X2)
+      s[(N - k) * P + l] = make_float2(a.x + b.y, -a.y + b.x);
+  }
+  __syncthreads();
+  fft_tile<N, TZ, T, +1>(s, tw);
+  float* __restrict__ dst = J.rout + r0 * N;
+  const float sc = J.scale;
+  for (int q = threadIdx.x; q < N * N; q += T) {
+    const int row = q / N, z = q % N;
+    const float2 v = s[z * P + (row >> 1)];
+    dst[q] = sc * ((row & 1) ? v.y : v.x);
+  }
+}
+
 // -------------------------------------------- full <-> half spectrum -----
 // full[b][x][y][z] (the reference's complex64 layout) from the half spectrum.
 __global__ void k_spec_to_full(const float2* __restrict__ spec,
@@ -956,6 +1067,43 @@ int launch_xpass(const Plan& p, const XJob& job, hipStream_t s) {
 #undef PMX_CASE
   }
   set_error("unsupported nx");
+  return kUnsupported;
+}
+
+template <int N>
+static int plane_n(const Plan& pl, const ZJobs* r2c, const ZJob* c2r,
+                   hipStream_t s) {
+  constexpr int T = 512;
+  const PlanDev& p = pl.d;
+  if (r2c) {
+    ProfScope prof_(kProfZr2c, s);
+    hipLaunchKernelGGL((k_plane_r2c<N, T>), dim3(p.B * p.nx, r2c->n), dim3(T),
+                       0, s, *r2c, p);
+    PMX_LAUNCH_CHECK();
+  }
+  if (c2r) {
+    ProfScope prof_(kProfZc2r, s);
+    hipLaunchKernelGGL((k_plane_c2r<N, T>), dim3(p.B * p.nx), dim3(T), 0, s,
+                       *c2r, p);
+    PMX_LAUNCH_CHECK();
+  }
+  return kOk;
+}
+bool plane_ok(const Plan& p) {
+  return p.d.ny == p.d.nz && p.d.nz <= kPlaneN;
+}
+int launch_plane(const Plan& p, const ZJobs* r2c, const ZJob* c2r,
+                 hipStream_t s) {
+  switch (p.d.nz) {
+#define PMX_CASE(n)                            \
+  case n:                                      \
+    if constexpr (n <= kPlaneN)                \
+      return plane_n<n>(p, r2c, c2r, s);       \
+    break;
+    PMX_FFT_SIZES(PMX_CASE)
+#undef PMX_CASE
+  }
+  set_error("unsupported plane");
   return kUnsupported;
 }
 

@@ -168,9 +168,25 @@ static int r2c_zy(const Plan& p, const float* const* in, float2* const* spec,
     zj.j[i] = zr2c(in[i], spec[i], scale);
     yj.j[i] = yfwd(spec[i]);
   }
+  if (plane_ok(p)) return launch_plane(p, &zj, nullptr, s);
   PMX_TRY(launch_zpass_r2c(p, zj, s));
   PMX_TRY(launch_ypass(p, yj, 0, s));
   return kOk;
+}
+
+// Inverse y and z passes of one spectrum (in place) whose x pass is done, to
+// the real mesh of job j.
+static int c2r_yz(const Plan& p, const ZJob& j, float2* spec, hipStream_t s) {
+  if (plane_ok(p) && j.ez == 0 && !j.accum && j.ostride <= 1 && j.ocomp == 0)
+    return launch_plane(p, nullptr, &j, s);
+  YJobs yj{};
+  yj.n = 1;
+  yj.j[0] = yfwd(spec);
+  PMX_TRY(launch_ypass(p, yj, 1, s));
+  ZJobs zj{};
+  zj.n = 1;
+  zj.j[0] = j;
+  return launch_zpass_c2r(p, zj, s);
 }
 
 // From a spectrum whose x pass is pending (fwd = 1) or done (fwd = 0):
@@ -257,17 +273,8 @@ static int force_mesh_f4(const Plan& p, const float* rho, float2* w,
   xj.do_fwd = 1;
   xj.do_inv = 1;
   PMX_TRY(launch_xpass(p, xj, s));
-  YJobs yj{};
-  yj.n = 1;
-  yj.j[0].in = w;
-  yj.j[0].nout = 1;
-  yj.j[0].out[0] = w;
-  yj.j[0].scale[0] = 1.0f;
-  PMX_TRY(launch_ypass(p, yj, 1, s));
-  ZJobs zj{};
-  zj.n = 1;
-  zj.j[0] = zc2r(w, phi, 1.0f, 0);
-  PMX_TRY(launch_zpass_c2r(p, zj, s));
+  ZJob zj = zc2r(w, phi, 1.0f, 0);
+  PMX_TRY(c2r_yz(p, zj, w, s));
   return nc ? launch_grad_mesh(p, phi, f4, nc, s) : kOk;
 }
 
@@ -308,21 +315,12 @@ static int force_meshes_adj(const Plan& p, const float* gx, const float* gy,
     xj.do_fwd = 1;
     xj.do_inv = 1;
     PMX_TRY(launch_xpass(p, xj, s));
-    YJobs yj{};
-    yj.n = 1;
-    yj.j[0].in = w;
-    yj.j[0].nout = 1;
-    yj.j[0].out[0] = w;
-    yj.j[0].scale[0] = 1.0f;
-    PMX_TRY(launch_ypass(p, yj, 1, s));
-    ZJobs zj{};
-    zj.n = 1;
-    zj.j[0] = zc2r(w, f4w ? f4w : grho, 1.0f, 0);
+    ZJob zj = zc2r(w, f4w ? f4w : grho, 1.0f, 0);
     if (f4w) {
-      zj.j[0].ostride = 4;
-      zj.j[0].ocomp = 3;
+      zj.ostride = 4;
+      zj.ocomp = 3;
     }
-    return launch_zpass_c2r(p, zj, s);
+    return c2r_yz(p, zj, w, s);
   }
   float2* ws[3] = {w, w + p.d.S, w + 2 * p.d.S};
   const float* in[3] = {gx, gy, gz};
@@ -338,21 +336,12 @@ static int force_meshes_adj(const Plan& p, const float* gx, const float* gy,
   xj.do_fwd = 1;
   xj.do_inv = 1;
   PMX_TRY(launch_xpass(p, xj, s));
-  YJobs yj{};
-  yj.n = 1;
-  yj.j[0].in = ws[0];
-  yj.j[0].nout = 1;
-  yj.j[0].out[0] = ws[0];
-  yj.j[0].scale[0] = 1.0f;
-  PMX_TRY(launch_ypass(p, yj, 1, s));
-  ZJobs zj{};
-  zj.n = 1;
-  zj.j[0] = zc2r(ws[0], f4w ? f4w : grho, 1.0f, 0);
+  ZJob zj = zc2r(ws[0], f4w ? f4w : grho, 1.0f, 0);
   if (f4w) {
-    zj.j[0].ostride = 4;
-    zj.j[0].ocomp = 3;
+    zj.ostride = 4;
+    zj.ocomp = 3;
   }
-  PMX_TRY(launch_zpass_c2r(p, zj, s));
+  PMX_TRY(c2r_yz(p, zj, ws[0], s));
   return kOk;
 }
 
@@ -400,18 +389,9 @@ static int fourier_apply(const Plan& p, int nin, const float* const* in,
   xj.do_fwd = 1;
   xj.do_inv = 1;
   PMX_TRY(launch_xpass(p, xj, s));
-  YJobs yj{};
-  yj.n = 1;
-  yj.j[0].in = ws[0];
-  yj.j[0].nout = 1;
-  yj.j[0].out[0] = ws[0];
-  yj.j[0].scale[0] = 1.0f;
-  PMX_TRY(launch_ypass(p, yj, 1, s));
-  ZJobs zj{};
-  zj.n = 1;
-  zj.j[0] = zc2r(ws[0], out, 1.0f, 0);
-  zj.j[0].accum = accum;
-  return launch_zpass_c2r(p, zj, s);
+  ZJob zj = zc2r(ws[0], out, 1.0f, 0);
+  zj.accum = accum;
+  return c2r_yz(p, zj, ws[0], s);
 }
 
 // ---------------------------------------------------------- LPT kernels --
@@ -1763,17 +1743,8 @@ int pmx_fft_c2r(const pmx_plan* plan, float* spec, float* out, float scale,
   xj.do_fwd = 0;
   xj.do_inv = 1;
   PMX_TRY(launch_xpass(p, xj, S(stream)));
-  YJobs yj{};
-  yj.n = 1;
-  yj.j[0].in = w;
-  yj.j[0].nout = 1;
-  yj.j[0].out[0] = w;
-  yj.j[0].scale[0] = 1.0f;
-  PMX_TRY(launch_ypass(p, yj, 1, S(stream)));
-  ZJobs zj{};
-  zj.n = 1;
-  zj.j[0] = zc2r(w, out, scale, 0);
-  return launch_zpass_c2r(p, zj, S(stream));
+  ZJob zj = zc2r(w, out, scale, 0);
+  return c2r_yz(p, zj, w, S(stream));
 }
 
 int pmx_spec_to_full(const pmx_plan* plan, const float* spec, float* full,

@@ -203,6 +203,11 @@ struct XJob {
 };
 
 // Host launchers (fft.hip).  All take the caller's stream.
+// z and y passes of square planes up to kPlaneN in one launch
+constexpr int kPlaneN = 64;
+bool plane_ok(const Plan& p);
+int launch_plane(const Plan& p, const ZJobs* r2c, const ZJob* c2r,
+                 hipStream_t s);
 int launch_zpass_r2c(const Plan& p, const ZJobs& jobs, hipStream_t s);
 int launch_zpass_c2r(const Plan& p, const ZJobs& jobs, hipStream_t s);
 int launch_ypass(const Plan& p, const YJobs& jobs, int inverse, hipStream_t s);
