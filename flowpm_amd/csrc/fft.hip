@@ -740,9 +740,12 @@ __global__ __launch_bounds__(T) void k_xpass(XJob J, PlanDev p) {
 // same order as the two passes, and the same results.  Small passes are bound
 // by their launch and its chain of loads, stages and stores, so one of them is
 // nearly saved: forward + inverse, four passes -> two planes, 32^3 15.2 -> 9.1
-// us, 64^3 18.9 -> 10.8, 16 x 64^3 39.2 -> 22.4 (half the traffic).  With 256
-// threads 9.6, 12.6 and 23.9, with 128 10.5, 16.8 and 25.1.  The limit is a
-// plane's two tiles, 34 KB at 64, for four workgroups per CU.
+// us, 64^3 18.9 -> 10.8, 16 x 64^3 39.2 -> 22.4 (half the traffic; with 256
+// threads 9.6, 12.6 and 23.9, with 128 10.5, 16.8 and 25.1).  Above 64 with
+// 1024 threads, as fewer workgroups share a CU: 80^3 22.1 -> 13.0, 96^3 30.1
+// -> 17.0, 128^3 36.1 -> 21.8, 256 x 128^2 50.4 -> 24.7, 4 x 128^3 56.8 ->
+// 47.0, 8 x 100^3 69.6 -> 63.2.  The limit: a plane's two tiles are 134 KB of
+// the CU's 160 KB at 128.
 template <int N, int T>
 __global__ __launch_bounds__(T) void k_plane_r2c(ZJobs jobs, PlanDev p) {
   constexpr int H = N / 2, TZ = N / 2, TY = H + 1;
@@ -1073,7 +1076,7 @@ int launch_xpass(const Plan& p, const XJob& job, hipStream_t s) {
 template <int N>
 static int plane_n(const Plan& pl, const ZJobs* r2c, const ZJob* c2r,
                    hipStream_t s) {
-  constexpr int T = 512;
+  constexpr int T = N > 64 ? 1024 : 512;
   const PlanDev& p = pl.d;
   if (r2c) {
     ProfScope prof_(kProfZr2c, s);

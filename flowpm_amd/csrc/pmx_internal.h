@@ -204,7 +204,7 @@ struct XJob {
 
 // Host launchers (fft.hip).  All take the caller's stream.
 // z and y passes of square planes up to kPlaneN in one launch
-constexpr int kPlaneN = 64;
+constexpr int kPlaneN = 128;
 bool plane_ok(const Plan& p);
 int launch_plane(const Plan& p, const ZJobs* r2c, const ZJob* c2r,
                  hipStream_t s);

@@ -1,5 +1,5 @@
 """Transforms whose z and y passes run as one launch (square y-z planes of up
-to 64 x 64) against torch's float64 transform, on both sides of the limit and
+to 128 x 128) against torch's float64 transform, on both sides of the limit and
 for sides of every radix.
 
 An axis takes at most 4 stages of some 5 roundings each, three axes 60: in
@@ -13,7 +13,8 @@ import flowpm_amd as fa
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [8, 12, 16, 20, 24, 32, 40, 48, 60, 64, 80])
+@pytest.mark.parametrize("n", [8, 12, 16, 20, 24, 32, 40, 48, 60, 64, 80, 96, 100,
+                               120, 128, 160])
 @pytest.mark.parametrize("nx,batch", [(8, 1), (20, 3)])
 def test_square_planes(gpu, n, nx, batch):
   gen = torch.Generator().manual_seed(n)
