@@ -850,56 +850,56 @@ __global__ __launch_bounds__(T) void k_plane_c2r(ZJob J, PlanDev p) {
 
 // -------------------------------------------- full <-> half spectrum -----
 // full[b][x][y][z] (the reference's complex64 layout) from the half spectrum.
-__global__ void k_spec_to_full(const float2* __restrict__ spec,
-                               float2* __restrict__ full, PlanDev p) {
-  const long long M = (long long)p.nx * p.ny * p.nz;
-  const long long tot = (long long)p.B * M;
-  for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < tot;
-       e += (long long)gridDim.x * blockDim.x) {
-    const int z = (int)(e % p.nz);
-    const long long r = e / p.nz;
-    const int y = (int)(r % p.ny);
-    const long long r2 = r / p.ny;
-    const int x = (int)(r2 % p.nx);
-    const int b = (int)(r2 / p.nx);
-    int xs = x, ys = y, zs = z;
-    bool cj = false;
-    if (z > p.H) {
-      xs = (p.nx - x) % p.nx;
-      ys = (p.ny - y) % p.ny;
-      zs = p.nz - z;
-      cj = true;
+// One wave per row, so that the row's indices and its mirror's are scalar (and
+// need no division per element): 200 x 240 x 160 30.0 -> 20.0 us (92 MB).
+struct RowPair {
+  long long row, mir;  // (b, x, y) and (b, -x, -y)
+};
+__device__ __forceinline__ RowPair row_pair(const PlanDev& p, long long row) {
+  const unsigned u = (unsigned)row;  // rows < 2^31
+  const unsigned y = u % p.ny, bx = u / p.ny, x = bx % p.nx, b0 = bx - x;
+  const unsigned xm = x ? p.nx - x : 0, ym = y ? p.ny - y : 0;
+  return {row, (long long)(b0 + xm) * p.ny + ym};
+}
+__global__ __launch_bounds__(256) void k_spec_to_full(
+    const float2* __restrict__ spec, float2* __restrict__ full, PlanDev p) {
+  const int ln = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (long long row = 4LL * blockIdx.x + wv; row < p.rows;
+       row += 4LL * gridDim.x) {
+    const RowPair q = row_pair(p, row);
+    const float2* const s = spec + q.row * p.H;
+    const float2* const m = spec + q.mir * p.H;
+    float2* const out = full + q.row * p.nz;
+#pragma unroll 4
+    for (int z = ln; z < p.nz; z += 64) {
+      const float2* const e =
+          z < p.H ? s + z : (z == p.H ? spec + p.nyq0 + q.row : m + p.nz - z);
+      float2 v = *e;
+      if (z > p.H) v.y = -v.y;
+      out[z] = v;
     }
-    const long long row = ((long long)b * p.nx + xs) * p.ny + ys;
-    float2 v = (zs == p.H) ? spec[p.nyq0 + row] : spec[row * p.H + zs];
-    if (cj) v.y = -v.y;
-    full[e] = v;
   }
 }
 
 // Hermitian projection of an arbitrary full spectrum, kept on the half grid:
 // real(ifft(c)) == C2R((c(k) + conj(c(-k)))/2).
-__global__ void k_full_to_spec(const float2* __restrict__ full,
-                               float2* __restrict__ spec, PlanDev p) {
-  const long long tot = (long long)p.rows * (p.H + 1);
-  for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < tot;
-       e += (long long)gridDim.x * blockDim.x) {
-    const int kz = (int)(e % (p.H + 1));
-    const long long row = e / (p.H + 1);
-    const int y = (int)(row % p.ny);
-    const long long r2 = row / p.ny;
-    const int x = (int)(r2 % p.nx);
-    const int b = (int)(r2 / p.nx);
-    const int xm = (p.nx - x) % p.nx, ym = (p.ny - y) % p.ny,
-              zm = (p.nz - kz) % p.nz;
-    const long long M = (long long)p.nx * p.ny * p.nz;
-    const float2 u = full[b * M + ((long long)x * p.ny + y) * p.nz + kz];
-    const float2 v = full[b * M + ((long long)xm * p.ny + ym) * p.nz + zm];
-    const float2 hv = make_float2(0.5f * (u.x + v.x), 0.5f * (u.y - v.y));
-    if (kz == p.H)
-      spec[p.nyq0 + row] = hv;
-    else
-      spec[row * p.H + kz] = hv;
+// (rows as above: 24.4 -> 18.2 us)
+__global__ __launch_bounds__(256) void k_full_to_spec(
+    const float2* __restrict__ full, float2* __restrict__ spec, PlanDev p) {
+  const int ln = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (long long row = 4LL * blockIdx.x + wv; row < p.rows;
+       row += 4LL * gridDim.x) {
+    const RowPair q = row_pair(p, row);
+    const float2* const s = full + q.row * p.nz;
+    const float2* const m = full + q.mir * p.nz;
+#pragma unroll 4
+    for (int kz = ln; kz <= p.H; kz += 64) {
+      const float2 u = s[kz], v = m[kz ? p.nz - kz : 0];
+      const float2 hv = make_float2(0.5f * (u.x + v.x), 0.5f * (u.y - v.y));
+      *(kz == p.H ? spec + p.nyq0 + q.row : spec + q.row * p.H + kz) = hv;
+    }
   }
 }
 
@@ -1110,16 +1110,20 @@ int launch_plane(const Plan& p, const ZJobs* r2c, const ZJob* c2r,
   return kUnsupported;
 }
 
+// a wave per row, a second one from 32768 rows on
+static unsigned row_grid(const Plan& p) {
+  return (unsigned)std::min<long long>((p.d.rows + 3) / 4, 8192);
+}
 int launch_spec_to_full(const Plan& p, const float2* spec, float2* full,
                         hipStream_t s) {
-  hipLaunchKernelGGL(k_spec_to_full, dim3(2048), dim3(256), 0, s, spec, full,
+  hipLaunchKernelGGL(k_spec_to_full, dim3(row_grid(p)), dim3(256), 0, s, spec, full,
                      p.d);
   PMX_LAUNCH_CHECK();
   return kOk;
 }
 int launch_full_to_spec(const Plan& p, const float2* full, float2* spec,
                         hipStream_t s) {
-  hipLaunchKernelGGL(k_full_to_spec, dim3(2048), dim3(256), 0, s, full, spec,
+  hipLaunchKernelGGL(k_full_to_spec, dim3(row_grid(p)), dim3(256), 0, s, full, spec,
                      p.d);
   PMX_LAUNCH_CHECK();
   return kOk;
