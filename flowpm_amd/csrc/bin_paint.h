@@ -33,8 +33,10 @@ constexpr int kBinTail = 512;    // workgroups for the rest
 // scatter 0.39 ns per particle.  Uniform ones, scatter / tiles in us: 32^3
 // 42599 19.1 / 20.2; 64^3 16385 8.9 / 13.0, 45511 20.0 / 14.0; 120^3 34561
 // 16.1 / 18.5, 108001 45 / 19, 1.3 per cell 863 / 114; 192^3 70779 31.7 / 38.2,
-// 141557 58 / 39; 250^3 156251 64 / 74, 312501 122 / 78.
-constexpr long long kBinMin = 19 * 2048, kBinSparse = 80;
+// 141557 58 / 39; 250^3 156251 64 / 74, 312501 122 / 78.  The line lies where
+// some 10 us are gained, as two launches more take the host as long (63975
+// particles on 5 x 48 x 48 x 24: 126 us a call by tiles, 122 by the scatter).
+constexpr long long kBinMin = 32 * 2048, kBinSparse = 80;
 
 struct BinArgs {
   float* mesh;

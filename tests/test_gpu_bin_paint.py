@@ -47,10 +47,10 @@ def _check(out, pos, w, n):
 # sides below, at and above a tile's, one-cell sides, ragged ones; a chunk of
 # 2048 particles less one, one more; more chunks than a tile's workgroup has
 # threads (256); more than one member
-CASES = [("uniform", (5, 7, 9), 1, 40000), ("uniform", (1, 40, 3), 2, 36863),
-         ("uniform", (8, 16, 16), 1, 40961), ("uniform", (9, 17, 33), 3, 18433),
-         ("uniform", (64, 50, 70), 1, 530000), ("far", (24, 33, 18), 2, 30000),
-         ("cell", (12, 20, 40), 1, 50000), ("grid", (64, 40, 48), 2, 122880),
+CASES = [("uniform", (5, 7, 9), 1, 70000), ("uniform", (1, 40, 3), 2, 36863),
+         ("uniform", (8, 16, 16), 1, 69633), ("uniform", (9, 17, 33), 3, 24577),
+         ("uniform", (64, 50, 70), 1, 530000), ("far", (24, 33, 18), 2, 36000),
+         ("cell", (12, 20, 40), 1, 70000), ("grid", (64, 40, 48), 2, 122880),
          ("uniform", (16, 16, 16), 1, 3), ("uniform", (30, 30, 30), 1, 2049)]
 
 
@@ -80,7 +80,7 @@ def test_paint_in_any_order(gpu, kind, n, batch, npart):
 def test_weights_without_a_value(gpu):
   """inf and nan weights reach their own corner cells only, and particles
   without a position none."""
-  n, npart = (20, 24, 28), 50000
+  n, npart = (20, 24, 28), 70000
   gen = torch.Generator().manual_seed(9)
   pos = torch.rand(1, npart, 3, generator=gen) * torch.tensor(n)
   pos[0, :2] = torch.tensor([[3.5, 15.5, 15.5], [7.5, 2.5, 27.5]])
