@@ -24,7 +24,8 @@ Reports (one JSON line):
                            automatic policy with the gradient w.r.t.
                            Omega_c as well;
                            fwd_adjoint_compact_tape_ms_per_step: the
-                           compact tape (positions and potentials)
+                           compact tape (positions and potentials, also the
+                           automatic policy's)
   roofline                 dominant kernel: algorithmic bytes per launch /
                            average launch time from HIP events recorded on
                            the launch stream during a forward run
@@ -64,10 +65,9 @@ def algorithmic_bytes(kind, n, N):
       "fft_x_fused": 2 * S8,
       "fft_y_inv": 2 * S8,
       "fft_z_c2r": S8 + 4 * M,
-      # potential in, the three force meshes out
-      "grad": 4 * M + 3 * 4 * M,
-      # X, P read and written; F stays in registers inside fused steps
-      "readout_kick_drift": 3 * 4 * M + 24 * N + 24 * N,
+      # potential in, X, P read and written; the gradient is formed in LDS and
+      # F stays in registers inside fused steps
+      "readout_kick_drift": 4 * M + 24 * N + 24 * N,
   }
   return table.get(kind)
 
@@ -327,12 +327,12 @@ def main():
 # kinds, for the kernels the forward step launches
 # ({ty} / {tx}: the column-tile widths of the y / x passes the run used)
 _KIND_KERNEL = {
-    "readout_kick_drift": r"k_readout_kick_drift<", "paint": r"k_brick_deposit<1>",
+    "readout_kick_drift": r"k_readout_box<", "paint": r"k_brick_deposit<1>",
     "paint_gather": r"k_brick_gather<1, ", "fft_z_r2c": r"k_zpass_r2c<",
     "fft_y_fwd": r"k_ypass<\d+, {ty}, \d+, -1, false>",
     "fft_x_fused": r"k_xpass<\d+, {tx}, \d+, false>",
     "fft_y_inv": r"k_ypass<\d+, {ty}, \d+, 1, false>",
-    "fft_z_c2r": r"k_zpass_c2r<\d+, 16, ", "grad": r"k_grad_mesh<3>", "fill": r"k_fill",
+    "fft_z_c2r": r"k_zpass_c2r<\d+, 16, ", "fill": r"k_fill",
 }
 TRAFFIC_TABLE = os.path.join(ROOT, "profiles", "pm_step_256_hbm_traffic.md")
 

@@ -509,8 +509,7 @@ int pmx_nbody_adjoint_taped(const pmx_plan* plan, float* tape, int nsteps,
  * keeping X and the potential of every force evaluation instead of its
  * float4 force mesh (pmx_nbody_compact_tape_floats(plan, N, nsteps) =
  * (nsteps + 1)(3 B N + B nx ny nz) floats, about half of
- * pmx_nbody_tape_floats); the forward uses the packed meshes of an untaped
- * run, and pmx_nbody_adjoint_compact_taped forms each step's force mesh from
+ * pmx_nbody_tape_floats); the forward runs as an untaped one, and pmx_nbody_adjoint_compact_taped forms each step's force mesh from
  * its potential with the gradient stencil before the step's VJP: the same
  * gradients as pmx_nbody_adjoint_taped, bit for bit.  work and gcoef as for
  * pmx_nbody_adjoint_taped. */
