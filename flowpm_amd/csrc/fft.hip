@@ -737,7 +737,8 @@ __global__ __launch_bounds__(T) void k_xpass(XJob J, PlanDev p) {
 // ---------------------------------------------------------- planes ------
 // The z and y passes of a whole y-z plane (square, sides up to kPlaneN) in one
 // launch: the plane stays in LDS between them.  The same operations in the
-// same order as the two passes, and the same results.  Small passes are bound
+// same order as the two passes: the same results bit for bit up to 64, and to
+// the last bits above (other products fused with their sums).  Small passes are bound
 // by their launch and its chain of loads, stages and stores, so one of them is
 // nearly saved: forward + inverse, four passes -> two planes, 32^3 15.2 -> 9.1
 // us, 64^3 18.9 -> 10.8, 16 x 64^3 39.2 -> 22.4 (half the traffic; with 256
