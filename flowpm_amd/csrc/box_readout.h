@@ -111,6 +111,7 @@ static __device__ __forceinline__ void sto(float v, float* base, unsigned off,
 }
 
 constexpr int kBoxT = 512;  // 4 particles per thread, one after the other
+static_assert(kWalkRounds * kBoxT == 2048, "bricks hold up to 2048 particles");
 // LDS window, floats: two workgroups per CU.  A box longer than it is taken in
 // x windows that overlap by 5 planes: with 13568 floats and three workgroups
 // (80 VGPRs) the late boxes take two, 287 us against 262 at 256^3.
@@ -255,31 +256,20 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
   int q0[3], cnt[3];
   brick_block(g, bid, q0, cnt);
   // z fastest, then x: the 4 rows of a wave are a plane apart in LDS
-  const int cx = cnt[0], cz = cnt[2], nloc = cx * cnt[1] * cz;
+  const BrickWalk wk = brick_walk(g, cnt, kBoxT);
+  const int nloc = wk.nloc;
   // the brick's first particle (uniform); particle t of the brick is poff(t)
   // bytes from there
   const long long o0 =
       3 * ((long long)b * d.N +
            ((long long)q0[0] * g.gy + q0[1]) * g.gz + q0[2]);
-  const float rz = 1.0f / (float)cz, rx = 1.0f / (float)cx;
-  auto poff = [&](int t) {
-    const int tt = t < nloc ? t : 0;
-    // exact divisions: tt < 2048, and (tt + 1/2) / c is 1 / 2c off a whole
-    // number
-    const int q = (int)(((float)tt + 0.5f) * rz), lz = tt - q * cz,
-              ly = (int)(((float)q + 0.5f) * rx), lx = q - ly * cx;
-    return 12u * (unsigned)((lx * g.gy + ly) * g.gz + lz);
-  };
-  // whole y planes of the brick per round of kBoxT particles: the next
-  // particle is a constant away (no division per particle)
-  const bool even = nloc % kBoxT == 0 && kBoxT % (cx * cz) == 0;
-  const unsigned pstep = even ? 12u * (unsigned)(kBoxT / (cx * cz)) * g.gz : 0u;
+  auto poff = [&](int t) { return 12u * walk_at(wk, t); };
   const bool kick = c.do_k2 || c.do_k1d;
   const bool useP = kick || (!PLAIN && c.copy_xp);
   const float* const Xl = (c.xin ? c.xin : X) + o0;
   const float* const Pl = (c.pin ? c.pin : P) + o0;
-  const unsigned o_first = poff(tid + ua * kBoxT);
-  unsigned on = o_first;
+  const unsigned t_first = walk_at(wk, tid + ua * kBoxT);
+  unsigned tn = t_first, on = 12u * tn;
   float xn[3], pn[3] = {0.f, 0.f, 0.f};
 #pragma unroll
   for (int e = 0; e < 3; ++e) xn[e] = ldo(Xl, on, e);
@@ -373,7 +363,8 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
         p[e] = pn[e];
       }
       // the next particle's loads (the first one's again for a next window)
-      on = u == ub - 1 ? o_first : (even ? on + pstep : poff(t + kBoxT));
+      tn = u == ub - 1 ? t_first : walk_next(wk, tn, t);
+      on = 12u * tn;
 #pragma unroll
       for (int e = 0; e < 3; ++e) xn[e] = ldo(Xl, on, e);
       if (useP) {
@@ -462,7 +453,7 @@ int launch_readout_box(float* X, float* P, float* F, const float* phi,
   const long long nb = (long long)g.nbricks * d.B;
   const int parts = nb <= 64 ? 4 : (nb <= 128 ? 2 : 1);
   hipLaunchKernelGGL(kern, dim3(g.nbricks, d.B, parts), dim3(kBoxT), 0, s, X,
-                     P, F, phi, meta, d, g, c, 4 / parts);
+                     P, F, phi, meta, d, g, c, kWalkRounds / parts);
   PMX_LAUNCH_CHECK();
   return kOk;
 }

@@ -88,6 +88,46 @@ PMX_HD void brick_block(const BrickGrid& g, int bid, int q0[3], int cnt[3]) {
   cnt[2] = imin(g.ez, g.gz - q0[2]);
 }
 
+// The order in which a workgroup of T threads reads a brick's particles (the
+// readout's): thread t takes the particles t, t + T, ..., numbered z fastest,
+// then x, then y.  Offsets are in particles from the brick's first; a number
+// past the end stands for the first particle, so that every load stays in the
+// brick.
+constexpr int kWalkRounds = 4;  // of T particles: the most a brick has
+struct BrickWalk {
+  int cx, cz, nloc, gy, gz, T;
+  float rx, rz;
+  bool even;       // every round is full and has whole y planes of the brick:
+                   // the next particle is a constant away
+  unsigned pstep;
+};
+PMX_HD BrickWalk brick_walk(const BrickGrid& g, const int cnt[3], int T) {
+  BrickWalk w;
+  w.cx = cnt[0];
+  w.cz = cnt[2];
+  w.nloc = cnt[0] * cnt[1] * cnt[2];
+  w.gy = g.gy;
+  w.gz = g.gz;
+  w.T = T;
+  w.rz = 1.0f / (float)w.cz;
+  w.rx = 1.0f / (float)w.cx;
+  w.even = w.nloc == kWalkRounds * T && T % (w.cx * w.cz) == 0;
+  w.pstep = w.even ? (unsigned)(T / (w.cx * w.cz)) * g.gz : 0u;
+  return w;
+}
+PMX_HD unsigned walk_at(const BrickWalk& w, int t) {
+  const int tt = t < w.nloc ? t : 0;
+  // exact divisions: tt < 2048, and (tt + 1/2) / c is 1 / 2c off a whole
+  // number
+  const int q = (int)(((float)tt + 0.5f) * w.rz), lz = tt - q * w.cz,
+            ly = (int)(((float)q + 0.5f) * w.rx), lx = q - ly * w.cx;
+  return (unsigned)((lx * w.gy + ly) * w.gz + lz);
+}
+// the particle after number t, which is at o (in the last round: not asked)
+PMX_HD unsigned walk_next(const BrickWalk& w, unsigned o, int t) {
+  return w.even ? o + w.pstep : walk_at(w, t + w.T);
+}
+
 // The deposit box of a brick from the floor bounds lo..hi of its particles'
 // (scaled) positions: extent hi - lo + 2 per axis (the CIC corners), mode 1
 // (an LDS box) when every extent fits the mesh, the volume fits the budget
