@@ -14,7 +14,14 @@
 //   The fixed-point scale is a power of two chosen per brick and channel from
 //   the sum S of the channel's |weights| so no cell can overflow: the scale
 //   is 2^(30 - ex) with S = m 2^ex, m in [0.5, 1), so one deposit is rounded
-//   by at most half a unit, 2^(ex - 31) <= 2^-30 S.
+//   by at most half a unit, 2^(ex - 31) <= 2^-30 S.  That unit is coarse where
+//   a cell holds little of S: of boxes beyond 64 KB (which at first were added
+//   to the mesh as floats) the mesh would be off by 3.4e-6 rms of itself.
+//   Those are accumulated in doubles, as whole numbers of the unit 2^(ex - 52)
+//   (exact, so in any order): 3.4e-8.  Twice the passes, in a few bricks:
+//   force and gradient at 256^3, a = 1, 2157 -> 2166 us; where the few bricks
+//   are the last ones to end, 3-channel deposit at 128 x 160 x 96 22.7 -> 31.1
+//   (64-bit integers 36.6: a conversion takes some 12 instructions).
 //   Every brick has a 56 KB piece of the arena per channel; a larger box, up
 //   to 128 KB, goes to a pool of 8 KB per brick (where a box lies does not
 //   change what is in it).  Without the pool (64 KB pieces) the late boxes
@@ -292,12 +299,12 @@ __global__ __launch_bounds__(kDT, 8) void k_brick_deposit(BrickArgs a) {
     }
     return;
   }
-  constexpr int OX[8] = {0, 1, 0, 0, 1, 1, 0, 1};
-  constexpr int OY[8] = {0, 0, 1, 0, 1, 0, 1, 1};
-  constexpr int OZ[8] = {0, 0, 0, 1, 0, 1, 1, 1};
-  const int plane = e1 * e2, hx = kWinFloats / plane;  // planes per pass
-  const bool clip = hx < e0;
+  // planes per pass; a box beyond kBoxFloats is accumulated in doubles
+  const bool wide = vol4 > kBoxFloats;
+  const int plane = e1 * e2, hx = (wide ? kWinFloats / 2 : kWinFloats) / plane;
+  const bool clip = hx < e0;  // (always, if wide)
   float* dst = nullptr;
+  double* const box64 = reinterpret_cast<double*>(box);
   // deposits channel c of the particles; with CLIP those whose corners fall
   // in x planes [x0, x0 + nxw) of the box, else all
   auto deposit = [&](auto clip_, int c, int x0, int nxw) {
@@ -319,12 +326,22 @@ __global__ __launch_bounds__(kDT, 8) void k_brick_deposit(BrickArgs a) {
       const int at = (ix * e1 + ((int)fly - lo[1])) * e2 + ((int)flz - lo[2]);
       const float wq = wc[u][c] * fxs[c];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        if (CLIP && (unsigned)(ix + OX[k]) >= (unsigned)nxw) continue;
-        const float kw = ((OX[k] ? w1x : w0x) * (OY[k] ? w1y : w0y)) *
-                         (OZ[k] ? w1z : w0z);
-        atomicAdd(box + at + ((OX[k] * e1 + OY[k]) * e2 + OZ[k]),
-                  __float2int_rn(wq * kw));
+      for (int ox = 0; ox < 2; ++ox) {
+        if (CLIP && (unsigned)(ix + ox) >= (unsigned)nxw) continue;
+        const int to = at + ox * plane;
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          v[k] = wq * (((ox ? w1x : w0x) * (k & 2 ? w1y : w0y)) *
+                       (k & 1 ? w1z : w0z));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int o = to + (k >> 1) * e2 + (k & 1);
+          if (CLIP && wide)
+            atomicAdd(box64 + o, (double)rintf(v[k] * 0x1p22f));
+          else
+            atomicAdd(box + o, __float2int_rn(v[k]));
+        }
       }
     }
   };
@@ -334,7 +351,7 @@ __global__ __launch_bounds__(kDT, 8) void k_brick_deposit(BrickArgs a) {
       const int nxw = min(hx, e0 - x0), nw = nxw * plane;
       const bool first_pass = c == 0 && x0 == 0;
       if (!first_pass) __syncthreads();  // the window is reused
-      for (int i = tid; 4 * i < nw; i += kDT)
+      for (int i = tid; 4 * i < (wide ? 2 * nw : nw); i += kDT)
         reinterpret_cast<int4*>(box)[i] = make_int4(0, 0, 0, 0);
       __syncthreads();
       if (clip)
@@ -366,9 +383,16 @@ __global__ __launch_bounds__(kDT, 8) void k_brick_deposit(BrickArgs a) {
       const float fi = fxinv[c];
       float* const o = dst + c * vol4 + x0 * plane;
       for (int i = tid; 4 * i < nw; i += kDT) {
-        const int4 v = reinterpret_cast<const int4*>(box)[i];
-        const Vec4u r = {(float)v.x * fi, (float)v.y * fi, (float)v.z * fi,
-                         (float)v.w * fi};
+        Vec4u r;
+        if (wide) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            r[e] = (float)box64[4 * i + e] * 0x1p-22f * fi;
+        } else {
+          const int4 v = reinterpret_cast<const int4*>(box)[i];
+          r = Vec4u{(float)v.x * fi, (float)v.y * fi, (float)v.z * fi,
+                    (float)v.w * fi};
+        }
         if (4 * i + 4 <= nw) {
           *reinterpret_cast<Vec4u*>(o + 4 * i) = r;
         } else {
