@@ -23,7 +23,7 @@ struct BrickGrid {
   unsigned my, mz;    // div_magic of nby and nbz
 };
 
-constexpr int kBoxFloats = 16384;  // the arena's floats per brick (64 KB)
+constexpr int kBoxFloats = 16384;  // a brick's own piece of the arena (64 KB)
 constexpr int kTile = 16;          // gather tile side
 
 PMX_HD int imin(int a, int b) { return a < b ? a : b; }

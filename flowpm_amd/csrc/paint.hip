@@ -22,10 +22,10 @@
 //   force and gradient at 256^3, a = 1, 2157 -> 2166 us; where the few bricks
 //   are the last ones to end, 3-channel deposit at 128 x 160 x 96 22.7 -> 31.1
 //   (64-bit integers 36.6: a conversion takes some 12 instructions).
-//   Every brick has a 56 KB piece of the arena per channel; a larger box, up
+//   Every brick has a 64 KB piece of the arena per channel; a larger box, up
 //   to 128 KB, goes to a pool of 8 KB per brick (where a box lies does not
-//   change what is in it).  Without the pool (64 KB pieces) the late boxes
-//   beyond them spilled: at 256^3, a = 1, 100 us of float atomics per density
+//   change what is in it).  Without the pool the late boxes beyond their pieces
+//   spilled: at 256^3, a = 1, 100 us of float atomics per density
 //   paint and 231 per three-channel one.
 //   A brick whose box is larger still, or finds the pool full, falls back to
 //   device-scope float atomics into the finished mesh (k_brick_spill, after
@@ -68,12 +68,15 @@ struct BrickArgs {
 };
 
 constexpr int kNoBox = -1;
-// The arena: a piece of kSlot floats per brick and channel, and the rest of
-// kBoxFloats per brick and channel as a pool for the boxes beyond that, handed
-// out by a fill count.  (Every brick taking what it needs from the count would
-// pack the arena, but 8192 returning device-scope atomics on one line take
-// 400 us.)
-constexpr int kSlot = kBoxFloats - 2048;
+// The arena: a piece of kBoxFloats (and a little, so that the pieces do not all
+// start on the same memory channels: 256^3 with 1 cell rms of noise 220 -> 216
+// us) per brick and channel, and kPoolFloats of each as a pool for the boxes
+// beyond that, handed out by a fill count.  (Every brick taking what it needs
+// from the count would pack the arena, but 8192 returning device-scope atomics
+// on one line take 400 us.  With pieces of 56 KB and the pool cut out of them,
+// states whose boxes are mostly around 60 KB filled the pool and spilled: 256^3
+// with 1.8 cells rms of noise 1003 us, 327 here.)
+constexpr int kPieceFloats = kBoxFloats + 272, kPoolFloats = 2048;
 constexpr int kCtrPool = 0, kCtrR = 2, kCtrInts = 8;  // (the count: 64 bits)
 
 // Reductions along a wave by DPP moves (no LDS traffic): the result of the
@@ -130,7 +133,7 @@ constexpr int kDT = 512;
 constexpr int kWinFloats = 10112;
 constexpr int kDW = kDT / 64;
 constexpr int kPPT = 2048 / kDT;
-// largest box: the arena holds kBoxFloats per brick and channel on average
+// largest box
 constexpr long long kBoxMax = 2 * kBoxFloats;
 static_assert(kDW == 8, "the workgroup reductions take 8 waves");
 
@@ -285,8 +288,8 @@ __global__ __launch_bounds__(kDT, 8) void k_brick_deposit(BrickArgs a) {
   // where the box goes, in 16-float units; a piece of the pool is asked for
   // by thread 0, and its answer used after the first pass
   const long long nb = (long long)gridDim.x * gridDim.y;
-  constexpr int kPiece = C * kSlot / 16, kPool = C * kBoxFloats / 16 - kPiece;
-  const bool pooled = vol4 > kSlot;
+  constexpr int kPiece = C * kPieceFloats / 16, kPool = C * kPoolFloats / 16;
+  const bool pooled = vol4 > kBoxFloats;
   const int units = (C * vol4 + 15) / 16;
   unsigned long long got = 0;
   if (tid == 0 && box_ok && pooled)
@@ -299,8 +302,8 @@ __global__ __launch_bounds__(kDT, 8) void k_brick_deposit(BrickArgs a) {
     }
     return;
   }
-  // planes per pass; a box beyond kBoxFloats is accumulated in doubles
-  const bool wide = vol4 > kBoxFloats;
+  // planes per pass; a box of the pool is accumulated in doubles
+  const bool wide = pooled;
   const int plane = e1 * e2, hx = (wide ? kWinFloats / 2 : kWinFloats) / plane;
   const bool clip = hx < e0;  // (always, if wide)
   float* dst = nullptr;
@@ -748,9 +751,13 @@ bool brick_paint_ok(const MeshDims& d, const BrickGrid& g) {
          g.nby <= 1024 && g.nbz <= 1024;
 }
 
+static long long arena_floats(const MeshDims& d, const BrickGrid& g, int C) {
+  return (long long)d.B * g.nbricks * C * (kPieceFloats + kPoolFloats);
+}
+
 long long brick_work_floats(const MeshDims& d, const BrickGrid& g, int C) {
-  // kBoxFloats per brick and channel; counters and alignment take the rest
-  const long long arena = (long long)d.B * g.nbricks * C * kBoxFloats;
+  // counters and alignment take the rest
+  const long long arena = arena_floats(d, g, C);
   const long long meta = 8LL * d.B * g.nbricks;
   return arena + meta + 16;
 }
@@ -767,8 +774,8 @@ static float* brick_arena(float* work) {
 }
 const int* brick_meta(const MeshDims& d, const BrickGrid& g, int C,
                       float* work) {
-  return reinterpret_cast<const int*>(
-      brick_arena(work) + (long long)d.B * g.nbricks * C * kBoxFloats);
+  return reinterpret_cast<const int*>(brick_arena(work) +
+                                      arena_floats(d, g, C));
 }
 
 int launch_brick_paint(float* const* mesh, int C, const float* X,
