@@ -1093,8 +1093,17 @@ static int plane_n(const Plan& pl, const ZJobs* r2c, const ZJob* c2r,
   }
   return kOk;
 }
-bool plane_ok(const Plan& p) {
-  return p.d.ny == p.d.nz && p.d.nz <= kPlaneN;
+// A small plane keeps few of its workgroup's 512 threads busy, and four
+// workgroups share a CU: from some thousands of planes on the two passes, whose
+// tiles are full, are the faster ones.  Forward + inverse transform, passes /
+// planes in us: 8^2 2048 planes 20.4 / 18.1, 4096 25.6 / 26.7; 16^2 26.3 / 24.8,
+// 36.4 / 39.2; 24^2 31.1 / 28.4, 45.8 / 46.6; 32^2 4096 65.6 / 62.6; 40^2 planes
+// at any number.  r2c3d + c2r3d: 8^2 250000 planes 740 / 1542, 32^2 15616 247 /
+// 286.
+bool plane_ok(const Plan& p, int jobs) {
+  const long long planes = (long long)p.d.B * p.d.nx * jobs;
+  return p.d.ny == p.d.nz && p.d.nz <= kPlaneN &&
+         (p.d.nz > 32 || planes <= (p.d.nz < 32 ? 2048 : 4096));
 }
 int launch_plane(const Plan& p, const ZJobs* r2c, const ZJob* c2r,
                  hipStream_t s) {

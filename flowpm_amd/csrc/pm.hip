@@ -168,7 +168,7 @@ static int r2c_zy(const Plan& p, const float* const* in, float2* const* spec,
     zj.j[i] = zr2c(in[i], spec[i], scale);
     yj.j[i] = yfwd(spec[i]);
   }
-  if (plane_ok(p)) return launch_plane(p, &zj, nullptr, s);
+  if (plane_ok(p, zj.n)) return launch_plane(p, &zj, nullptr, s);
   PMX_TRY(launch_zpass_r2c(p, zj, s));
   PMX_TRY(launch_ypass(p, yj, 0, s));
   return kOk;
@@ -177,7 +177,7 @@ static int r2c_zy(const Plan& p, const float* const* in, float2* const* spec,
 // Inverse y and z passes of one spectrum (in place) whose x pass is done, to
 // the real mesh of job j.
 static int c2r_yz(const Plan& p, const ZJob& j, float2* spec, hipStream_t s) {
-  if (plane_ok(p) && j.ez == 0 && !j.accum && j.ostride <= 1 && j.ocomp == 0)
+  if (plane_ok(p, 1) && j.ez == 0 && !j.accum && j.ostride <= 1 && j.ocomp == 0)
     return launch_plane(p, nullptr, &j, s);
   YJobs yj{};
   yj.n = 1;

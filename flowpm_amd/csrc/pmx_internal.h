@@ -203,9 +203,10 @@ struct XJob {
 };
 
 // Host launchers (fft.hip).  All take the caller's stream.
-// z and y passes of square planes up to kPlaneN in one launch
+// z and y passes of square planes up to kPlaneN in one launch (of small planes
+// up to a number of them, of all jobs together)
 constexpr int kPlaneN = 128;
-bool plane_ok(const Plan& p);
+bool plane_ok(const Plan& p, int jobs);
 int launch_plane(const Plan& p, const ZJobs* r2c, const ZJob* c2r,
                  hipStream_t s);
 int launch_zpass_r2c(const Plan& p, const ZJobs& jobs, hipStream_t s);
