@@ -851,8 +851,10 @@ __global__ __launch_bounds__(T) void k_plane_c2r(ZJob J, PlanDev p) {
 
 // -------------------------------------------- full <-> half spectrum -----
 // full[b][x][y][z] (the reference's complex64 layout) from the half spectrum.
-// One wave per row, so that the row's indices and its mirror's are scalar (and
-// need no division per element): 200 x 240 x 160 30.0 -> 20.0 us (92 MB).
+// L lanes per row: a wave, so that the row's indices and its mirror's are scalar
+// (and need no division per element), 200 x 240 x 160 30.0 -> 20.0 us (92 MB);
+// for rows of up to 32 elements the next power of two, as most of a wave would
+// have nothing to do.
 struct RowPair {
   long long row, mir;  // (b, x, y) and (b, -x, -y)
 };
@@ -862,18 +864,26 @@ __device__ __forceinline__ RowPair row_pair(const PlanDev& p, long long row) {
   const unsigned xm = x ? p.nx - x : 0, ym = y ? p.ny - y : 0;
   return {row, (long long)(b0 + xm) * p.ny + ym};
 }
+// the first row of a thread: with L = 64 the same for its wave
+template <int L>
+__device__ __forceinline__ long long first_row() {
+  constexpr int R = 256 / L;
+  const int r = threadIdx.x / L;
+  return (long long)R * blockIdx.x +
+         (L == 64 ? __builtin_amdgcn_readfirstlane(r) : r);
+}
+template <int L>
 __global__ __launch_bounds__(256) void k_spec_to_full(
     const float2* __restrict__ spec, float2* __restrict__ full, PlanDev p) {
-  const int ln = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (long long row = 4LL * blockIdx.x + wv; row < p.rows;
-       row += 4LL * gridDim.x) {
+  const int ln = threadIdx.x % L;
+  for (long long row = first_row<L>(); row < p.rows;
+       row += (256LL / L) * gridDim.x) {
     const RowPair q = row_pair(p, row);
     const float2* const s = spec + q.row * p.H;
     const float2* const m = spec + q.mir * p.H;
     float2* const out = full + q.row * p.nz;
 #pragma unroll 4
-    for (int z = ln; z < p.nz; z += 64) {
+    for (int z = ln; z < p.nz; z += L) {
       const float2* const e =
           z < p.H ? s + z : (z == p.H ? spec + p.nyq0 + q.row : m + p.nz - z);
       float2 v = *e;
@@ -886,17 +896,17 @@ __global__ __launch_bounds__(256) void k_spec_to_full(
 // Hermitian projection of an arbitrary full spectrum, kept on the half grid:
 // real(ifft(c)) == C2R((c(k) + conj(c(-k)))/2).
 // (rows as above: 24.4 -> 18.2 us)
+template <int L>
 __global__ __launch_bounds__(256) void k_full_to_spec(
     const float2* __restrict__ full, float2* __restrict__ spec, PlanDev p) {
-  const int ln = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (long long row = 4LL * blockIdx.x + wv; row < p.rows;
-       row += 4LL * gridDim.x) {
+  const int ln = threadIdx.x % L;
+  for (long long row = first_row<L>(); row < p.rows;
+       row += (256LL / L) * gridDim.x) {
     const RowPair q = row_pair(p, row);
     const float2* const s = full + q.row * p.nz;
     const float2* const m = full + q.mir * p.nz;
 #pragma unroll 4
-    for (int kz = ln; kz <= p.H; kz += 64) {
+    for (int kz = ln; kz <= p.H; kz += L) {
       const float2 u = s[kz], v = m[kz ? p.nz - kz : 0];
       const float2 hv = make_float2(0.5f * (u.x + v.x), 0.5f * (u.y - v.y));
       *(kz == p.H ? spec + p.nyq0 + q.row : spec + q.row * p.H + kz) = hv;
@@ -1120,21 +1130,31 @@ int launch_plane(const Plan& p, const ZJobs* r2c, const ZJob* c2r,
   return kUnsupported;
 }
 
-// a wave per row, a second one from 32768 rows on
-static unsigned row_grid(const Plan& p) {
-  return (unsigned)std::min<long long>((p.d.rows + 3) / 4, 8192);
+// a row per L lanes, a second one from 8192 workgroups on
+template <int L, class Kern>
+static void launch_rows(Kern kern, const float2* in, float2* out,
+                        const Plan& p, hipStream_t s) {
+  constexpr int R = 256 / L;
+  const unsigned grid =
+      (unsigned)std::min<long long>((p.d.rows + R - 1) / R, 8192);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, in, out, p.d);
 }
 int launch_spec_to_full(const Plan& p, const float2* spec, float2* full,
                         hipStream_t s) {
-  hipLaunchKernelGGL(k_spec_to_full, dim3(row_grid(p)), dim3(256), 0, s, spec, full,
-                     p.d);
+  if (p.d.nz <= 8) launch_rows<8>(k_spec_to_full<8>, spec, full, p, s);
+  else if (p.d.nz <= 16) launch_rows<16>(k_spec_to_full<16>, spec, full, p, s);
+  else if (p.d.nz <= 32) launch_rows<32>(k_spec_to_full<32>, spec, full, p, s);
+  else launch_rows<64>(k_spec_to_full<64>, spec, full, p, s);
   PMX_LAUNCH_CHECK();
   return kOk;
 }
 int launch_full_to_spec(const Plan& p, const float2* full, float2* spec,
                         hipStream_t s) {
-  hipLaunchKernelGGL(k_full_to_spec, dim3(row_grid(p)), dim3(256), 0, s, full, spec,
-                     p.d);
+  const int n = p.d.H + 1;
+  if (n <= 8) launch_rows<8>(k_full_to_spec<8>, full, spec, p, s);
+  else if (n <= 16) launch_rows<16>(k_full_to_spec<16>, full, spec, p, s);
+  else if (n <= 32) launch_rows<32>(k_full_to_spec<32>, full, spec, p, s);
+  else launch_rows<64>(k_full_to_spec<64>, full, spec, p, s);
   PMX_LAUNCH_CHECK();
   return kOk;
 }
