@@ -133,8 +133,15 @@ constexpr int kDT = 512;
 constexpr int kWinFloats = 10112;
 constexpr int kDW = kDT / 64;
 constexpr int kPPT = 2048 / kDT;
-// largest box
-constexpr long long kBoxMax = 2 * kBoxFloats;
+// The largest box of a brick of nloc particles.  Those of a finer force mesh
+// have 256 or fewer: added one by one they cost less than the many passes over
+// a large box take the workgroup, which ends last.  Force and gradient, boxes
+// up to 128 / 80 / 64 KB in us: 64 x 80 x 48, f = 2, a = 1 261.5 / 263.7 / 270;
+// grids with 2 spacings rms of noise, f = 2 32^3 191 / 172 / 168, 64^3 604 / 562
+// / 565, 64 x 80 x 48 604 / 594 / 565, f = 4 64^3 1322 / 1219 / 1212.
+PMX_HD long long box_max(int nloc) {
+  return nloc <= 512 ? 5 * kBoxFloats / 4 : 2 * kBoxFloats;
+}
 static_assert(kDW == 8, "the workgroup reductions take 8 waves");
 
 // four consecutive floats of a box row, at any dword
@@ -278,7 +285,7 @@ __global__ __launch_bounds__(kDT, 8) void k_brick_deposit(BrickArgs a) {
     fxinv[c] = __int_as_float((127 - es) << 23);
   }
   const int n[3] = {a.d.nx, a.d.ny, a.d.nz};
-  BrickBox bx = brick_box(lo, hi, n, q0, cnt, g.f, wfin, kBoxMax);
+  BrickBox bx = brick_box(lo, hi, n, q0, cnt, g.f, wfin, box_max(nloc));
   // (the window has to hold a plane of the deposits' two)
   if (bx.mode == 1 && 2LL * bx.ext[1] * bx.ext[2] > kWinFloats) bx.mode = 2;
   int* const m = a.meta + 8LL * ((long long)b * g.nbricks + bid);
