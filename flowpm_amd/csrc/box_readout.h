@@ -200,13 +200,18 @@ static __device__ __forceinline__ void fill_box(float* win, const float* pm,
 }
 
 // potential pairs of the cell whose lower corner is (ix, iy, iz), from the
-// mesh itself: the wrapped offsets of the 6 planes, rows and cells, taken once
+// mesh itself: the wrapped offsets of the 6 planes and rows and of the 3 pairs
+// of cells, taken once.  A pair is one 8-byte load; the few that wrap between
+// their cells take the second one by itself (two 4-byte loads each: 256^3 with 4
+// cells rms of noise 7970 us a force, so 7709; two members of 12 x 256 x 256
+// with 1 cell, a run of two steps, 1333 / 1212).
 struct MeshPair {
   const float* pm;
   unsigned ox[6], oy[6], oz[6];
+  unsigned last;  // the last cell of a row
   __device__ __forceinline__ MeshPair(const float* pm_, int ix, int iy, int iz,
                                       const MeshDims& d)
-      : pm(pm_) {
+      : pm(pm_), last(d.nz - 1) {
     axis(ox, ix, d.nx, (unsigned)d.ny * d.nz);
     axis(oy, iy, d.ny, (unsigned)d.nz);
     axis(oz, iz, d.nz, 1u);
@@ -214,7 +219,7 @@ struct MeshPair {
   static __device__ __forceinline__ void axis(unsigned (&o)[6], int i, int n,
                                               unsigned stride) {
     // sides are 8 or more: - 2 .. 3 wraps at most once
-    const int w = imod(i, n);
+    const int w = near_mod(i, n);
 #pragma unroll
     for (int e = 0; e < 6; ++e) {
       int v = w + e - 2;
@@ -223,10 +228,53 @@ struct MeshPair {
     }
   }
   __device__ __forceinline__ V2 operator()(int a, int b, int c) const {
-    const unsigned r = ox[a + 2] + oy[b + 2];
-    return V2{pm[r + oz[c + 2]], pm[r + oz[c + 3]]};
+    const float* const r = pm + (ox[a + 2] + oy[b + 2]);
+    const unsigned z = oz[c + 2];
+    V2 v = *reinterpret_cast<const V2u*>(r + min(z, last - 1));
+    if (z == last) v = V2{v.y, *r};
+    return v;
   }
 };
+// The same readout from the packed force mesh of the member: three values at each
+// corner, in the same order.
+static __device__ __forceinline__ void mesh_readout(const float* m, int ix,
+                                                    int iy, int iz, float x,
+                                                    float y, float z,
+                                                    const MeshDims& d,
+                                                    float (&out)[3]) {
+  constexpr int OX[8] = {0, 1, 0, 0, 1, 1, 0, 1};
+  constexpr int OY[8] = {0, 0, 1, 0, 1, 0, 1, 1};
+  constexpr int OZ[8] = {0, 0, 0, 1, 0, 1, 1, 1};
+  const int n[3] = {d.nx, d.ny, d.nz};
+  const int i[3] = {ix, iy, iz};
+  unsigned o[3][2];
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    const unsigned w = (unsigned)near_mod(i[e], n[e]);
+    o[e][0] = w;
+    o[e][1] = w + 1 == (unsigned)n[e] ? 0u : w + 1;
+  }
+  float v[8][3];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const float* const g =
+        m + 3LL * ((o[0][OX[q]] * (unsigned)d.ny + o[1][OY[q]]) *
+                       (unsigned)d.nz + o[2][OZ[q]]);
+#pragma unroll
+    for (int e = 0; e < 3; ++e) v[q][e] = g[e];
+  }
+  const float fx = floorf(x), fy = floorf(y), fz = floorf(z);
+  const float wx[2] = {1.0f - fabsf(x - fx), 1.0f - fabsf(x - (fx + 1.0f))};
+  const float wy[2] = {1.0f - fabsf(y - fy), 1.0f - fabsf(y - (fy + 1.0f))};
+  const float wz[2] = {1.0f - fabsf(z - fz), 1.0f - fabsf(z - (fz + 1.0f))};
+  out[0] = out[1] = out[2] = 0.0f;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const float k = (wx[OX[q]] * wy[OY[q]]) * wz[OZ[q]];
+#pragma unroll
+    for (int e = 0; e < 3; ++e) out[e] += v[q][e] * k;
+  }
+}
 // and from a window whose cell (ix - 2, iy - 2, iz - 2) is w
 struct WinPair {
   const float* w;
@@ -244,8 +292,8 @@ struct WinPair {
 template <bool META, bool PLAIN>
 __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
     float* X, float* P, float* F, const float* __restrict__ phi,
-    const int* __restrict__ meta, MeshDims d, BrickGrid g, KickDrift c,
-    int rounds_each) {
+    const int* __restrict__ meta, BoxlessMesh b3, MeshDims d, BrickGrid g,
+    KickDrift c, int rounds_each) {
   __shared__ float win[kBoxWin];
   __shared__ int red[META ? 1 : kBoxT / 64][6];
   const int tid = threadIdx.x;
@@ -338,6 +386,10 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
   const float* const pm =
       phi + (long long)b * ((long long)d.nx * d.ny * d.nz);
   const long long tot = (long long)d.B * d.N;
+  const float* const m3 =
+      hx < 6 && b3.mesh && *b3.count >= b3.need
+          ? b3.mesh + 3LL * b * ((long long)d.nx * d.ny * d.nz)
+          : nullptr;
   // without a box every particle reads the mesh, in one round
   const int rounds = hx >= 6 ? q.px - 5 : 1, step = hx >= 6 ? hx - 5 : 1;
   unsigned done = 0;
@@ -383,6 +435,8 @@ __global__ __launch_bounds__(kBoxT, 4) void k_readout_box(
                                    (iz - 2 - q.z0),
                                q.plane, q.pz},
                        x[0], x[1], x[2], r);
+        } else if (m3) {
+          mesh_readout(m3, ix, iy, iz, x[0], x[1], x[2], d, r);
         } else {
           grad_readout(MeshPair(pm, ix, iy, iz, d), x[0], x[1], x[2], r);
         }
@@ -435,8 +489,8 @@ bool readout_box_ok(const MeshDims& d, const KickDrift& c, const float* X,
 }
 
 int launch_readout_box(float* X, float* P, float* F, const float* phi,
-                       const int* meta, const MeshDims& d, const KickDrift& c,
-                       hipStream_t s) {
+                       const int* meta, const BoxlessMesh& b3,
+                       const MeshDims& d, const KickDrift& c, hipStream_t s) {
   if ((long long)d.B * d.N == 0) return kOk;
   PMX_REQUIRE(readout_box_ok(d, c, X, P, F, phi),
               "readout_box: one particle per cell, 16-byte aligned arrays");
@@ -453,7 +507,7 @@ int launch_readout_box(float* X, float* P, float* F, const float* phi,
   const long long nb = (long long)g.nbricks * d.B;
   const int parts = nb <= 64 ? 4 : (nb <= 128 ? 2 : 1);
   hipLaunchKernelGGL(kern, dim3(g.nbricks, d.B, parts), dim3(kBoxT), 0, s, X,
-                     P, F, phi, meta, d, g, c, kWalkRounds / parts);
+                     P, F, phi, meta, b3, d, g, c, kWalkRounds / parts);
   PMX_LAUNCH_CHECK();
   return kOk;
 }

@@ -57,7 +57,9 @@ struct BrickArgs {
                          // box reaches past the brick), where its box lies in
                          // the arena (16-float units; kNoBox: it spills)
   int* ctr;              // [kCtrPool] the pool's fill count, [kCtrR] the
-                         // largest R; zero before and after every paint
+                         // largest R; zero before and after every paint.
+                         // [kCtrBoxless] bricks without a box, left for the
+                         // readout until the next paint's gather clears it
   const float* X;        // positions [B][N][3]
   const float* w;        // weights [B][N][wstride] or null
   int wstride;
@@ -77,7 +79,8 @@ constexpr int kNoBox = -1;
 // states whose boxes are mostly around 60 KB filled the pool and spilled: 256^3
 // with 1.8 cells rms of noise 1003 us, 327 here.)
 constexpr int kPieceFloats = kBoxFloats + 272, kPoolFloats = 2048;
-constexpr int kCtrPool = 0, kCtrR = 2, kCtrInts = 8;  // (the count: 64 bits)
+constexpr int kCtrPool = 0, kCtrR = 2, kCtrInts = 8;  // (the fill: 64 bits)
+constexpr int kCtrBoxless = 4;
 
 // Reductions along a wave by DPP moves (no LDS traffic): the result of the
 // first 8 << k lanes of a row ends up in the last of them; wave_* in lane 63.
@@ -472,6 +475,7 @@ __global__ __launch_bounds__(256) void k_brick_gather(BrickArgs a) {
   const int b = blockIdx.y;
   const int ntx = (d.nx + TX - 1) / TX, nty = (d.ny + kTile - 1) / kTile,
             ntz = (d.nz + kTile - 1) / kTile;
+  if (blockIdx.x == 0 && b == 0 && tid == 0) a.ctr[kCtrBoxless] = 0;
   const int tt = (int)xcd_block(blockIdx.x, gridDim.x);
   const int tz = tt % ntz, ty = (tt / ntz) % nty, tx = tt / (ntz * nty);
   const int t0x = tx * TX, t0y = ty * kTile, t0z = tz * kTile;
@@ -732,15 +736,18 @@ __device__ __forceinline__ void spill_brick(const BrickArgs& a, long long q) {
 // spread over more than the mesh; non-finite weights) are added to the
 // gathered mesh with device-scope float atomics, one thread per particle.
 // Every workgroup looks through the flags of its own bricks at once; without
-// a marked one it returns after that load.  The counters are left zero.
+// a marked one it returns after that load.  The pool's and R's counters are
+// left zero.
 template <int C>
 __global__ __launch_bounds__(256) void k_brick_spill(BrickArgs a) {
-  if (blockIdx.x == 0 && threadIdx.x < kCtrInts) a.ctr[threadIdx.x] = 0;
+  if (blockIdx.x == 0 && threadIdx.x < kCtrBoxless) a.ctr[threadIdx.x] = 0;
   const long long nq = (long long)a.d.B * a.g.nbricks;
   for (long long k0 = blockIdx.x; k0 < nq; k0 += 256LL * gridDim.x) {
     const long long mine = k0 + (long long)threadIdx.x * gridDim.x;
     const bool hit = mine < nq && a.meta[8 * mine + 7] == kNoBox;
-    if (!__syncthreads_or(hit)) continue;
+    const int n = __syncthreads_count(hit);
+    if (n == 0) continue;
+    if (threadIdx.x == 0) atomicAdd(a.ctr + kCtrBoxless, n);
     for (int w = 0; w < 256; ++w) {
       const long long q = k0 + (long long)w * gridDim.x;
       if (q >= nq) break;
@@ -784,6 +791,8 @@ const int* brick_meta(const MeshDims& d, const BrickGrid& g, int C,
   return reinterpret_cast<const int*>(brick_arena(work) +
                                       arena_floats(d, g, C));
 }
+
+const int* brick_boxless(float* work) { return brick_ctr(work) + kCtrBoxless; }
 
 int launch_brick_paint(float* const* mesh, int C, const float* X,
                        const float* w, int wstride, float wscale, float ps,

@@ -722,6 +722,16 @@ static bool box_run(const Plan& p, long long N, float f) {
          N == (long long)p.d.nx * p.d.ny * p.d.nz;
 }
 
+// A particle without a box reads 20 rows of the potential, of a force mesh 4.
+// Where bricks without one (particles in no order, or scattered by many cells)
+// are an eighth or more, the force mesh is formed for them.  Potential / force
+// mesh, one force evaluation in us: 256^3 in no order 14446 / 8738, with 10 and
+// 4 cells rms of noise 9645 / 7966, 7969 / 7347.  The launch that looks at the
+// count costs every force 2.2 us (256^3 571 -> 572), so members below 2^22
+// cells go without (128^3 94 -> 96 us; in no order 1364 / 1062, with 4 cells
+// 985 / 892; 64^3 nothing to gain).
+constexpr long long kBoxlessCells = 1 << 22, kBoxlessShare = 8 * 2048;
+
 // pgd (optional): (alpha, kl, ks) of every step; after the drift of step
 // i the positions move by the PGD displacement (tfpm.py:487-488).
 // src (optional, not with pgd, at least one step or the jump-start force):
@@ -826,7 +836,14 @@ static int nbody_run(const Plan& p, float* state, long long N, float f,
               ? nullptr
               : brick_meta(md, make_brick_grid(md.nx, md.ny, md.nz, 1), 1,
                            nw.brick);
-      return launch_readout_box(Xf, P, F, phi, meta, md, kd, s);
+      BoxlessMesh b3{};
+      if (meta && N >= kBoxlessCells) {
+        b3.mesh = nw.f4;
+        b3.count = brick_boxless(nw.brick);
+        b3.need = (int)((long long)md.B * md.N / kBoxlessShare);
+        PMX_TRY(launch_grad_mesh_if(p, phi, nw.f4, b3.count, b3.need, s));
+      }
+      return launch_readout_box(Xf, P, F, phi, meta, b3, md, kd, s);
     }
     const int nc = fkeep ? 4 : 3;
     PMX_TRY(force_k(k, Xforce, nw, nc));

@@ -233,6 +233,9 @@ bool grad_stencil_ok(const Plan& p);
 // (w4, with nc = 4: a mesh for the fourth component instead of 0)
 int launch_grad_mesh(const Plan& p, const float* phi, float* fm, int nc,
                      hipStream_t s, const float* w4 = nullptr);
+// the packed mesh, if *count (on the device) is at least need
+int launch_grad_mesh_if(const Plan& p, const float* phi, float* fm,
+                        const int* count, int need, hipStream_t s);
 int launch_grad_adj(const Plan& p, const float* gx, const float* gy,
                     const float* gz, float* out, hipStream_t s);
 int launch_paint(float* mesh, const float* pos, const float* w, float wscale,
@@ -293,9 +296,16 @@ int launch_readout_kick_drift(float* X, float* P, float* F, const Mesh3& m,
 bool readout_box_ok(const MeshDims& d, const KickDrift& c, const float* X,
                     const float* P, const float* F, const float* phi);
 // meta: the boxes the paint of the same positions left (brick_meta), or null.
+// b3 (mesh set): with *count of at least need the bricks without a box read
+// the force from this packed force mesh.
+struct BoxlessMesh {
+  const float* mesh;
+  const int* count;
+  int need;
+};
 int launch_readout_box(float* X, float* P, float* F, const float* phi,
-                       const int* meta, const MeshDims& d, const KickDrift& c,
-                       hipStream_t s);
+                       const int* meta, const BoxlessMesh& b3,
+                       const MeshDims& d, const KickDrift& c, hipStream_t s);
 
 // out += scale * sum_p sum_c G[p][c] readout(m_c, X_p * f) (float64)
 int launch_readout_dot(const float* X, const float* G, const Mesh3& m,
@@ -347,6 +357,8 @@ long long brick_work_floats(const MeshDims& d, const BrickGrid& g, int C);
 // where launch_brick_paint leaves the boxes of its bricks (8 ints each)
 const int* brick_meta(const MeshDims& d, const BrickGrid& g, int C,
                       float* work);
+// and the number of those without a box
+const int* brick_boxless(float* work);
 // mesh[c] = sum_p w[p*wstride+c]*wscale * CIC(X*ps) (every cell written), plus
 // base, if given (C = 1; it may be the mesh itself).  ready (optional, in / out): whether a paint
 // has left this workspace's counters zero since anything else wrote there.

@@ -71,11 +71,12 @@ static __device__ __forceinline__ Cell cell_at(const GridDims& g, unsigned i) {
   c.z0 = (int)(4 * q);
   return c;
 }
-static __device__ __forceinline__ unsigned block_first(void) {
-  return (unsigned)xcd_block(blockIdx.x, gridDim.x) * blockDim.x;
+// the first item of block i of nb
+static __device__ __forceinline__ unsigned block_first(unsigned i, unsigned nb) {
+  return (unsigned)xcd_block(i, nb) * blockDim.x;
 }
 static __device__ __forceinline__ Cell cell_of(const GridDims& g) {
-  return cell_at(g, block_first() + threadIdx.x);
+  return cell_at(g, block_first(blockIdx.x, gridDim.x) + threadIdx.x);
 }
 
 // D_z of the 4 cells z0 .. z0 + 3 of the row at p (row length nz)
@@ -124,11 +125,12 @@ static __device__ __forceinline__ Nbr nbr_of(const Cell& c, const GridDims& g) {
 // go through LDS instead and every store instruction writes one contiguous
 // 1 KB run per wave (measured at 256^3 with NC = 4: 78 us against 103).
 template <int NC>
-__global__ __launch_bounds__(256) void k_grad_mesh(const float* __restrict__ phi,
-                                                   float* __restrict__ fm,
-                                                   const float* __restrict__ w4,
-                                                   GridDims g) {
-  const Cell c = cell_of(g);
+static __device__ __forceinline__ void grad_block(const float* __restrict__ phi,
+                                                  float* __restrict__ fm,
+                                                  const float* __restrict__ w4,
+                                                  const GridDims& g,
+                                                  unsigned i0) {
+  const Cell c = cell_at(g, i0 + threadIdx.x);
   float4 gx = make_float4(0.f, 0.f, 0.f, 0.f), gy = gx, gz = gx, gw = gx;
   if (c.ok) {
     const Nbr n = nbr_of(c, g);
@@ -158,7 +160,6 @@ __global__ __launch_bounds__(256) void k_grad_mesh(const float* __restrict__ phi
   // first one (the host keeps every block inside one band row group):
   // NC * 256 float4, 16-byte aligned (the first cell's offset is a multiple
   // of 4 * 256, or of the row length when rows are longer)
-  const unsigned i0 = block_first();
   const Cell c0 = cell_at(g, i0);
   const long long cell0 =
       (((long long)c0.b * g.nx + c0.x) * g.ny + c0.y) * g.nz + c0.z0;
@@ -168,6 +169,24 @@ __global__ __launch_bounds__(256) void k_grad_mesh(const float* __restrict__ phi
   for (int k = 0; k < NC; ++k) {
     const int q = t + 256 * k;
     if (q < nv) out[q] = st[q];
+  }
+}
+template <int NC>
+__global__ __launch_bounds__(256) void k_grad_mesh(const float* __restrict__ phi,
+                                                   float* __restrict__ fm,
+                                                   const float* __restrict__ w4,
+                                                   GridDims g) {
+  grad_block<NC>(phi, fm, w4, g, block_first(blockIdx.x, gridDim.x));
+}
+// The packed mesh, if *count is at least need (a count an earlier kernel left);
+// few workgroups, so that the launch costs little if not.
+__global__ __launch_bounds__(256) void k_grad_mesh_if(
+    const float* __restrict__ phi, float* __restrict__ fm,
+    const int* __restrict__ count, int need, GridDims g, unsigned nb) {
+  if (*count < need) return;
+  for (unsigned i = blockIdx.x; i < nb; i += gridDim.x) {
+    grad_block<3>(phi, fm, nullptr, g, block_first(i, nb));
+    __syncthreads();  // the next block's cells take the same LDS
   }
 }
 
@@ -234,6 +253,18 @@ int launch_grad_mesh(const Plan& p, const float* phi, float* fm, int nc,
   else
     hipLaunchKernelGGL(k_grad_mesh<3>, dim3(nblocks(g)), dim3(256), 0, s, phi,
                        fm, nullptr, g);
+  PMX_LAUNCH_CHECK();
+  return kOk;
+}
+
+int launch_grad_mesh_if(const Plan& p, const float* phi, float* fm,
+                        const int* count, int need, hipStream_t s) {
+  PMX_REQUIRE(grad_stencil_ok(p), "gradient stencil: sides");
+  const GridDims g = grid_dims(p, 1);
+  const unsigned nb = nblocks(g);
+  ProfScope prof_(kProfGrad, s);
+  hipLaunchKernelGGL(k_grad_mesh_if, dim3(std::min(nb, 2048u)), dim3(256), 0, s,
+                     phi, fm, count, need, g, nb);
   PMX_LAUNCH_CHECK();
   return kOk;
 }
