@@ -717,9 +717,19 @@ struct Tape {
 
 // One particle per cell in grid order: the readout and its adjoint work on
 // the potential itself (box_readout.h), so no force mesh is formed or kept.
+// Not on sides that bricks of 8 x 16 x 16 particles mostly have no box in (it
+// may not be longer than the side), unless the run is so small that the host's
+// one launch less per force counts: a run of two steps from force meshes / from
+// the potential in us, 128 x 20^3 with 0.5 cells rms of noise 637 / 754, 32 x
+// 20^3 273 / 301, 12 x 256 x 256 (2 members) 680 / 772, 256 x 256 x 16 789 /
+// 835; but 32 x 16^3 273 / 263, 64 x 12^3 286 / 264; with boxes, 20 x 256 x 256
+// 308 / 283, 256 x 24 x 256 333 / 299.
+constexpr long long kThinParticles = 200000;
 static bool box_run(const Plan& p, long long N, float f) {
+  const bool thin = p.d.nx < 16 || p.d.ny < 24 || p.d.nz < 24;
   return f == 1.0f && p.d.nz % 4 == 0 &&
-         N == (long long)p.d.nx * p.d.ny * p.d.nz;
+         N == (long long)p.d.nx * p.d.ny * p.d.nz &&
+         !(thin && p.d.B * N >= kThinParticles);
 }
 
 // A particle without a box reads 20 rows of the potential, of a force mesh 4.
