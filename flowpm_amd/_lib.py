@@ -123,6 +123,7 @@ _SIGS = {
                                     _c.POINTER(_f), _c.POINTER(_dp),
                                     _c.POINTER(_i), _c.POINTER(_i),
                                     _c.POINTER(_i), _c.POINTER(_vp), _vp]),
+    "pmx_nbody_keeps_potentials": (_i, [_vp, _ll, _f]),
     "pmx_nbody_tape_floats": (_ll, [_vp, _ll, _i]),
     "pmx_nbody_compact_tape_floats": (_ll, [_vp, _ll, _i]),
     "pmx_nbody_run_compact_taped": (_i, [_vp, _vp, _ll, _f, _f, _dp, _i, _vp,

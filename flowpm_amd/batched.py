@@ -45,7 +45,7 @@ class _Group:
       # holds the cotangent of the final state, gstate receives the
       # cotangent of the initial state
       h = self.plan.handle
-      self.compact = tfpm._compact()
+      self.compact = tfpm._compact(self.plan, self.N, self.f)
       self.tape = tfpm._tape(self.plan, self.N, self.nsteps, self.compact,
                              dev)
       self.adj_work = torch.empty(L.pmx_nbody_adj_work_floats(h, self.N, 0),

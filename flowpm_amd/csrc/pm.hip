@@ -2326,6 +2326,10 @@ int pmx_nbody_batched_step(int ngroups, const pmx_plan* const* plans,
   return 0;
 }
 
+int pmx_nbody_keeps_potentials(const pmx_plan* plan, long long N, float f) {
+  return plan && N >= 1 && box_run(P(plan), N, f);
+}
+
 long long pmx_nbody_tape_floats(const pmx_plan* plan, long long N,
                                 int nsteps) {
   return (plan && N >= 1 && nsteps >= 0) ? tape_floats(P(plan), N, nsteps)

@@ -85,8 +85,9 @@ def set_compact_tape(compact):
   (about half the memory: at 256^3 x 40 steps 11 GB against 18.8 GB; the
   backward pass forms each force mesh from it together with the density
   cotangent; the same gradients): True, False, or None (automatic: True).
-  With one particle per cell (pm_nc_factor 1) either tape keeps potentials:
-  the forward pass reads the potential itself."""
+  A run of one particle per cell (pm_nc_factor 1) keeps potentials either way
+  wherever its forward pass reads the potential itself: on all meshes but large
+  ones with a short side (pmx_nbody_keeps_potentials)."""
   _COMPACT[0] = None if compact is None else bool(compact)
 
 
@@ -95,17 +96,19 @@ def _tape_fits(plan, N, nsteps, device, name):
   return need <= _TAPE_FRACTION * torch.cuda.mem_get_info(device)[0]
 
 
-def _compact():
-  return _COMPACT[0] is not False
+def _compact(plan, N, f):
+  """Whether a tape of this run keeps potentials."""
+  return _COMPACT[0] is not False or \
+      _lib.lib().pmx_nbody_keeps_potentials(plan.handle, N, f) == 1
 
 
-def _resolve_every(plan, N, nsteps, every, device):
+def _resolve_every(plan, N, nsteps, every, device, f=1.0):
   """Checkpoint interval of the automatic policy: 0 (a tape, when it fits in
   half of the free device memory), else segments of 8 steps."""
   if every is not None:
     return int(every)
   if _tape_fits(plan, N, nsteps, device, "pmx_nbody_%stape_floats" %
-                ("compact_" if _compact() else "")):
+                ("compact_" if _compact(plan, N, f) else "")):
     return 0
   return _AUTO_SEGMENT
 
@@ -791,7 +794,7 @@ class _Force(torch.autograd.Function):
   @staticmethod
   def forward(ctx, state, plan, N, f, fac, fac_t=None):
     x0 = _f32(state)
-    compact = _compact()
+    compact = _compact(plan, N, f)
     tape = _tape(plan, N, 0, compact, x0.device)
     st = _run_from(plan, x0, N, f, fac, None, 0, _work(plan), tape, compact)
     ctx.save_for_backward(tape)
@@ -906,7 +909,7 @@ class _Nbody(torch.autograd.Function):
     if every == 0:
       # the compact tape (X and the potential of every force), or the full
       # one (X and the float4 force mesh)
-      ctx.compact = _compact()
+      ctx.compact = _compact(plan, N, f)
       tape = _tape(plan, N, nsteps, ctx.compact, x0.device)
       st = _run_from(plan, x0, N, f, fac, cptr, nsteps, work, tape,
                      ctx.compact)
@@ -1150,7 +1153,7 @@ def nbody(cosmo, state, stages, nc, pm_nc_factor=1,
                                            cpar is not None)
   every = checkpoint_every if checkpoint_every is not None else _CKPT_EVERY[0]
   every = _resolve_every(plan, N, len(coef) // 3, every,
-                         state.device) if need_grad else 1
+                         state.device, f) if need_grad else 1
   return _Nbody.apply(state, plan, N, f, fac, coef, every, need_grad, cpar)
 
 
@@ -1186,7 +1189,8 @@ def _nbody_states_differentiable(state, stages, plan, N, f, fac, coef,
                                           cp is not None)
       every = checkpoint_every if checkpoint_every is not None else \
           _CKPT_EVERY[0]
-      every = _resolve_every(plan, N, 1, every, st.device) if need else 1
+      every = _resolve_every(plan, N, 1, every, st.device,
+                             f) if need else 1
       st = _Nbody.apply(st, plan, N, f, fac, c, every, need, cp)
     out.append((stages[i + 1], st))
   return out

@@ -493,7 +493,11 @@ int pmx_nbody_batched_step(int ngroups, const pmx_plan* const* plans,
  * (pmx_nbody_tape_floats(plan, N, nsteps) floats), so that
  * pmx_nbody_adjoint_taped needs no recomputation.  This replaces TF's
  * stored forward intermediates of tfpm.py:425-503 under autodiff; the
- * adjoint work is pmx_nbody_adj_work_floats(plan, N, 0) floats. */
+ * adjoint work is pmx_nbody_adj_work_floats(plan, N, 0) floats.
+ * Runs that form no force mesh (pmx_nbody_keeps_potentials: one particle per
+ * cell, but for large meshes with a short side) record potentials instead, laid
+ * out like the compact tape below, and need no more than its floats. */
+int pmx_nbody_keeps_potentials(const pmx_plan* plan, long long N, float f);
 long long pmx_nbody_tape_floats(const pmx_plan* plan, long long N,
                                 int nsteps);
 int pmx_nbody_run_taped(const pmx_plan* plan, float* state, long long N,
@@ -509,8 +513,9 @@ int pmx_nbody_adjoint_taped(const pmx_plan* plan, float* tape, int nsteps,
  * keeping X and the potential of every force evaluation instead of its
  * float4 force mesh (pmx_nbody_compact_tape_floats(plan, N, nsteps) =
  * (nsteps + 1)(3 B N + B nx ny nz) floats, about half of
- * pmx_nbody_tape_floats); the forward runs as an untaped one, and pmx_nbody_adjoint_compact_taped forms each step's force mesh from
- * its potential with the gradient stencil before the step's VJP: the same
+ * pmx_nbody_tape_floats); the forward runs as an untaped one, and
+ * pmx_nbody_adjoint_compact_taped forms each step's force mesh from its
+ * potential with the gradient stencil before the step's VJP: the same
  * gradients as pmx_nbody_adjoint_taped, bit for bit.  work and gcoef as for
  * pmx_nbody_adjoint_taped. */
 long long pmx_nbody_compact_tape_floats(const pmx_plan* plan, long long N,
