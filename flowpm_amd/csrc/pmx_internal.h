@@ -292,9 +292,8 @@ int launch_readout_kick_drift(float* X, float* P, float* F, const Mesh3& m,
                               hipStream_t s);
 
 // The same from the potential (box_readout.h), for one particle per cell
-// (c.f == 1, the particle grid the mesh's own) and 16-byte aligned arrays.
-bool readout_box_ok(const MeshDims& d, const KickDrift& c, const float* X,
-                    const float* P, const float* F, const float* phi);
+// (c.f == 1, the particle grid the mesh's own).
+bool readout_box_ok(const MeshDims& d, const KickDrift& c);
 // meta: the boxes the paint of the same positions left (brick_meta), or null.
 // b3 (mesh set): with *count of at least need the bricks without a box read
 // the force from this packed force mesh.
