@@ -1,6 +1,6 @@
 // CIC paint of particles in any order, by mesh tiles (part of paint.hip).
 //
-// Two launches, without device-scope atomics and without counters:
+// Three launches, almost without device-scope atomics:
 // k_bin_sort: one workgroup per kBinChunk consecutive particles sorts the
 //   chunk's particle numbers by the mesh tiles their corners touch (mostly
 //   one; at the faces of a tile up to eight), with a histogram in LDS, and
@@ -8,13 +8,15 @@
 // k_bin_paint: one workgroup per tile collects its runs of all chunks, reads
 //   those particles, adds the corners that lie in the tile to a box in LDS in
 //   float64, and adds the box to the mesh (or writes it) with plain accesses.
-// k_bin_tail: what a tile holds beyond kBinShare entries is shared out to
-//   further workgroups, which add their boxes with float atomics (a catalogue
-//   within one tile of 120^3: 300001 particles 412 us by the scatter, 1730 in
-//   one workgroup, 63 in shares).
-// The sums are float64 (the LDS atomics' order shows in the 53rd bit), so the
-// result is rounded once per cell; float64 LDS atomics run at 2.8 per clock
-// and CU here, 32-bit integers at 8.8, 64-bit ones at 5.3, float32 at 0.3.
+// k_bin_tail: what a tile holds beyond kBinShare entries (k_bin_paint counts
+//   such tiles with an atomic) is shared out to further workgroups, which add
+//   their boxes with float atomics (a catalogue within one tile of 120^3: 300001
+//   particles 412 us by the scatter, 1730 in one workgroup, 63 in shares).
+// The sums are float64 (the LDS atomics' order shows in the 53rd bit), so a cell
+// of a tile of up to kBinShare entries is rounded once, and repeats but for that;
+// in a fuller tile it is rounded once per share, in an order that may vary.
+// float64 LDS atomics run at 2.8 per clock and CU here, 32-bit integers at 8.8,
+// 64-bit ones at 5.3, float32 at 0.3.
 // The scatter's device-scope atomics run at 27 per ns on the whole chip: the
 // paint of 300007 particles on 120^3 126 us -> 30, that of 2 x 96^3 in the
 // readout's adjoint 485 -> 62.

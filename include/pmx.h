@@ -69,9 +69,11 @@ int pmx_cic_paint(float* mesh, const float* pos, const float* weight, int B,
  * (N = nx*ny*nz, pos_scale 1: the final paint of an nbody run) go through
  * the brick paint of the time loop, which writes the mesh without atomics
  * (mesh += paint, as pmx_cic_paint); others, from some tens of thousands
- * on, are sorted by mesh tiles, which are painted without atomics; the rest
- * goes through pmx_cic_paint's scatter.  work: pmx_cic_paint_work_floats() floats (0: not applicable;
- * work may then be NULL). */
+ * on, are sorted by mesh tiles, whose sums are float64 and stored without
+ * atomics (but tiles of more than 8192 deposits: each further 8192 are one
+ * float32 addition per cell, in an order that may vary); the rest goes through
+ * pmx_cic_paint's scatter.  work: pmx_cic_paint_work_floats() floats (0: not
+ * applicable; work may then be NULL). */
 long long pmx_cic_paint_work_floats(int B, long long N, int nx, int ny,
                                     int nz, float pos_scale);
 int pmx_cic_paint_ws(float* mesh, const float* pos, const float* weight,
@@ -101,8 +103,8 @@ int pmx_cic_readout_adj(float* gmesh, float* dpos, const float* gout,
                         void* stream);
 /* The same with gmesh overwritten (it need not be cleared) and a workspace of
  * pmx_cic_readout_adj_work_floats() floats, in which the particles are sorted
- * by mesh tiles, so that the mesh is written without atomics (0: not
- * applicable; work may then be NULL). */
+ * by mesh tiles as in pmx_cic_paint_ws (0: not applicable; work may then be
+ * NULL). */
 long long pmx_cic_readout_adj_work_floats(int B, long long N, int nx, int ny,
                                           int nz);
 int pmx_cic_readout_adj_ws(float* gmesh, float* dpos, const float* gout,
