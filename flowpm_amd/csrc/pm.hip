@@ -1125,9 +1125,9 @@ static Tape tape_of(const Plan& p, float* tape, long long N, int nsteps,
 // Compact tape of a whole run: X of the jump-start force and of every step,
 // then the potential of every force evaluation (slot 0 the jump start,
 // 1 + i step i) instead of its float4 force mesh: (nsteps + 1)(BN3 + M)
-// floats against (nsteps + 1)(BN3 + 4M).  The forward run keeps the packed
-// force meshes of an untaped run; the reverse sweep takes each step's
-// float4 mesh from its potential with the gradient stencil.
+// floats against (nsteps + 1)(BN3 + 4M).  The forward run goes as an untaped one;
+// the reverse sweep takes each step's float4 mesh from its potential with the
+// gradient stencil.
 static long long compact_tape_floats(const Plan& p, long long N, int nsteps) {
   const long long M = p.d.rows * p.d.nz;
   const long long BN3 = 3LL * p.d.B * N;
