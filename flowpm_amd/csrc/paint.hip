@@ -23,10 +23,10 @@
 //   are the last ones to end, 3-channel deposit at 128 x 160 x 96 22.7 -> 31.1
 //   (64-bit integers 36.6: a conversion takes some 12 instructions).
 //   Every brick has a 64 KB piece of the arena per channel; a larger box, up
-//   to 128 KB, goes to a pool of 8 KB per brick (where a box lies does not
-//   change what is in it).  Without the pool the late boxes beyond their pieces
-//   spilled: at 256^3, a = 1, 100 us of float atomics per density
-//   paint and 231 per three-channel one.
+//   to 128 KB (of many particles: box_max), goes to a pool of 8 KB per brick
+//   (where a box lies does not change what is in it).  Without the pool the
+//   late boxes beyond their pieces spilled: at 256^3, a = 1, 100 us of float
+//   atomics per density paint and 231 per three-channel one.
 //   A brick whose box is larger still, or finds the pool full, falls back to
 //   device-scope float atomics into the finished mesh (k_brick_spill, after
 //   phase 2).
@@ -137,13 +137,16 @@ constexpr int kWinFloats = 10112;
 constexpr int kDW = kDT / 64;
 constexpr int kPPT = 2048 / kDT;
 // The largest box of a brick of nloc particles.  Those of a finer force mesh
-// have 256 or fewer: added one by one they cost less than the many passes over
-// a large box take the workgroup, which ends last.  Force and gradient, boxes
-// up to 128 / 80 / 64 KB in us: 64 x 80 x 48, f = 2, a = 1 261.5 / 263.7 / 270;
-// grids with 2 spacings rms of noise, f = 2 32^3 191 / 172 / 168, 64^3 604 / 562
-// / 565, 64 x 80 x 48 604 / 594 / 565, f = 4 64^3 1322 / 1219 / 1212.
+// have 256 (f = 2) or 32 (f = 4): added one by one they cost less than the many
+// passes over a large box take the workgroup, which ends last.  Force and
+// gradient, boxes up to 128 / 80 / 64 KB in us: 64 x 80 x 48, f = 2, a = 1 261.5
+// / 263.7 / 270; grids with 2 spacings rms of noise, f = 2 32^3 191 / 172 / 168,
+// 64^3 604 / 562 / 565, 64 x 80 x 48 604 / 594 / 565; f = 4, 1 spacing 32^3 278 /
+// 274 / 251, 64^3 1620 / 1602 / 1561.
 PMX_HD long long box_max(int nloc) {
-  return nloc <= 512 ? 5 * kBoxFloats / 4 : 2 * kBoxFloats;
+  return nloc <= 64    ? kBoxFloats
+         : nloc <= 512 ? 5 * kBoxFloats / 4
+                       : 2 * kBoxFloats;
 }
 static_assert(kDW == 8, "the workgroup reductions take 8 waves");
 

@@ -17,9 +17,9 @@ from oracle.background import GrowthTable, planck15
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("f,n,amp", [(2, (24, 32, 32), 1.6),
-                                     (4, (12, 16, 16), 1.3)])
-def test_boxes_around_the_largest(gpu, f, n, amp):
+@pytest.mark.parametrize("f,n,amp,most", [(2, (24, 32, 32), 1.6, 20480),
+                                          (4, (12, 16, 16), 1.1, 16384)])
+def test_boxes_around_the_largest(gpu, f, n, amp, most):
   gen = torch.Generator().manual_seed(31)
   q = torch.as_tensor(np.indices(n).reshape(3, -1).T.astype(np.float32))
   x = (q + amp * torch.randn(q.shape, generator=gen) - 1.75)[None]
@@ -28,8 +28,8 @@ def test_boxes_around_the_largest(gpu, f, n, amp):
   b = m.unfold(0, e[0], e[0]).unfold(1, e[1], e[1]).unfold(2, e[2], e[2])
   b = b.flatten(4)
   vol = (b.amax(-1) - b.amin(-1) + 2).prod(-1)
-  # (80 KB: a fifth of the bricks or more on either side)
-  assert 0.2 < float((vol > 20480).float().mean()) < 0.8
+  # (a fifth of the bricks or more on either side)
+  assert 0.2 < float((vol > most).float().mean()) < 0.8
   g = torch.randn(1, x.shape[1], 3, generator=gen)
 
   def both(dev, dt, run):
